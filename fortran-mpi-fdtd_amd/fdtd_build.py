@@ -65,7 +65,7 @@ def build_fortran_host():
 def build_oracles(with_reference=True):
     odir = os.path.join(REPO, "oracle")
     _run(["make", "-C", odir, "all"])
-    if with_reference and os.path.isdir("/root/reference") and shutil.which(FLANG):
+    if with_reference and os.path.isdir("/root/reference/modules/src") and shutil.which(FLANG):
         _run(["make", "-C", odir, "ref"])
         _run(["make", "-C", odir, "ref2d"])
         if os.path.isfile("/opt/conda/include/mpif.h"):  # the 1D TFSF driver links MPICH
