@@ -1,14 +1,18 @@
 // fdtd2d.hip -- gfx950 2D stepper behind include/fdtd2d.h: TEz (Hz, Ex,
 // Ey), the reference's 2D driver, and TMz (Ez, Hx, Hy).
 //
-// One code path steps one simulation or a batch of many.  A step is five
+// One code path steps one simulation or a batch of many.  A step is two
 // launches over every simulation of the batch: the E half step over a
-// packed list of 64x4-cell tiles, the dispersive cells, the H half step,
-// the monitors, and a one-thread-per-simulation step advance.  Thirty-two
-// steps and the DFT fold are captured once in a HIP graph and replayed; the
-// step number of each simulation lives on the device, so simulations with
-// different step counts share the replays (a finished one skips its tiles).
-// A single simulation is a batch of one.
+// packed list of 64x16-cell tiles with the dispersive cells beside them, and
+// the H half step, whose threads also write the monitors' samples (each
+// launch costs a small simulation 2-4 us however little it does: the
+// shipped 2D case takes 22.3 us a step with the dispersive cells, the
+// monitors and the step advance in launches of their own, 15.2 us without).
+// Thirty-two steps, the DFT fold and the advance of the step counters are
+// captured once in a HIP graph and replayed; the step number of each
+// simulation lives on the device, so simulations with different step counts
+// share the replays (a finished one skips its tiles).  A single simulation
+// is a batch of one.
 //
 // Per simulation, D-form in the reference's order (sim2/program.f90:320-370,
 // sim2 = FDTDsimulations/2D/air-nanoAntennas_Si02-Sisubstrate/):
@@ -69,7 +73,7 @@ using cplx = std::complex<double>;
 template <typename real>
 struct Mat {
   real gax[2];
-  int32_t act[2];  // ACT_KEEP / ACT_DIEL / ACT_ADE per component (Ex, Ey)
+  int32_t act[2];  // ACT_KEEP / ACT_DIEL / ACT_ADE per component (Ex, Ey); Lorentz-Jp: ACT_KEEP
 };
 // TMz: act[0], gax[0] act on Ez; gax[1] is the PML medium (1/eps of the last
 // dielectric written to the cell, 1 where none); act[1] is unused.
@@ -119,11 +123,11 @@ struct Inst {
   real* pml[2][4];
   const real* prof[2];
   int32_t prow0[2], P;
-  // sources: value of the step about to run, computed by the advance kernel
+  // sources: values of the block's steps, computed by the advance kernel
   int32_t nsrc;
   int32_t src_j[kMaxLine];
   double src_t0[kMaxLine], src_st[kMaxLine], src_w0[kMaxLine], src_amp[kMaxLine];
-  real* src_val;
+  real* src_val;  // [step of the block][source]
   int32_t ngroup;
   AdeDev<real> grp[kMaxGroup];
   int32_t nljp;
@@ -134,7 +138,8 @@ struct Inst {
   int32_t probe_c[kMaxProbe];  // ghosted cell offsets
   double* probe_rec;           // [n-1][probe][3]
   int32_t probe_cap;           // steps the buffer holds
-  int32_t* ctl;                // [0] steps done, [1] target
+  // rows with a DFT line or a probe
+  int32_t nmon, mon_row[kMaxDft + kMaxProbe];
   // TMz: fields, Ez splits (PML cells only), profiles f1 f2 g1 g2 [nx+2]
   // along x then [ny+2] along y, PML depths Px (x) and P (y, above)
   int32_t tmz, Px;
@@ -247,16 +252,14 @@ struct Batch {
   int device = 0;
   hipStream_t stream = nullptr;
   void* d_inst = nullptr;
-  int32_t* d_ctl = nullptr;  // [count][2]
+  int32_t* d_ctl = nullptr;  // [count][2]: steps done at the block's start, target
   int32_t* d_tile_inst = nullptr;
   int4* d_ade = nullptr;     // (q, group, first cell, 0)
   int4* d_ljp = nullptr;     // (q, Lorentz-Jp group, first cell, 0)
   int nljp = 0;
-  int4* d_mon = nullptr;     // (q, line or -1 for probes, first i, 0)
   int4* d_fold = nullptr;    // (q, line, first i, first frequency)
-  int2* d_lines = nullptr;   // (q, line)
   int32_t* d_tfl = nullptr;  // simulations with a TFSF
-  int ntiles = 0, nade = 0, nmon = 0, nlines = 0, ntf = 0, nfold = 0;
+  int ntiles = 0, nade = 0, ntf = 0, nfold = 0;
   std::vector<int32_t> ctl;  // host mirror
   // order of the simulations in the packed tile list: largest first, so
   // the small ones' tiles fill the end of each launch
@@ -334,7 +337,7 @@ __device__ __forceinline__ bool tf_h_term(const Inst<real>& S, int j, real& v) {
 // TMz E half step of cell (i, j); loads first (the pointers may alias as far
 // as the compiler knows)
 template <typename real>
-__device__ __forceinline__ void e_tmz(const Inst<real>& S, int i, int j, real& carry, bool use_carry) {
+__device__ __forceinline__ void e_tmz(const Inst<real>& S, int i, int j, int st, real& carry, bool use_carry) {
   const int px = S.px;
   const int c = i + px * j;
   bool src = false;
@@ -342,7 +345,7 @@ __device__ __forceinline__ void e_tmz(const Inst<real>& S, int i, int j, real& c
   for (int s = 0; s < S.nsrc; ++s)
     if (j == S.src_j[s]) {
       src = true;
-      sv = S.src_val[s];
+      sv = S.src_val[st * kMaxLine + s];
     }
   const bool pml = in_pml_tmz(S, i, j);
   real cv = 0;
@@ -357,7 +360,7 @@ __device__ __forceinline__ void e_tmz(const Inst<real>& S, int i, int j, real& c
     dz = dz + S.ku * ((hyc - hyi) + (-hxc + hxj));
     if (src) dz = dz + sv;
     if (corr) dz = dz + cv;
-    S.dz[c] = dz;
+    if (m.act[0] != ACT_ADE) S.dz[c] = dz;  // the dispersive cells advance their own D
     if (m.act[0] == ACT_DIEL) {
       ez = dz * m.gax[0];
       wrote = true;
@@ -420,7 +423,7 @@ __device__ __forceinline__ void h_tmz(const Inst<real>& S, int i, int j, real& c
 
 // TEz E half step of cell (i, j); carry: Hz of the row below when use_carry
 template <typename real>
-__device__ __forceinline__ void e_tez(const Inst<real>& S, int i, int j, real& carry, bool use_carry) {
+__device__ __forceinline__ void e_tez(const Inst<real>& S, int i, int j, int st, real& carry, bool use_carry) {
   const int px = S.px;
   const int c = i + px * j;
   const bool main = j >= S.j0 && j <= S.j1;
@@ -429,7 +432,7 @@ __device__ __forceinline__ void e_tez(const Inst<real>& S, int i, int j, real& c
   for (int s = 0; s < S.nsrc; ++s)
     if (j == S.src_j[s]) {
       src = true;
-      sv = S.src_val[s];
+      sv = S.src_val[st * kMaxLine + s];
     }
   const bool slab = S.has_pml && (j <= S.ja || j >= S.jb);
   real cv = 0;
@@ -447,8 +450,9 @@ __device__ __forceinline__ void e_tez(const Inst<real>& S, int i, int j, real& c
   }
   if (src) dxv = dxv + sv;
   if (corr) dxv = dxv + cv;
-  if (main) S.dy[c] = dyv;
-  if (main || src || corr) S.dx[c] = dxv;
+  // the dispersive cells advance their own D
+  if (main && m.act[1] != ACT_ADE) S.dy[c] = dyv;
+  if ((main || src || corr) && m.act[0] != ACT_ADE) S.dx[c] = dxv;
   // dielectric writers (graphene's Ey = Dy is one with gax 1)
   if (m.act[1] == ACT_DIEL) {
     const real ey = dyv * m.gax[1];
@@ -534,16 +538,16 @@ __device__ __forceinline__ void h_tez(const Inst<real>& S, int i, int j, real& c
 // logical blocks, so the x neighbours of a tile (whose edge lines it reads)
 // mostly run on the same XCD and come from its L2, while the runs stay
 // short enough that every XCD gets a like mix of tiles (TEz/TMz, PML rows).
-// The grid is a multiple of 8 * kXcdRun (set at launch).
+// The tiles' part of the grid is a multiple of 8 * kXcdRun (set at launch).
 constexpr int kXcdRun = 32;
-__device__ __forceinline__ int xcd_block() {
-  const int b = blockIdx.x, k = b >> 3;
+__device__ __forceinline__ int xcd_block(int b) {
+  const int k = b >> 3;
   return (k / kXcdRun) * (8 * kXcdRun) + (b & 7) * kXcdRun + k % kXcdRun;
 }
 
 // ---- plain row strips ------------------------------------------------------------
-// A wavefront's kRowsPerWave rows are "plain" when none is a PML, source or
-// TFSF row and (TMz) none of its lanes lies in an x slab: the cell update is
+// A wavefront's kRowsPerWave rows are "plain" when none is a PML, source
+// (E), monitor (H) or TFSF row and (TMz) none of its lanes lies in an x slab: the cell update is
 // then the interior one of e_tez / h_tez / e_tmz / h_tmz, and the loads of
 // all rows are issued before the first row's stores (one memory round trip
 // for the strip instead of one per row).  The arithmetic is the same,
@@ -571,10 +575,47 @@ __device__ __forceinline__ bool strip_plain(const Inst<real>& S, int i0, int j0,
     if (a >= j0 && a <= j1) return false;
     if (S.tf_hi > 0 && b >= j0 && b <= j1) return false;
   }
-  if (e_half)
+  if (e_half) {
     for (int j = j0; j <= j1; ++j)
       if (src_row(S, j)) return false;
+  } else {
+    for (int m = 0; m < S.nmon; ++m)
+      if (S.mon_row[m] >= j0 && S.mon_row[m] <= j1) return false;
+  }
   return true;
+}
+
+// Monitors of cell (i, j) after step n, block slot b: the DFT lines' samples
+// of the row (sample step recorded by the row's first cell, 0 when the
+// line's gate is closed) and the probes at the cell.  Called by the thread
+// that has just written the cell's H, so it reads E and H as the step left
+// them.
+template <typename real>
+__device__ __forceinline__ void mon_cell(const Inst<real>& S, int i, int j, int n, int b) {
+  const int c = i + S.px * j;
+  const real e = (S.tmz ? S.ez : S.ex)[c], h = (S.tmz ? S.hx : S.hz)[c];
+  const int e_bit = S.tmz ? FDTD2D_DFT_EZ : FDTD2D_DFT_EX, h_bit = S.tmz ? FDTD2D_DFT_HX : FDTD2D_DFT_HZ;
+  for (int l = 0; l < S.ndft; ++l) {
+    const DftDev& D = S.dft[l];
+    if (D.j != j) continue;
+    const bool open = n >= D.n_begin && (D.n_end <= 0 || n <= D.n_end);
+    if (i == 1) D.sstep[b] = open ? n : 0;
+    if (!open) continue;
+    real* samp = (real*)D.samp + (int64_t)b * D.nslots * S.nx + (i - 1);
+    if (D.mask & e_bit) {
+      *samp = e;
+      samp += S.nx;
+    }
+    if (D.mask & h_bit) *samp = h;
+  }
+  // probes: (n*dt, Ex, Hz), sim2/program.f90:376,397,417; TMz (n*dt, Ez, Hx)
+  for (int p = 0; p < S.nprobe; ++p)
+    if (S.probe_c[p] == c && n - 1 < S.probe_cap) {
+      double* r = S.probe_rec + ((int64_t)(n - 1) * S.nprobe + p) * 3;
+      r[0] = (double)n * S.dt;
+      r[1] = (double)e;
+      r[2] = (double)h;
+    }
 }
 
 template <typename real>
@@ -602,8 +643,8 @@ __device__ __forceinline__ void e_tez_strip(const Inst<real>& S, int i, int j0) 
     const int c = c0 + px * r;
     const real dxv = dx[r] + S.ku * (hz[r + 1] - hz[r]);
     const real dyv = dy[r] - S.ku * (hz[r + 1] - hzi[r]);
-    S.dy[c] = dyv;
-    S.dx[c] = dxv;
+    if (m[r].act[1] != ACT_ADE) S.dy[c] = dyv;
+    if (m[r].act[0] != ACT_ADE) S.dx[c] = dxv;
     if (m[r].act[1] == ACT_DIEL) {
       const real ey = dyv * m[r].gax[1];
       S.ey[c] = ey;
@@ -664,7 +705,7 @@ __device__ __forceinline__ void e_tmz_strip(const Inst<real>& S, int i, int j0) 
   for (int r = 0; r < R; ++r) {
     const int c = c0 + px * r;
     const real d = dz[r] + S.ku * ((hy[r] - hyi[r]) + (-hx[r + 1] + hx[r]));
-    S.dz[c] = d;
+    if (m[r].act[0] != ACT_ADE) S.dz[c] = d;
     if (m[r].act[0] == ACT_DIEL) {
       const real ez = d * m[r].gax[0];
       S.ez[c] = ez;
@@ -701,95 +742,47 @@ __device__ __forceinline__ void h_tmz_strip(const Inst<real>& S, int i, int j0) 
   }
 }
 
-// E and H over the packed tile list: block = one tile at a time, wavefront
-// w marches rows 4w..4w+3 of the tile (j uniform per wavefront).
-template <typename real>
-__global__ __launch_bounds__(kTX * kWaves) void k2_e(const Inst<real>* __restrict__ I,
-                                                     const int32_t* __restrict__ tile_inst, int ntiles) {
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  for (int t = xcd_block(); t < ntiles; t += gridDim.x) {
-    const int q = tile_inst[t];
-    const Inst<real>& S = I[q];
-    if (S.ctl[0] >= S.ctl[1]) continue;  // finished: nothing to do this step
-    const int lt = t - S.tile0;
-    const int i = (lt % S.ntx) * kTX + lane + 1;
-    const int j0 = (lt / S.ntx) * kTY + wave * kRowsPerWave + 1;
-    if (i > S.nx) continue;
-    if (strip_plain(S, (lt % S.ntx) * kTX, j0, true)) {
-      if (S.tmz)
-        e_tmz_strip(S, i, j0);
-      else
-        e_tez_strip(S, i, j0);
-      continue;
-    }
-    real carry = 0;
-    for (int r = 0; r < kRowsPerWave; ++r) {
-      const int j = j0 + r;
-      if (j > S.ny) break;
-      if (S.tmz)
-        e_tmz(S, i, j, carry, r > 0);
-      else
-        e_tez(S, i, j, carry, r > 0);
-    }
-  }
-}
-
-template <typename real>
-__global__ __launch_bounds__(kTX * kWaves) void k2_h(const Inst<real>* __restrict__ I,
-                                                     const int32_t* __restrict__ tile_inst, int ntiles) {
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  for (int t = xcd_block(); t < ntiles; t += gridDim.x) {
-    const int q = tile_inst[t];
-    const Inst<real>& S = I[q];
-    if (S.ctl[0] >= S.ctl[1]) continue;
-    const int lt = t - S.tile0;
-    const int i = (lt % S.ntx) * kTX + lane + 1;
-    const int j0 = (lt / S.ntx) * kTY + wave * kRowsPerWave + 1;
-    if (i > S.nx) continue;
-    if (strip_plain(S, (lt % S.ntx) * kTX, j0, false)) {
-      if (S.tmz)
-        h_tmz_strip(S, i, j0);
-      else
-        h_tez_strip(S, i, j0);
-      continue;
-    }
-    real carry = 0;
-    for (int r = 0; r < kRowsPerWave; ++r) {
-      const int j = j0 + r;
-      if (j > S.ny) break;
-      if (S.tmz)
-        h_tmz(S, i, j, carry, r > 0);
-      else
-        h_tez(S, i, j, carry, r > 0);
-    }
-  }
-}
-
 // Dispersive cells (mod2/gold_mod.f90:54-73, mod2/graphene_mod.f90:63-92):
-// E = Re[(D - I + ha S + sum_p gb_p g_p) / (ga + Sn)], then the state.
+// D += Ku curl H (the cell kernels leave these components' D to this one, so
+// that both run in one launch), the row's line source and TFSF term, then
+// E = Re[(D - I + ha S + sum_p gb_p g_p) / (ga + Sn)] and the state.  They lie
+// outside the PML (commit).
 template <typename real>
-__global__ __launch_bounds__(256) void k2_ade(const Inst<real>* __restrict__ I, const int4* __restrict__ work,
-                                              int nwork) {
-  const int w = blockIdx.x;
-  if (w >= nwork) return;
-  const int4 wk = work[w];
-  const Inst<real>& S = I[wk.x];
-  if (S.ctl[0] >= S.ctl[1]) return;
-  const AdeDev<real>& G = S.grp[wk.y];
-  const int e = wk.z + (int)threadIdx.x;
+__device__ __forceinline__ void ade_cells(const Inst<real>& S, const AdeDev<real>& G, int e, int st) {
   if (e >= G.ncells) return;
   const int n = G.ncells;
   const int c = G.cells[e];
   const int mask = G.mask[e];
   const AdeCoef<double>& co = G.co;
   const int ncp = co.ncp;
-  const int i = c % S.px;
+  const int px = S.px;
+  const int i = c % px, j = c / px;
+  bool src = false;
+  real sv = 0;
+  for (int s = 0; s < S.nsrc; ++s)
+    if (j == S.src_j[s]) {
+      src = true;
+      sv = S.src_val[st * kMaxLine + s];
+    }
+  real cv = 0;
+  const bool corr = tf_d_term(S, j, cv);
+  real d[2];
+  if (S.tmz) {
+    const real hxc = S.hx[c], hxj = S.hx[c - px], hyc = S.hy[c], hyi = S.hy[c - 1];
+    d[0] = S.dz[c] + S.ku * ((hyc - hyi) + (-hxc + hxj));
+    d[1] = 0;
+  } else {
+    const real hzc = S.hz[c], hzj = S.hz[c - px], hzi = S.hz[c - 1];
+    d[0] = S.dx[c] + S.ku * (hzc - hzj);
+    d[1] = S.dy[c] - S.ku * (hzc - hzi);
+  }
+  if (src) d[0] = d[0] + sv;
+  if (corr) d[0] = d[0] + cv;
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     if (!(mask & (1 << q))) continue;
-    const double dv = S.tmz ? S.dz[c] : (q == 0 ? S.dx[c] : S.dy[c]);
+    (S.tmz ? S.dz : (q == 0 ? S.dx : S.dy))[c] = d[q];
+    const double dv = d[q];
     double* Ip = G.state + (int64_t)(0 * 2 + q) * n + e;
     double* Sp = G.state + (int64_t)(1 * 2 + q) * n + e;
     const double Iv = *Ip, Sv = *Sp;
@@ -836,19 +829,108 @@ __global__ __launch_bounds__(256) void k2_ade(const Inst<real>* __restrict__ I, 
   }
 }
 
+// blocks of a launch that come before its tiles, a whole number of rounds
+// over the XCDs so that the tiles' dealing stays as it is
+__host__ __device__ __forceinline__ int list_blocks(int n) { return (n + 7) & ~7; }
+
+// E and H over the packed tile list: block = one tile at a time, wavefront
+// w marches rows 4w..4w+3 of the tile (j uniform per wavefront).  st is the
+// step's place in the 32-step block: simulation q runs step ctl[2q] + st + 1
+// while that does not pass its target ctl[2q+1].  The E launch starts with
+// the dispersive cells' work list (no cell reads what another of the launch
+// writes); they come first because a cell's 12-26 words of FP64 state take
+// longer than a tile.
+template <typename real>
+__global__ __launch_bounds__(kTX * kWaves) void k2_e(const Inst<real>* __restrict__ I, const int32_t* __restrict__ ctl,
+                                                     const int32_t* __restrict__ tile_inst, int ntiles,
+                                                     const int4* __restrict__ ade, int nade, int st) {
+  const int nl = list_blocks(nade);
+  if ((int)blockIdx.x < nl) {
+    if ((int)blockIdx.x >= nade) return;
+    const int4 wk = ade[blockIdx.x];
+    if (ctl[2 * wk.x] + st >= ctl[2 * wk.x + 1]) return;
+    const Inst<real>& S = I[wk.x];
+    ade_cells(S, S.grp[wk.y], wk.z + (int)threadIdx.x, st);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  for (int t = xcd_block((int)blockIdx.x - nl); t < ntiles; t += (int)gridDim.x - nl) {
+    const int q = tile_inst[t];
+    const Inst<real>& S = I[q];
+    if (ctl[2 * q] + st >= ctl[2 * q + 1]) continue;  // finished: nothing to do this step
+    const int lt = t - S.tile0;
+    const int i = (lt % S.ntx) * kTX + lane + 1;
+    const int j0 = (lt / S.ntx) * kTY + wave * kRowsPerWave + 1;
+    if (i > S.nx) continue;
+    if (strip_plain(S, (lt % S.ntx) * kTX, j0, true)) {
+      if (S.tmz)
+        e_tmz_strip(S, i, j0);
+      else
+        e_tez_strip(S, i, j0);
+      continue;
+    }
+    real carry = 0;
+    for (int r = 0; r < kRowsPerWave; ++r) {
+      const int j = j0 + r;
+      if (j > S.ny) break;
+      if (S.tmz)
+        e_tmz(S, i, j, st, carry, r > 0);
+      else
+        e_tez(S, i, j, st, carry, r > 0);
+    }
+  }
+}
+
+template <typename real>
+__global__ __launch_bounds__(kTX * kWaves) void k2_h(const Inst<real>* __restrict__ I, const int32_t* __restrict__ ctl,
+                                                     const int32_t* __restrict__ tile_inst, int ntiles, int st) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  for (int t = xcd_block((int)blockIdx.x); t < ntiles; t += gridDim.x) {
+    const int q = tile_inst[t];
+    const Inst<real>& S = I[q];
+    const int n = ctl[2 * q] + st + 1;
+    if (n > ctl[2 * q + 1]) continue;
+    const int lt = t - S.tile0;
+    const int i = (lt % S.ntx) * kTX + lane + 1;
+    const int j0 = (lt / S.ntx) * kTY + wave * kRowsPerWave + 1;
+    if (i > S.nx) continue;
+    if (strip_plain(S, (lt % S.ntx) * kTX, j0, false)) {
+      if (S.tmz)
+        h_tmz_strip(S, i, j0);
+      else
+        h_tez_strip(S, i, j0);
+      continue;
+    }
+    real carry = 0;
+    for (int r = 0; r < kRowsPerWave; ++r) {
+      const int j = j0 + r;
+      if (j > S.ny) break;
+      if (S.tmz)
+        h_tmz(S, i, j, carry, r > 0);
+      else
+        h_tez(S, i, j, carry, r > 0);
+      bool mon = false;
+      for (int m = 0; m < S.nmon; ++m) mon |= S.mon_row[m] == j;
+      if (mon) mon_cell(S, i, j, n, st);
+    }
+  }
+}
+
 // Lorentz-Jp cells, E form (mod2/filmGoldLorentzJp_mod.f90:35-75,
 // siLorentzJp_mod.f90, graphene3LorentzJp1nm_mod.f90: E_q += Ku*ga*(curl_q -
 // ds*JpT_q), then the poles from the new E).  E is read as the previous
 // step left it (k2_e does not write these components), the update runs in
 // FP64, the line source of the row adds ga*g.
 template <typename real>
-__global__ __launch_bounds__(256) void k2_ljp(const Inst<real>* __restrict__ I, const int4* __restrict__ work,
-                                              int nwork) {
+__global__ __launch_bounds__(256) void k2_ljp(const Inst<real>* __restrict__ I, const int32_t* __restrict__ ctl,
+                                              const int4* __restrict__ work, int nwork, int st) {
   const int w = blockIdx.x;
   if (w >= nwork) return;
   const int4 wk = work[w];
   const Inst<real>& S = I[wk.x];
-  if (S.ctl[0] >= S.ctl[1]) return;
+  if (ctl[2 * wk.x] + st >= ctl[2 * wk.x + 1]) return;
   const LjpDev& G = S.ljp[wk.y];
   const int e = wk.z + (int)threadIdx.x;
   if (e >= G.ncells) return;
@@ -875,7 +957,7 @@ __global__ __launch_bounds__(256) void k2_ljp(const Inst<real>* __restrict__ I, 
   bool hit = false;  // the line source drives local component 0 (Dx or Dz)
   for (int s = 0; s < S.nsrc; ++s)
     if (j == S.src_j[s]) {
-      sv += S.src_val[s];
+      sv += S.src_val[st * kMaxLine + s];
       hit = true;
     }
   const int np = co.npols;
@@ -919,62 +1001,27 @@ __global__ __launch_bounds__(256) void k2_ljp(const Inst<real>* __restrict__ I, 
   }
 }
 
-// Monitors after step n = ctl[0] + 1: DFT line samples into ring slot b
-// (sample step recorded, 0 when the line's gate is closed) and probes.
+// After a block of steps, one workgroup per simulation: its step counter
+// moves by the steps it made (inc, 0 before the first block of a run), its
+// ring of samples is folded and empty again (the sample steps cleared, by a
+// kernel so that the node replays safely in the captured graph), and the
+// line sources' values of the next block's steps (sim2/program.f90:337,
+// t = (n-1)*dt).
 template <typename real>
-__global__ __launch_bounds__(256) void k2_mon(const Inst<real>* __restrict__ I, const int4* __restrict__ work,
-                                              int nwork, int b) {
-  const int w = blockIdx.x;
-  if (w >= nwork) return;
-  const int4 wk = work[w];
-  const Inst<real>& S = I[wk.x];
-  if (S.ctl[0] >= S.ctl[1]) return;
-  const int n = S.ctl[0] + 1;
-  if (wk.y < 0) {  // probes: (n*dt, Ex, Hz), sim2/program.f90:376,397,417; TMz (n*dt, Ez, Hx)
-    const int p = threadIdx.x;
-    if (p < S.nprobe && n - 1 < S.probe_cap) {
-      double* r = S.probe_rec + ((int64_t)(n - 1) * S.nprobe + p) * 3;
-      r[0] = (double)n * S.dt;
-      r[1] = (double)(S.tmz ? S.ez : S.ex)[S.probe_c[p]];
-      r[2] = (double)(S.tmz ? S.hx : S.hz)[S.probe_c[p]];
-    }
-    return;
-  }
-  const DftDev& D = S.dft[wk.y];
-  const bool open = n >= D.n_begin && (D.n_end <= 0 || n <= D.n_end);
-  if (wk.z == 0 && threadIdx.x == 0) D.sstep[b] = open ? n : 0;
-  if (!open) return;
-  const int i = wk.z + (int)threadIdx.x + 1;
-  if (i > S.nx) return;
-  const int c = i + S.px * D.j;
-  real* samp = (real*)D.samp + (int64_t)b * D.nslots * S.nx;
-  int slot = 0;
-  if (S.tmz) {
-    if (D.mask & FDTD2D_DFT_EZ) samp[(int64_t)(slot++) * S.nx + (i - 1)] = S.ez[c];
-    if (D.mask & FDTD2D_DFT_HX) samp[(int64_t)slot * S.nx + (i - 1)] = S.hx[c];
-    return;
-  }
-  if (D.mask & FDTD2D_DFT_EX) samp[(int64_t)(slot++) * S.nx + (i - 1)] = S.ex[c];
-  if (D.mask & FDTD2D_DFT_HZ) samp[(int64_t)slot * S.nx + (i - 1)] = S.hz[c];
-}
-
-// Step advance: ctl[0] += 1 for every unfinished simulation, and the line
-// sources' values for the step that follows (sim2/program.f90:337,
-// t = (n-1)*dt).  inc = 0 only computes the values.
-template <typename real>
-__global__ void k2_adv(const Inst<real>* __restrict__ I, int count, int inc) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= count) return;
+__global__ __launch_bounds__(64) void k2_adv(const Inst<real>* __restrict__ I, int32_t* __restrict__ ctl, int inc) {
+  const int q = blockIdx.x;
   const Inst<real>& S = I[q];
-  int nd = S.ctl[0];
-  if (inc) {
-    if (nd >= S.ctl[1]) return;
-    S.ctl[0] = ++nd;
-  }
-  const double t = (double)nd * S.dt;  // the next step is nd + 1
-  for (int s = 0; s < S.nsrc; ++s) {
+  const int nd = min(ctl[2 * q] + inc, ctl[2 * q + 1]);
+  __syncthreads();
+  if (threadIdx.x == 0) ctl[2 * q] = nd;
+  if (inc)
+    for (int e = threadIdx.x; e < S.ndft * kBlockSteps; e += blockDim.x)
+      S.dft[e / kBlockSteps].sstep[e % kBlockSteps] = 0;
+  for (int e = threadIdx.x; e < S.nsrc * kBlockSteps; e += blockDim.x) {
+    const int b = e % kBlockSteps, s = e / kBlockSteps;
+    const double t = (double)(nd + b) * S.dt;  // step nd + b + 1
     const double a = (t - S.src_t0[s]) / S.src_st[s];
-    S.src_val[s] = (real)(S.src_amp[s] * (exp(-0.5 * (a * a)) * sin(S.src_w0[s] * t)));
+    S.src_val[b * kMaxLine + s] = (real)(S.src_amp[s] * (exp(-0.5 * (a * a)) * sin(S.src_w0[s] * t)));
   }
 }
 
@@ -983,12 +1030,14 @@ __global__ void k2_adv(const Inst<real>* __restrict__ I, int count, int inc) {
 // the hand-over of its end slabs; sim1/program.f90:222-231) and H half step
 // (hz_inc update, mypmly_inc%updateH; :252-255).
 template <typename real>
-__global__ __launch_bounds__(256) void k2_tfsf_line(const Inst<real>* __restrict__ I, const int32_t* __restrict__ list,
-                                                    int n, int h_half) {
+__global__ __launch_bounds__(256) void k2_tfsf_line(const Inst<real>* __restrict__ I, const int32_t* __restrict__ ctl,
+                                                    const int32_t* __restrict__ list, int n, int h_half, int st) {
   const int w = blockIdx.x;
   if (w >= n) return;
-  const Inst<real>& S = I[list[w]];
-  if (S.ctl[0] >= S.ctl[1]) return;
+  const int q = list[w];
+  const Inst<real>& S = I[q];
+  const int nd = ctl[2 * q] + st;
+  if (nd >= ctl[2 * q + 1]) return;
   const int N = S.ny, P = S.tf_npml, hi = N - P + 1;
   const int64_t m = N + 2;
   double* e = S.tf_line;
@@ -1000,7 +1049,7 @@ __global__ __launch_bounds__(256) void k2_tfsf_line(const Inst<real>* __restrict
   const double* g1 = e + 6 * m;
   const double* g2 = e + 7 * m;
   if (!h_half) {
-    const double t = (double)S.ctl[0] * S.dt;  // step ctl[0]+1
+    const double t = (double)nd * S.dt;  // step nd + 1
     const double a = (t - S.tf_t0) / S.tf_st;
     const double g = S.tf_amp * (exp(-0.5 * (a * a)) * sin(S.tf_w0 * t));
     for (int j = P + 1 + (int)threadIdx.x; j <= hi - 1; j += blockDim.x) {
@@ -1090,16 +1139,6 @@ __global__ __launch_bounds__(256) void k2_flush(const Inst<real>* __restrict__ I
       im[o] += si * S.dt;
     }
   }
-}
-
-// The ring is folded: clear the sample steps (a kernel, not a memset, so
-// the node replays safely in the captured graph).
-template <typename real>
-__global__ void k2_clear(const Inst<real>* __restrict__ I, const int2* __restrict__ lines, int nlines) {
-  const int l = blockIdx.x;
-  if (l >= nlines) return;
-  const int2 ln = lines[l];
-  if (threadIdx.x < kBlockSteps) I[ln.x].dft[ln.y].sstep[threadIdx.x] = 0;
 }
 
 // ---- host: set-up ------------------------------------------------------------------
@@ -1445,7 +1484,7 @@ int commit_impl(Sim* s) {
         const HostMat& m = s->mats[w];
         tab[q].act[0] = m.type == 0 ? ACT_DIEL : ACT_ADE;
         if (m.type == 0) tab[q].gax[0] = m.eps_r == 0.0 ? 0.0 : 1.0 / m.eps_r;
-        if (m.type == 3 && !ljp_comp(m, true, 0)) tab[q].act[0] = ACT_DIEL;  // E = D
+        if (m.type == 3) tab[q].act[0] = ljp_comp(m, true, 0) ? ACT_KEEP : ACT_DIEL;  // k2_ljp, or E = D
       }
       if (d >= 0) tab[q].gax[1] = s->mats[d].eps_r == 0.0 ? 0.0 : 1.0 / s->mats[d].eps_r;
     }
@@ -1463,6 +1502,8 @@ int commit_impl(Sim* s) {
       } else if (m.type == 3 && !ljp_comp(m, false, c)) {
         tab[q].act[c] = ACT_DIEL;  // a component outside jp_mask: E = D
         tab[q].gax[c] = 1.0;
+      } else if (m.type == 3) {
+        tab[q].act[c] = ACT_KEEP;  // written by k2_ljp
       } else if (m.type == 2 && c == 1) {
         tab[q].act[c] = ACT_DIEL;  // graphene: Ey = Dy (graphene_mod.f90:68)
         tab[q].gax[c] = 1.0;
@@ -1572,7 +1613,7 @@ int commit_impl(Sim* s) {
     d.d_sstep = (int32_t*)alloc_in(s->allocs, &s->dev_bytes, sizeof(int32_t) * kBlockSteps);
     if (!d.d_omega || !d.d_acc || !d.d_samp || !d.d_sstep) return set_error(FDTD_ERR_NOMEM, "DFT accumulators");
   }
-  s->d_srcval = alloc_in(s->allocs, &s->dev_bytes, sizeof(double) * kMaxLine);
+  s->d_srcval = alloc_in(s->allocs, &s->dev_bytes, sizeof(double) * kMaxLine * kBlockSteps);
   if (!s->d_srcval) return set_error(FDTD_ERR_NOMEM, "source values");
   FDTD_HIP(hipDeviceSynchronize());
   s->committed = true;
@@ -1597,7 +1638,7 @@ int ensure_probe_cap(Sim* s, int steps) {
 }
 
 template <typename real>
-Inst<real> make_inst(Sim* s, int32_t* ctl, int tile0) {
+Inst<real> make_inst(Sim* s, int tile0) {
   Inst<real> d{};
   if (s->tmz) {
     d.tmz = 1;
@@ -1668,7 +1709,15 @@ Inst<real> make_inst(Sim* s, int32_t* ctl, int tile0) {
     d.probe_c[p] = (int32_t)(s->probes[p].first + s->px * s->probes[p].second);
   d.probe_rec = s->d_probe;
   d.probe_cap = s->probe_cap;
-  d.ctl = ctl;
+  {
+    std::vector<int32_t> rows;
+    for (const auto& h : s->dfts) rows.push_back(h.j);
+    for (const auto& pr : s->probes) rows.push_back(pr.second);
+    std::sort(rows.begin(), rows.end());
+    rows.erase(std::unique(rows.begin(), rows.end()), rows.end());
+    d.nmon = (int32_t)rows.size();
+    std::copy(rows.begin(), rows.end(), d.mon_row);
+  }
   if (s->has_tf) {
     d.tf_on = 1;
     d.tf_lo = s->tfp.lo;
@@ -1693,7 +1742,7 @@ int build_inst(Batch* b) {
   int tile0 = 0;
   for (int q : b->order) {
     Sim* s = b->sims[(size_t)q];
-    v[(size_t)q] = make_inst<real>(s, b->d_ctl + 2 * q, tile0);
+    v[(size_t)q] = make_inst<real>(s, tile0);
     tile0 += v[(size_t)q].ntx * v[(size_t)q].nty;
   }
   const size_t bytes = v.size() * sizeof(Inst<real>);
@@ -1714,8 +1763,7 @@ int batch_build(Batch* b) {
   b->d_ctl = (int32_t*)alloc_in(b->allocs, nullptr, sizeof(int32_t) * 2 * count);
   if (!b->d_inst || !b->d_ctl) return set_error(FDTD_ERR_NOMEM, "batch descriptors");
   std::vector<int32_t> tile_inst, tfl;
-  std::vector<int4> ade, mon, ljp, fold;
-  std::vector<int2> lines;
+  std::vector<int4> ade, ljp, fold;
   b->order.resize((size_t)count);
   for (int q = 0; q < count; ++q) b->order[(size_t)q] = q;
   std::stable_sort(b->order.begin(), b->order.end(), [&](int u, int v) {
@@ -1732,31 +1780,22 @@ int batch_build(Batch* b) {
       for (int64_t c0 = 0; c0 < s->groups[g].ncells; c0 += kChunk) ade.push_back(make_int4(q, (int)g, (int)c0, 0));
     for (size_t g = 0; g < s->ljps.size(); ++g)
       for (int64_t c0 = 0; c0 < s->ljps[g].ncells; c0 += kChunk) ljp.push_back(make_int4(q, (int)g, (int)c0, 0));
-    for (size_t l = 0; l < s->dfts.size(); ++l) {
-      for (int i0 = 0; i0 < s->nx; i0 += kChunk) {
-        mon.push_back(make_int4(q, (int)l, i0, 0));
+    for (size_t l = 0; l < s->dfts.size(); ++l)
+      for (int i0 = 0; i0 < s->nx; i0 += kChunk)
         for (int m0 = 0; m0 < s->dfts[l].nfreq; m0 += kMC) fold.push_back(make_int4(q, (int)l, i0, m0));
-      }
-      lines.push_back(make_int2(q, (int)l));
-    }
-    if (!s->probes.empty()) mon.push_back(make_int4(q, -1, 0, 0));
     if (s->has_tf) tfl.push_back(q);
   }
   b->ntiles = (int)tile_inst.size();
   b->nade = (int)ade.size();
-  b->nmon = (int)mon.size();
-  b->nlines = (int)lines.size();
   b->nfold = (int)fold.size();
   b->d_tile_inst = (int32_t*)upload(b->allocs, nullptr, tile_inst.data(), tile_inst.size() * sizeof(int32_t));
   b->d_ade = (int4*)upload(b->allocs, nullptr, ade.data(), ade.size() * sizeof(int4));
-  b->d_mon = (int4*)upload(b->allocs, nullptr, mon.data(), mon.size() * sizeof(int4));
   b->d_fold = (int4*)upload(b->allocs, nullptr, fold.data(), fold.size() * sizeof(int4));
-  b->d_lines = (int2*)upload(b->allocs, nullptr, lines.data(), lines.size() * sizeof(int2));
   b->ntf = (int)tfl.size();
   b->nljp = (int)ljp.size();
   b->d_ljp = (int4*)upload(b->allocs, nullptr, ljp.data(), ljp.size() * sizeof(int4));
   b->d_tfl = (int32_t*)upload(b->allocs, nullptr, tfl.data(), tfl.size() * sizeof(int32_t));
-  if (!b->d_tile_inst || !b->d_ade || !b->d_mon || !b->d_fold || !b->d_lines || !b->d_tfl || !b->d_ljp)
+  if (!b->d_tile_inst || !b->d_ade || !b->d_fold || !b->d_tfl || !b->d_ljp)
     return set_error(FDTD_ERR_NOMEM, "batch work lists");
   b->ctl.assign(2 * (size_t)count, 0);
   for (int q = 0; q < count; ++q) b->ctl[2 * q] = b->ctl[2 * q + 1] = b->sims[q]->n_done;
@@ -1776,23 +1815,24 @@ void enqueue_block(Batch* b) {
   }
   unsigned grid = (unsigned)std::min(b->ntiles, std::max(8192, (b->ntiles + tpb - 1) / tpb));
   grid = (grid + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);  // whole XCD runs (xcd_block)
-  const int count = (int)b->sims.size();
+  const unsigned count = (unsigned)b->sims.size();
+  const int32_t* ctl = b->d_ctl;
   for (int s = 0; s < kBlockSteps; ++s) {
     // the line's E half step may precede k2_e, which reads only the line's h
-    if (b->ntf) hipLaunchKernelGGL(k2_tfsf_line<real>, dim3((unsigned)b->ntf), dim3(256), 0, st, I, b->d_tfl, b->ntf, 0);
-    hipLaunchKernelGGL(k2_e<real>, dim3(grid), dim3(kTX * kWaves), 0, st, I, b->d_tile_inst, b->ntiles);
-    if (b->nade) hipLaunchKernelGGL(k2_ade<real>, dim3((unsigned)b->nade), dim3(kChunk), 0, st, I, b->d_ade, b->nade);
-    if (b->nljp) hipLaunchKernelGGL(k2_ljp<real>, dim3((unsigned)b->nljp), dim3(kChunk), 0, st, I, b->d_ljp, b->nljp);
-    hipLaunchKernelGGL(k2_h<real>, dim3(grid), dim3(kTX * kWaves), 0, st, I, b->d_tile_inst, b->ntiles);
+    if (b->ntf)
+      hipLaunchKernelGGL(k2_tfsf_line<real>, dim3((unsigned)b->ntf), dim3(256), 0, st, I, ctl, b->d_tfl, b->ntf, 0, s);
+    hipLaunchKernelGGL(k2_e<real>, dim3(grid + (unsigned)list_blocks(b->nade)), dim3(kTX * kWaves), 0, st, I, ctl,
+                       b->d_tile_inst, b->ntiles, b->d_ade, b->nade, s);
+    if (b->nljp)
+      hipLaunchKernelGGL(k2_ljp<real>, dim3((unsigned)b->nljp), dim3(kChunk), 0, st, I, ctl, b->d_ljp, b->nljp, s);
+    hipLaunchKernelGGL(k2_h<real>, dim3(grid), dim3(kTX * kWaves), 0, st, I, ctl, b->d_tile_inst, b->ntiles, s);
     // k2_h read the line's new e; its H half step follows
-    if (b->ntf) hipLaunchKernelGGL(k2_tfsf_line<real>, dim3((unsigned)b->ntf), dim3(256), 0, st, I, b->d_tfl, b->ntf, 1);
-    if (b->nmon) hipLaunchKernelGGL(k2_mon<real>, dim3((unsigned)b->nmon), dim3(kChunk), 0, st, I, b->d_mon, b->nmon, s);
-    hipLaunchKernelGGL(k2_adv<real>, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, st, I, count, 1);
+    if (b->ntf)
+      hipLaunchKernelGGL(k2_tfsf_line<real>, dim3((unsigned)b->ntf), dim3(256), 0, st, I, ctl, b->d_tfl, b->ntf, 1, s);
   }
-  if (b->nlines) {
+  if (b->nfold)
     hipLaunchKernelGGL(k2_flush<real>, dim3((unsigned)b->nfold), dim3(kChunk), 0, st, I, b->d_fold, b->nfold);
-    hipLaunchKernelGGL(k2_clear<real>, dim3((unsigned)b->nlines), dim3(64), 0, st, I, b->d_lines, b->nlines);
-  }
+  hipLaunchKernelGGL(k2_adv<real>, dim3(count), dim3(64), 0, st, I, b->d_ctl, kBlockSteps);
 }
 
 // Captures one 32-step block and instantiates it.  The exec holds its own
@@ -1849,11 +1889,11 @@ int batch_run(Batch* b, const int32_t* nsteps) {
   }
   FDTD_HIP(hipMemcpy(b->d_ctl, b->ctl.data(), sizeof(int32_t) * 2 * count, hipMemcpyHostToDevice));
   if (b->prec == FDTD_FP32)
-    hipLaunchKernelGGL(k2_adv<float>, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, b->stream,
-                       (const Inst<float>*)b->d_inst, count, 0);
+    hipLaunchKernelGGL(k2_adv<float>, dim3((unsigned)count), dim3(64), 0, b->stream, (const Inst<float>*)b->d_inst,
+                       b->d_ctl, 0);
   else
-    hipLaunchKernelGGL(k2_adv<double>, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, b->stream,
-                       (const Inst<double>*)b->d_inst, count, 0);
+    hipLaunchKernelGGL(k2_adv<double>, dim3((unsigned)count), dim3(64), 0, b->stream, (const Inst<double>*)b->d_inst,
+                       b->d_ctl, 0);
   const int nblocks = (maxn + kBlockSteps - 1) / kBlockSteps;
   // FDTD2D_GRAPH=0: the same launches of each 32-step block are enqueued
   // directly instead of replaying the captured graph (for tools that cannot

@@ -29,3 +29,45 @@ def test_fold_chunks(polarization, nx, nfreq):
             check(f"fold {polarization} {nx} {nfreq} {c}", relerr(a, b), 1e-12)
     gs.close()
     os_.close()
+
+
+@pytest.mark.parametrize("polarization", ["tez", "tmz"])
+@pytest.mark.parametrize("tfsf", [False, True])
+def test_dispersive_cells_and_monitors_on_shared_rows(polarization, tfsf):
+    """Gold cells on the line source's row, on a TFSF row and on the
+    monitors' rows, monitors on the first and last rows of tiles and of
+    wavefront strips, probes at tile corners and in gold: the rows where the
+    E launch's dispersive cells and the H launch's samples take part (FP64
+    against the oracle, the parity bar)."""
+    import oracle
+    from fdtd_amd import sim2d
+
+    spec = sim2d.sweep_instance(np.random.default_rng(7), side=130, nsteps=150, npml=8, polarization=polarization)
+    nx, ny = 130, 130
+    om = spec["dft"][0]["omega"][:6]
+    spec["materials"] = [spec["materials"][0],
+                         {"type": "drude2cp", "region": sim2d.box2((1, 20), (70, 40))},
+                         {"type": "drude2cp", "region": sim2d.box2((60, 60), (nx, 66))}]
+    spec["sources"][0]["j"] = 24
+    spec["dft"] = [{"j": j, "omega": om} for j in (16, 33, 64, 9)]
+    spec["probes"] = [[1, 16], [64, 17], [65, 33], [nx, 64], [65, 62], [5, 30]]
+    if tfsf:
+        pul = {k: spec["sources"][0][k] for k in ("t0", "st", "w0")}
+        spec["tfsf"] = [dict(lo=28, hi=90, src_index=20, npml=8, **pul)]
+    gs, gi, gp = sim2d.make_simulation2d(spec, precision="fp64")
+    os_, oi, op = oracle.make_simulation2d(spec)
+    for n in (1, 32, 117):
+        gs.step(n)
+        os_.step(n)
+    comps = (sim2d.EZ2, sim2d.HX2, sim2d.HY2, sim2d.DZ2) if polarization == "tmz" else \
+        (sim2d.EX2, sim2d.EY2, sim2d.HZ2, sim2d.DX2, sim2d.DY2)
+    for c in comps:
+        check(f"rows {polarization} {tfsf} {c}", relerr(gs.field(c), os_.field(c)), 1e-12)
+    for a, b in zip(gi, oi):
+        for c in comps[:1] + ((sim2d.HX2,) if polarization == "tmz" else (sim2d.HZ2,)):
+            for x, y in zip(gs.dft(a, c), os_.dft(b, c)):
+                check(f"rows dft {polarization} {tfsf} {c}", relerr(x, y), 1e-12)
+    for a, b in zip(gp, op):
+        check(f"rows probe {polarization} {tfsf}", relerr(gs.probe(a), os_.probe(b)), 1e-12)
+    gs.close()
+    os_.close()
