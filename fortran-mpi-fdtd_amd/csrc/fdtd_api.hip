@@ -462,6 +462,10 @@ int setup_ref_y(Sim* s) {
   return 0;
 }
 
+// The one-pass march addresses a cell by a 32-bit byte offset inside its
+// plane: grids of wider planes keep the two-kernel step.
+bool onepass_fits(const Sim* s) { return (uint64_t)s->pxy * s->wsize < ((uint64_t)1 << 32); }
+
 inline bool cell_in_pml(const Sim* s, int i, int j, int k) {
   if (s->pml_mode != FDTD_PML_ALL_FACES) return false;
   const int* P = s->P;
@@ -546,7 +550,7 @@ int commit_impl(Sim* s) {
     // the one-pass step stays off unless asked for (FDTD_ONEPASS=1) or
     // picked by fdtd_autotune, which then allocates the second copies
     const char* env = std::getenv("FDTD_ONEPASS");
-    s->onepass = !ljp && env && std::atoi(env) == 1;
+    s->onepass = !ljp && env && std::atoi(env) == 1 && onepass_fits(s);
     if (const char* e = std::getenv("FDTD_ONEPASS_BY")) {
       const int v = std::atoi(e);
       if (v == 2 || v == 4 || (v == 8 && s->prec == FDTD_FP32)) s->op_by = v;
@@ -555,7 +559,6 @@ int commit_impl(Sim* s) {
       const int v = std::atoi(e);
       if (v >= 2 && v <= 4096) s->op_kc = v;
     }
-    if (const char* e = std::getenv("FDTD_DFT_FUSE")) s->dft_fuse = std::atoi(e) != 0;
     if (const char* e = std::getenv("FDTD_ZMARCH")) {
       const int v = std::atoi(e);
       if (v == 1 || v == 2 || v == 4 || v == 8) s->zm = v;
@@ -1666,7 +1669,7 @@ int fdtd_autotune(fdtd_sim* s, int steps, int* out_by, int* out_kc) {
   bool ljp = false;
   for (const auto& m : s->mats) ljp |= m.type == 3;
   bool added = false;  // second copies allocated here for the trial
-  if (s->engine == FDTD_ENGINE_FUSED && !ljp && !s->E2[0]) {
+  if (s->engine == FDTD_ENGINE_FUSED && !ljp && !s->E2[0] && onepass_fits(s)) {
     rc = alloc_onepass_copies(s);
     if (rc) return rc;
     added = true;
@@ -1695,6 +1698,7 @@ int fdtd_autotune(fdtd_sim* s, int steps, int* out_by, int* out_kc) {
   std::pair<int, int> pick = cand[0];
   for (const auto& c : cand) {
     s->onepass = c.first > 0;
+    s->mon_pend.clear();
     if (c.first > 0) {
       s->op_by = c.first;
       s->op_kc = c.second;
@@ -1715,6 +1719,7 @@ int fdtd_autotune(fdtd_sim* s, int steps, int* out_by, int* out_kc) {
     }
   }
   s->dry = false;
+  s->mon_pend.clear();  // a dry step's samples
   s->profiling = prof;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

@@ -133,7 +133,16 @@ struct DftPlane {
   int n_first = 0;           // step of the first buffered sample
   int slot[6];
   int nslots = 0;
-  bool fused_now = false;  // this step's sample is written by the H kernel
+};
+
+// Samples of a DFT plane still to be taken (the launch that takes them comes
+// with the next step): components by sel (byte q: component | slot << 4 of
+// the q-th), to the ring slot dst.
+struct MonPend {
+  int axis, index, n1, nsel;
+  int64_t np;
+  uint64_t sel;
+  void* dst;
 };
 
 struct Probe {
@@ -249,9 +258,13 @@ struct Sim {
   // two-kernel step: E and H tiles span zm planes (1, 2, 4 or 8), each
   // thread marching its column and carrying the neighbour plane in registers
   int zm = 1;
-  // FP32 two-kernel step: the H kernel writes the monitor-plane samples
-  // (FDTD_DFT_FUSE=0: the separate sample kernel does, bitwise the same)
-  int dft_fuse = 1;
+  // monitors of the last step made that are still to be sampled (at the
+  // latest at the end of the fdtd_step call), and its probes: 1 the time and
+  // E, 2 H, 3 all of a record at probe_out
+  std::vector<MonPend> mon_pend;
+  int probe_part = 0;
+  double* probe_out = nullptr;
+  double probe_tn = 0;
   // dry steps (autotuner): no sources, TFSF or monitors, no step count; run
   // only while every field is still zero, so they leave the state as it was
   bool dry = false;

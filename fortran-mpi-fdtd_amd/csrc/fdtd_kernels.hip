@@ -38,25 +38,51 @@ struct FieldArgs {
   int32_t per[3];
   int32_t px, pxy;          // offsets fit 32 bits (checked at commit)
   real ku;
-  // tile grid of the cell-parallel kernels: ntx*nty*ntz tiles of
-  // blockDim.x*blockDim.y cells, dealt out so each of the 8 XCDs (one L2
-  // each) walks a contiguous run of `tper` tiles: neighbouring rows and
-  // planes are then read from the same L2.
-  int32_t ntx, nty, ntz, tper, xcdmap;
+  int32_t xcdmap;  // deal blocks to the 8 XCDs (one L2 each) in contiguous runs
 };
 
-// Tile coordinates of this block (false: padding block, nothing to do).
+// element at byte offset `off` of the row or plane that starts at p; with p
+// wave-uniform the access takes a scalar address and the 32-bit offset, and
+// no address arithmetic per access
 template <typename real>
-__device__ __forceinline__ bool tile_of(const FieldArgs<real>& a, int& tx, int& ty, int& tz) {
-  const int b = blockIdx.x;
-  const int t = a.xcdmap ? (b & 7) * a.tper + (b >> 3) : b;
-  if (t >= a.ntx * a.nty * a.ntz) return false;
-  tx = t % a.ntx;
-  const int r = t / a.ntx;
-  ty = r % a.nty;
-  tz = r / a.nty;
-  return true;
+__device__ __forceinline__ real ld_at(const real* p, uint32_t off) {
+  return *(const real*)((const char*)p + off);
 }
+template <typename real>
+__device__ __forceinline__ void st_at(real* p, uint32_t off, real v) {
+  *(real*)((char*)p + off) = v;
+}
+
+// A launch of several parts gives each a whole number of rounds over the
+// XCDs, so that the dealing of a part's blocks does not depend on the parts
+// before it.
+__host__ __device__ __forceinline__ int round8(int n) { return (n + 7) & ~7; }
+
+// Exact quotient by a divisor known on the host, of any 31-bit number (m =
+// ceil(2^(31+s) / d), s = ceil(log2 d): Granlund and Montgomery, "Division by
+// invariant integers using multiplication", 1994): a scalar multiply and a
+// shift for the wave-uniform indices, which hardware divides in vector
+// floating point otherwise.
+struct FastDiv {
+  uint32_t m, sh;
+  int32_t d;
+};
+inline FastDiv fast_div(int d) {
+  FastDiv f;
+  f.d = d;
+  uint32_t sc = 0;
+  while (((uint64_t)1 << sc) < (uint64_t)d) ++sc;
+  f.sh = 31 + sc;
+  f.m = (uint32_t)((((uint64_t)1 << f.sh) + (uint64_t)d - 1) / (uint64_t)d);
+  return f;
+}
+__device__ __forceinline__ int fast_quot(const FastDiv& f, int v) {
+  return (int)(((uint64_t)(uint32_t)v * f.m) >> f.sh);
+}
+
+// Logical block of block b of a part of nb blocks (padded to 8 * tper):
+// each XCD takes a contiguous run of tper.
+__device__ __forceinline__ int deal(int b, int tper, int xcdmap) { return xcdmap ? (b & 7) * tper + (b >> 3) : b; }
 
 template <typename real>
 struct PmlArgs {
@@ -381,7 +407,7 @@ __device__ __forceinline__ void e_column(const FieldArgs<real>& a, const PmlArgs
     const int k = tz * KZ + r + 1;
     if (k > a.nz) break;
     const int rm = a.rowmat[__builtin_amdgcn_readfirstlane(j + (a.ny + 2) * k)];
-    if (rm < 0) {  // a mixed row: k_fused_e_mixed updates it
+    if (rm < 0) {  // a mixed row: e_mixed_block updates it
       have = false;
       continue;
     }
@@ -393,30 +419,32 @@ __device__ __forceinline__ void e_column(const FieldArgs<real>& a, const PmlArgs
   }
 }
 
-// Rows with one material id (all but the rows that cross a particle
-// surface): the table entry is a wave-uniform scalar load.  A tile spans KZ
-// planes: each thread marches its (i,j) column through them, carrying H of
-// the plane below in registers (KZ = 1: one plane, nothing carried).
-template <typename real, int KZ>
-__global__ __launch_bounds__(512) void k_fused_e(FieldArgs<real> a, PmlArgs<real> p, SrcArgs<real> src,
-                                                 int nsrc) {
-  int tx, ty, tz;
-  if (!tile_of(a, tx, ty, tz)) return;
-  const int i = tx * blockDim.x + threadIdx.x + 1;
-  // blockDim.x is a multiple of 64 (set at commit): a wavefront lies in one
-  // (j,k) row, so j and k are wave-uniform and row data are scalar loads
-  const int j = ty * blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y) + 1;
-  if (i > a.nx || j > a.ny) return;
-  e_column<real, KZ>(a, p, src, nsrc, i, j, tz, a.h[0], a.h[1], a.h[2], a.e[0], a.e[1], a.e[2]);
+// Row segments of the cell-parallel launches: a wavefront takes 64 cells of
+// one (j,k) row (or of a tile of planes above it), four consecutive segments
+// (x fastest) a workgroup, so j and k are wave-uniform and row data are
+// scalar loads.  w counts segments; false: past the end.
+struct SegGrid {
+  int32_t n, tper;     // segments in all, blocks per XCD run
+  FastDiv ntx, ny;     // by the segments a row, by the rows a plane
+};
+__device__ __forceinline__ bool seg_of(const SegGrid& g, int b, int xcdmap, int& tx, int& row) {
+  const int w = deal(b, g.tper, xcdmap) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (w >= g.n) return false;
+  row = fast_quot(g.ntx, w);
+  tx = w - row * g.ntx.d;
+  return true;
 }
 
-// Rows that mix material ids: block b updates x tile b % ntx of row
-// rows[b / ntx] (row index j + (ny+2)*k), gathering table entries per cell.
+// Rows that mix material ids: wavefront w updates segment w % ntx of row
+// rows[w / ntx] (row index j + (ny+2)*k), gathering table entries per cell.
 template <typename real>
-__global__ __launch_bounds__(256) void k_fused_e_mixed(FieldArgs<real> a, PmlArgs<real> p, SrcArgs<real> src,
-                                                       int nsrc, const int32_t* rows, int ntx) {
-  const int r = rows[blockIdx.x / ntx];
-  const int i = (blockIdx.x % ntx) * blockDim.x + threadIdx.x + 1;
+__device__ __forceinline__ void e_mixed_block(const FieldArgs<real>& a, const PmlArgs<real>& p,
+                                              const SrcArgs<real>& src, int nsrc, const int32_t* rows,
+                                              const SegGrid& g, int b) {
+  int tx, q;
+  if (!seg_of(g, b, 0, tx, q)) return;
+  const int r = rows[q];
+  const int i = tx * 64 + ((int)threadIdx.x & 63) + 1;
   const int j = r % (a.ny + 2), k = r / (a.ny + 2);
   if (i > a.nx) return;
   real sv[3] = {0, 0, 0};
@@ -427,40 +455,7 @@ __global__ __launch_bounds__(256) void k_fused_e_mixed(FieldArgs<real> a, PmlArg
                             a.e[1], a.e[2], a.e[0], a.e[1], a.e[2]);
 }
 
-// Monitor planes sampled by the FUSED H kernel: a cell on such a plane
-// writes its E and new H components to the plane's sample buffer (the same
-// values and layout as k_monitors, which would read them again
-// afterwards; an x-normal plane has one sample per 128-byte line).
-// FP32 only: in FP64 the extra registers cut the H kernel's occupancy
-// (8 -> 5 waves per SIMD) and cost more than the separate sample launch.
-constexpr int kFuseDft = 4;
-template <typename real>
-constexpr bool kFuseDftReal = sizeof(real) == 4;
-template <typename real>
-struct DftFuse {
-  int32_t n;
-  int32_t axis[kFuseDft], index[kFuseDft], n1[kFuseDft], ns[kFuseDft];
-  int64_t np[kFuseDft];
-  int32_t comp[kFuseDft][6];
-  real* dst[kFuseDft];
-};
-
-template <typename real>
-__device__ __forceinline__ void dft_fuse_write(const DftFuse<real>& df, int i, int j, int k, real ex, real ey,
-                                               real ez, real hx, real hy, real hz) {
-  for (int q = 0; q < df.n; ++q) {
-    const int ax = df.axis[q];
-    if ((ax == 0 ? i : (ax == 1 ? j : k)) != df.index[q]) continue;
-    const int u = ax == 0 ? j : i, v = ax == 2 ? j : k;
-    const int64_t o = (int64_t)(u - 1) + (int64_t)(v - 1) * df.n1[q];
-    for (int sl = 0; sl < df.ns[q]; ++sl) {
-      const int c = df.comp[q][sl];
-      const real x = c == 0 ? ex : c == 1 ? ey : c == 2 ? ez : c == 3 ? hx : c == 4 ? hy : hz;
-      df.dst[q][sl * df.np[q] + o] = x;
-    }
-  }
-}
-
+// ---------------------------------------------------------------------------
 // FUSED engine: H half step (myfdtd_func.f90:45-64 + split-field H) of one
 // cell, as the E step in a load phase (h_cell_load) and an arithmetic and
 // store phase (h_cell_store).  z march: with use_carry, Ex and Ey of plane
@@ -469,7 +464,8 @@ __device__ __forceinline__ void dft_fuse_write(const DftFuse<real>& df, int i, i
 // H and splits come from HO* and p, the new ones go to H* and pw.
 template <typename real>
 struct HCellIn {
-  int c, s;
+  int c, rb, s;
+  uint32_t ib;
   bool pml, sx, sy, sz;
   real ex, ey, ez, ey_kp, ex_kp, ez_jp, ex_jp, ez_ip, ey_ip;
   real h0[3], sp[6], gx1, gx2, gy1, gy2, gz1, gz2;
@@ -477,17 +473,22 @@ struct HCellIn {
 
 template <typename real, int FACE = 0>
 __device__ __forceinline__ void h_cell_load(const FieldArgs<real>& a, const PmlArgs<real>& p, int i, int j, int k,
-                                            bool use_carry, real cex, real cey, const real* E0, const real* E1,
+                                            int jb, bool use_carry, real cex, real cey, const real* E0, const real* E1,
                                             const real* E2, const real* HO0, const real* HO1, const real* HO2,
                                             HCellIn<real>& in) {
-  const int c = i + a.px * j + a.pxy * k;
+  const int rb = a.px * jb + a.pxy * k, co = i + a.px * (j - jb), c = rb + co;
+  const uint32_t ib = (uint32_t)co * (uint32_t)sizeof(real), ip = ib + (uint32_t)sizeof(real);
+  // wave-uniform row addresses and the cell's 32-bit byte offset from them
+  // (the E update holds too many of them: 64-bit offsets are faster there)
   in.c = c;
-  in.ex = use_carry ? cex : E0[c];
-  in.ey = use_carry ? cey : E1[c];
-  in.ez = E2[c];
-  in.ey_kp = E1[c + a.pxy]; in.ex_kp = E0[c + a.pxy];
-  in.ez_jp = E2[c + a.px]; in.ex_jp = E0[c + a.px];
-  in.ez_ip = E2[c + 1]; in.ey_ip = E1[c + 1];
+  in.rb = rb;
+  in.ib = ib;
+  in.ex = use_carry ? cex : ld_at(E0 + rb, ib);
+  in.ey = use_carry ? cey : ld_at(E1 + rb, ib);
+  in.ez = ld_at(E2 + rb, ib);
+  in.ey_kp = ld_at(E1 + (rb + a.pxy), ib); in.ex_kp = ld_at(E0 + (rb + a.pxy), ib);
+  in.ez_jp = ld_at(E2 + (rb + a.px), ib); in.ex_jp = ld_at(E0 + (rb + a.px), ib);
+  in.ez_ip = ld_at(E2 + rb, ip); in.ey_ip = ld_at(E1 + rb, ip);
   in.pml = FACE ? true : in_pml(p.P, i, j, k, a.nx, a.ny, a.nz);
   in.s = 0;
   in.sx = in.sy = in.sz = false;
@@ -519,18 +520,17 @@ __device__ __forceinline__ void h_cell_load(const FieldArgs<real>& a, const PmlA
     if (sx) { in.sp[0] = p.s[S_HYX][s]; in.sp[1] = p.s[S_HZX][s]; }
     if (sy) { in.sp[2] = p.s[S_HXY][s]; in.sp[3] = p.s[S_HZY][s]; }
     if (sz) { in.sp[4] = p.s[S_HXZ][s]; in.sp[5] = p.s[S_HYZ][s]; }
-    if (!(sy && sz)) in.h0[0] = HO0[c];
-    if (!(sz && sx)) in.h0[1] = HO1[c];
-    if (!(sx && sy)) in.h0[2] = HO2[c];
+    if (!(sy && sz)) in.h0[0] = ld_at(HO0 + rb, ib);
+    if (!(sz && sx)) in.h0[1] = ld_at(HO1 + rb, ib);
+    if (!(sx && sy)) in.h0[2] = ld_at(HO2 + rb, ib);
   } else {
-    in.h0[0] = HO0[c]; in.h0[1] = HO1[c]; in.h0[2] = HO2[c];
+    in.h0[0] = ld_at(HO0 + rb, ib); in.h0[1] = ld_at(HO1 + rb, ib); in.h0[2] = ld_at(HO2 + rb, ib);
   }
 }
 
 template <typename real>
-__device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const PmlArgs<real>& pw,
-                                             const DftFuse<real>& df, int i, int j, int k, const HCellIn<real>& in,
-                                             real* H0, real* H1, real* H2) {
+__device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const PmlArgs<real>& pw, int i, int j, int k,
+                                             const HCellIn<real>& in, real* H0, real* H1, real* H2) {
   const int c = in.c;
   const real ex = in.ex, ey = in.ey, ez = in.ez, ey_kp = in.ey_kp, ex_kp = in.ex_kp, ez_jp = in.ez_jp,
              ex_jp = in.ex_jp, ez_ip = in.ez_ip, ey_ip = in.ey_ip;
@@ -547,13 +547,12 @@ __device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const Pml
     if (in.sy) { pw.s[S_HXY][s] = hxy; pw.s[S_HZY][s] = hzy; }
     if (in.sz) { pw.s[S_HXZ][s] = hxz; pw.s[S_HYZ][s] = hyz; }
     const real hx = hxy + hxz, hy = hyz + hyx, hz = hzx + hzy;
-    H0[c] = hx;
-    H1[c] = hy;
-    H2[c] = hz;
+    st_at(H0 + in.rb, in.ib, hx);
+    st_at(H1 + in.rb, in.ib, hy);
+    st_at(H2 + in.rb, in.ib, hz);
     put_h_ghost(H0, hx, i, j, k, c, a);
     put_h_ghost(H1, hy, i, j, k, c, a);
     put_h_ghost(H2, hz, i, j, k, c, a);
-    if constexpr (kFuseDftReal<real>) dft_fuse_write(df, i, j, k, ex, ey, ez, hx, hy, hz);
     return;
   }
   const real curleyz = ey_kp - ey, curlezy = -ez_jp + ez;
@@ -562,33 +561,30 @@ __device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const Pml
   const real hx = in.h0[0] + a.ku * (curleyz + curlezy);
   const real hy = in.h0[1] + a.ku * (curlezx + curlexz);
   const real hz = in.h0[2] + a.ku * (curlexy + curleyx);
-  H0[c] = hx;
-  H1[c] = hy;
-  H2[c] = hz;
+  st_at(H0 + in.rb, in.ib, hx);
+  st_at(H1 + in.rb, in.ib, hy);
+  st_at(H2 + in.rb, in.ib, hz);
   put_h_ghost(H0, hx, i, j, k, c, a);
   put_h_ghost(H1, hy, i, j, k, c, a);
   put_h_ghost(H2, hz, i, j, k, c, a);
-  if constexpr (kFuseDftReal<real>) dft_fuse_write(df, i, j, k, ex, ey, ez, hx, hy, hz);
 }
 
 template <typename real>
 __device__ __forceinline__ void fused_h_cell(const FieldArgs<real>& a, const PmlArgs<real>& p,
-                                             const PmlArgs<real>& pw, const DftFuse<real>& df, int i, int j, int k,
-                                             real& cex, real& cey, bool use_carry, const real* E0, const real* E1,
+                                             const PmlArgs<real>& pw, int i, int j, int k, real& cex, real& cey, bool use_carry, const real* E0, const real* E1,
                                              const real* E2, const real* HO0, const real* HO1, const real* HO2,
                                              real* H0, real* H1, real* H2) {
   HCellIn<real> in;
-  h_cell_load(a, p, i, j, k, use_carry, cex, cey, E0, E1, E2, HO0, HO1, HO2, in);
+  h_cell_load(a, p, i, j, k, j, use_carry, cex, cey, E0, E1, E2, HO0, HO1, HO2, in);
   cex = in.ex_kp;
   cey = in.ey_kp;
-  h_cell_store(a, pw, df, i, j, k, in, H0, H1, H2);
+  h_cell_store(a, pw, i, j, k, in, H0, H1, H2);
 }
 
 // H over tiles of KZ planes, each thread marching its (i,j) column; restrict
 // pointers as in e_column (no E array is written here).
 template <typename real, int KZ>
-__device__ __forceinline__ void h_column(const FieldArgs<real>& a, const PmlArgs<real>& p, const DftFuse<real>& df,
-                                         int i, int j, int tz,
+__device__ __forceinline__ void h_column(const FieldArgs<real>& a, const PmlArgs<real>& p, int i, int j, int tz,
                                          const real* __restrict__ E0, const real* __restrict__ E1,
                                          const real* __restrict__ E2, real* __restrict__ H0, real* __restrict__ H1,
                                          real* __restrict__ H2) {
@@ -597,21 +593,15 @@ __device__ __forceinline__ void h_column(const FieldArgs<real>& a, const PmlArgs
   for (int r = 0; r < KZ; ++r) {
     const int k = tz * KZ + r + 1;
     if (k > a.nz) break;
-    fused_h_cell(a, p, p, df, i, j, k, cex, cey, r > 0, E0, E1, E2, H0, H1, H2, H0, H1, H2);
+    fused_h_cell(a, p, p, i, j, k, cex, cey, r > 0, E0, E1, E2, H0, H1, H2, H0, H1, H2);
   }
 }
 
-template <typename real, int KZ>
-__global__ __launch_bounds__(512) void k_fused_h(FieldArgs<real> a, PmlArgs<real> p, DftFuse<real> df) {
-  int tx, ty, tz;
-  if (!tile_of(a, tx, ty, tz)) return;
-  const int i = tx * blockDim.x + threadIdx.x + 1;
-  const int j = ty * blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y) + 1;  // wave-uniform row
-  if (i > a.nx || j > a.ny) return;
-  h_column<real, KZ>(a, p, df, i, j, tz, a.e[0], a.e[1], a.e[2], a.h[0], a.h[1], a.h[2]);
-}
-
 // ---------------------------------------------------------------------------
+// x-face tiles exist in FP32 (build_march_tiles)
+template <typename real>
+constexpr bool kXface = sizeof(real) == 4;
+
 // One-pass step (FUSED engine): the E and the H half step of a time step
 // read from one copy of the fields and written to the other (old: m.eo,
 // m.ho and the splits p.s; new: a.e, a.h and pw.s), so no cell reads a value
@@ -621,7 +611,7 @@ __global__ __launch_bounds__(512) void k_fused_h(FieldArgs<real> a, PmlArgs<real
 //
 //  plain tiles (one dielectric material, no PML cell among the cells they
 //  own, no x- or y-normal source plane; z-normal sources are added per
-//  plane) go to k_march_plain: one wavefront marches the tile through its
+//  plane) go to march_block: one wavefront marches the tile through its
 //  planes and does E and H in one pass, so each field crosses HBM once per
 //  step (12 words per cell where the two-kernel step moves 18).  A plain
 //  tile owns the cells of its x range [xlo, xhi]; every cell whose new E
@@ -631,27 +621,36 @@ __global__ __launch_bounds__(512) void k_fused_h(FieldArgs<real> a, PmlArgs<real
 //  x-face tiles (FP32): plain tiles whose lanes reach into an x PML slab;
 //  those lanes keep the x slab's parts (yx, zx) of E and H and take the
 //  split-field update of a face cell (e_pml_split / h_pml_split, as the
-//  general kernels do), the other lanes the plain one.  They run as a
-//  launch of their own (k_march_plain<real, R, true>), so the plain tiles'
-//  kernel keeps its registers.
+//  general kernels do), the other lanes the plain one.  They share the
+//  plain tiles' launch (k_march).
 //
 //  general tiles (PML, dispersive or mixed materials, other sources, and
 //  the x-slab parts of plain tiles) go to k_gen_e and then k_gen_h, the
-//  fused cell updates of k_fused_e / k_fused_h over the two copies.
+//  fused cell updates of the two-kernel step over the two copies.
+//  Dispersive components are written into the new E in k_gen_e's launch.
 //
 // The arithmetic of every cell is that of the two-kernel step term for
-// term, so both forms give the same bits.  Dispersive components were
-// written into the new E by k_ade before these kernels.
+// term, so both forms give the same bits.
+//
+// Everything of a tile but its lanes' columns is wave-uniform (tile index
+// through readfirstlane): loop control, row and plane tests and addresses
+// are scalar, an access is a scalar plane address plus a 32-bit lane offset.
+// Against per-lane 64-bit addresses the FP32 kernel of 4 rows went from 195
+// to 144 registers and from 1610 to 816 vector instructions; the large grids,
+// bound by HBM, gained 0-2 % (320^3 FP64 113.0 -> 111.1 ms per 96 steps), the
+// registers let the x-face tiles share the launch.
 template <typename real>
 struct MarchArgs {
   const real* eo[3];      // E after the previous step
   const real* ho[3];      // H after the previous step
-  // 8 words per entry; plain tiles: i0, j0, k0, k1, xlo, xhi (owned x
-  // range), material id, x face; general workgroups: x0, x1, j0, j1, k0,
-  // width, k1, face
+};
+
+// 8 words per entry; plain tiles: i0, j0, k0, k1, xlo, xhi (owned x range),
+// material id, x face; general workgroups: x0, x1, j0, j1, k0, width, k1, face
+struct TileList {
   const int32_t* tiles;
-  int32_t ntiles, tper;
-  int32_t nsplit;  // general workgroups: workgroups per entry (its planes, k_gen_e) or 1
+  int32_t n, tper;
+  int32_t nsplit;  // general workgroups: workgroups per entry (its planes, the E update) or 1
 };
 
 
@@ -695,19 +694,32 @@ __device__ __forceinline__ real lane_at(real v, int l) {
 // cell index v of an axis of n cells as a tile sees it: v <= n is the cell
 // itself; v = n+1 is cell 1 on a periodic axis and a dead (zero) ghost
 // otherwise
+template <bool PER>
 __device__ __forceinline__ int march_map(int v, int n, int per, bool& live) {
-  live = v <= n || (v == n + 1 && per);
+  live = v <= n || (PER && v == n + 1 && per);
   return v <= n ? v : 1;
 }
 
 // What a wavefront marches: its columns and rows (physical cells after the
-// periodic wrap) and which of them are live / owned.
+// periodic wrap) and which of them are live / owned.  Everything but ip,
+// the offsets and the lane flags is wave-uniform (scalar registers and
+// branches).  The offsets are byte offsets inside a plane, fixed over the
+// march: an access is a scalar plane address plus one of them, no address
+// arithmetic per load (a plane is below 4 GiB: fdtd_api.hip onepass_fits).
 template <int R>
 struct MarchTile {
-  int ip, i0, ixh, j0, jyh, jrow[R], jxg, jxl, k0, k1;
+  int ip, i0, j0, jyh, jrow[R], k0, k1;
+  uint32_t o[R], oyl, oyh, oxh, oxl;  // rows, row j0-1, row j0+R, columns i0+64 and i0-1
   bool lane_live, lane_own, xh_need, xg_live, yh_live, yh_need;
   bool row_live[R], row_own[R];
+  bool ghosts;  // the tile owns cells on a periodic boundary
 };
+
+// Keeps an offset's widening to 64 bits inside the loop that uses it: hoisted
+// out, the compiler forgets that the offset is an unsigned 32-bit one and
+// adds it to the plane's address per access (a 64-bit VALU add each) instead
+// of letting the access do it.  No instruction.
+__device__ __forceinline__ void opaque(uint32_t& off) { asm volatile("" : "+v"(off)); }
 
 // Old fields of one plane of a plain tile, loaded a plane ahead of use.
 template <typename real, int R>
@@ -764,46 +776,46 @@ __device__ __forceinline__ int xf_row(const XfArgs<real>& x, int j, int k) {
 // the loads stay in flight until the plane that uses them.
 template <typename real, int R, bool XF>
 __device__ __forceinline__ void plain_load(const FieldArgs<real>& a, const MarchArgs<real>& m, const XfArgs<real>& x,
-                                           const XfLane<real>& xl, const MarchTile<R>& w, int k,
+                                           const XfLane<real>& xl, MarchTile<R>& w, int k,
                                            PlainPlane<real, R>& P) {
-  const int px = a.px;
-  const int kb = a.pxy * k;
+  const int64_t kb = (int64_t)a.pxy * k;
+#pragma unroll
+  for (int r = 0; r < R; ++r) opaque(w.o[r]);
+  opaque(w.oyl);
+  opaque(w.oyh);
+  opaque(w.oxh);
+  opaque(w.oxl);
+  const real *e0 = m.eo[0] + kb, *e1 = m.eo[1] + kb, *e2 = m.eo[2] + kb;
+  const real *h0 = m.ho[0] + kb, *h1 = m.ho[1] + kb, *h2 = m.ho[2] + kb;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int c = kb + w.ip + px * w.jrow[r];
-    P.ex[r] = m.eo[0][c];
-    P.ey[r] = m.eo[1][c];
-    P.ez[r] = m.eo[2][c];
-    P.hx[r] = m.ho[0][c];
-    P.hy[r] = m.ho[1][c];
-    P.hz[r] = m.ho[2][c];
+    P.ex[r] = ld_at(e0, w.o[r]);
+    P.ey[r] = ld_at(e1, w.o[r]);
+    P.ez[r] = ld_at(e2, w.o[r]);
+    P.hx[r] = ld_at(h0, w.o[r]);
+    P.hy[r] = ld_at(h1, w.o[r]);
+    P.hz[r] = ld_at(h2, w.o[r]);
   }
-  {  // row j0-1 (a real row or the ghost row 0)
-    const int c = kb + w.ip + px * (w.j0 - 1);
-    P.yl_hz = m.ho[2][c];
-    P.yl_hx = m.ho[0][c];
-  }
+  // row j0-1 (a real row or the ghost row 0)
+  P.yl_hz = ld_at(h2, w.oyl);
+  P.yl_hx = ld_at(h0, w.oyl);
   if (w.yh_need) {  // row j0+R
-    const int c = kb + w.ip + px * w.jyh;
-    P.yh_ex = m.eo[0][c];
-    P.yh_ez = m.eo[2][c];
-    P.yh_hx = m.ho[0][c];
-    P.yh_hy = m.ho[1][c];
-    P.yh_hz = m.ho[2][c];
+    P.yh_ex = ld_at(e0, w.oyh);
+    P.yh_ez = ld_at(e2, w.oyh);
+    P.yh_hx = ld_at(h0, w.oyh);
+    P.yh_hy = ld_at(h1, w.oyh);
+    P.yh_hz = ld_at(h2, w.oyh);
   }
   if (w.xh_need) {  // column i0+64, one row per lane 0..R (lane 0: row j0-1, Hx only)
-    const int c = kb + w.ixh + px * w.jxg;
-    P.xh_hx = m.ho[0][c];
-    P.xh_ey = m.eo[1][c];
-    P.xh_ez = m.eo[2][c];
-    P.xh_hy = m.ho[1][c];
-    P.xh_hz = m.ho[2][c];
+    P.xh_hx = ld_at(h0, w.oxh);
+    P.xh_ey = ld_at(e1, w.oxh);
+    P.xh_ez = ld_at(e2, w.oxh);
+    P.xh_hy = ld_at(h1, w.oxh);
+    P.xh_hz = ld_at(h2, w.oxh);
   }
-  {  // column i0-1 (a real column or the ghost column 0), one row per lane
-    const int c = kb + (w.i0 - 1) + px * w.jxl;
-    P.xl_hz = m.ho[2][c];
-    P.xl_hy = m.ho[1][c];
-  }
+  // column i0-1 (a real column or the ghost column 0), one row per lane
+  P.xl_hz = ld_at(h2, w.oxl);
+  P.xl_hy = ld_at(h1, w.oxl);
   if constexpr (XF) {
     if (xl.on) {
 #pragma unroll
@@ -851,19 +863,19 @@ __device__ __forceinline__ real plain_e(const PlainCoef<real>& q, int c, real e0
   return ev;
 }
 
-template <typename real, int R, bool XF>
+template <typename real, int R, bool XF, bool PER>
 __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const MarchArgs<real>& m,
                                             const XfArgs<real>& x, const XfLane<real>& xl,
                                             const SrcArgs<real>& src, int nsrc, PlainCoef<real> q,
-                                            const MarchTile<R>& w, int lane, int k,
+                                            MarchTile<R>& w, int lane, int k,
                                             const PlainPlane<real, R>& cur, PlainPlane<real, R>& nxt,
                                             PlainCarry<real, R>& c) {
   if (k + 1 <= w.k1 + 1) {
     bool lv;
-    plain_load<real, R, XF>(a, m, x, xl, w, march_map(k + 1, a.nz, a.per[2], lv), nxt);
+    plain_load<real, R, XF>(a, m, x, xl, w, march_map<PER>(k + 1, a.nz, a.per[2], lv), nxt);
   }
   bool live_k;
-  const int kk = march_map(k, a.nz, a.per[2], live_k);
+  const int kk = march_map<PER>(k, a.nz, a.per[2], live_k);
   const bool store_k = k <= w.k1;
   // this plane's z-normal sources (wave-uniform), in source order
   q.sv[0] = q.sv[1] = q.sv[2] = 0;
@@ -959,17 +971,21 @@ __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const Marc
     xez = live ? ez : (real)0;
   }
   // stores of the new E of plane k
-  if (store_k) {
+  if (store_k && w.lane_own) {
+    const int64_t kb = (int64_t)a.pxy * kk;
+    real *e0 = a.e[0] + kb, *e1 = a.e[1] + kb, *e2 = a.e[2] + kb;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      if (!(w.lane_own && w.row_own[r])) continue;
-      const int cc = w.ip + a.px * w.jrow[r] + a.pxy * kk;
-      a.e[0][cc] = exn[r];
-      a.e[1][cc] = eyn[r];
-      a.e[2][cc] = ezn[r];
-      put_e_ghost(a.e[0], exn[r], w.ip, w.jrow[r], kk, cc, a);
-      put_e_ghost(a.e[1], eyn[r], w.ip, w.jrow[r], kk, cc, a);
-      put_e_ghost(a.e[2], ezn[r], w.ip, w.jrow[r], kk, cc, a);
+      if (!w.row_own[r]) continue;
+      st_at(e0, w.o[r], exn[r]);
+      st_at(e1, w.o[r], eyn[r]);
+      st_at(e2, w.o[r], ezn[r]);
+      if (PER && w.ghosts) {
+        const int64_t cc = w.ip + a.px * w.jrow[r] + kb;
+        put_e_ghost(a.e[0], exn[r], w.ip, w.jrow[r], kk, cc, a);
+        put_e_ghost(a.e[1], eyn[r], w.ip, w.jrow[r], kk, cc, a);
+        put_e_ghost(a.e[2], ezn[r], w.ip, w.jrow[r], kk, cc, a);
+      }
       if constexpr (XF) {
         if (xl.on) {
           const int sc = xl.sb + xf_row(x, w.jrow[r], kk);
@@ -981,6 +997,8 @@ __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const Marc
   }
   // new H of plane k-1 (myfdtd_func.f90:45-64)
   if (k > w.k0) {
+    const int64_t kb = (int64_t)a.pxy * (k - 1);
+    real *h0 = a.h[0] + kb, *h1 = a.h[1] + kb, *h2 = a.h[2] + kb;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const real ez_jp = r < R - 1 ? c.ez[r + 1] : c.yh_ez;
@@ -1013,13 +1031,15 @@ __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const Marc
           x.hn[1][sc] = n[1];
         }
       }
-      const int cc = w.ip + a.px * w.jrow[r] + a.pxy * kh;
-      a.h[0][cc] = hx;
-      a.h[1][cc] = hy;
-      a.h[2][cc] = hz;
-      put_h_ghost(a.h[0], hx, w.ip, w.jrow[r], kh, cc, a);
-      put_h_ghost(a.h[1], hy, w.ip, w.jrow[r], kh, cc, a);
-      put_h_ghost(a.h[2], hz, w.ip, w.jrow[r], kh, cc, a);
+      st_at(h0, w.o[r], hx);
+      st_at(h1, w.o[r], hy);
+      st_at(h2, w.o[r], hz);
+      if (PER && w.ghosts) {
+        const int64_t cc = w.ip + a.px * w.jrow[r] + kb;
+        put_h_ghost(a.h[0], hx, w.ip, w.jrow[r], kh, cc, a);
+        put_h_ghost(a.h[1], hy, w.ip, w.jrow[r], kh, cc, a);
+        put_h_ghost(a.h[2], hz, w.ip, w.jrow[r], kh, cc, a);
+      }
     }
   }
 #pragma unroll
@@ -1052,22 +1072,23 @@ __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const Marc
 // from halos it loads and recomputes itself: row j0-1 (old Hz, Hx), row
 // j0+R (its new Ex, Ez), column i0-1 (old Hz, Hy: lanes 0..R gather one
 // row each), column i0+64 (its new Ey, Ez: lanes 1..R), plane k1+1 (its new
-// E).  No LDS and no barrier.
-template <typename real, int R, bool XF>
-__global__ __launch_bounds__(256) void k_march_plain(FieldArgs<real> a, MarchArgs<real> m, SrcArgs<real> src,
-                                                     int nsrc, XfArgs<real> x) {
+// E).  No LDS and no barrier.  PER: some axis is periodic (the ghost stores
+// and the wrapped maps cost registers and scalar branches per row and plane,
+// so the handles without a periodic axis run a kernel without them).
+template <typename real, int R, bool XF, bool PER>
+__device__ __forceinline__ void march_block(const FieldArgs<real>& a, const MarchArgs<real>& m, const TileList& tl,
+                                            const SrcArgs<real>& src, int nsrc, const XfArgs<real>& x, int b) {
   const int lane = threadIdx.x & 63;
-  const int b = blockIdx.x;
-  const int lb = a.xcdmap ? (b & 7) * m.tper + (b >> 3) : b;
-  const int tile = lb * 4 + (int)(threadIdx.x >> 6);
-  if (tile >= m.ntiles) return;  // whole wavefront
-  const int32_t* T = m.tiles + 8 * tile;
+  const int tile = deal(b, tl.tper, a.xcdmap) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (tile >= tl.n) return;  // whole wavefront
+  const int32_t* T = tl.tiles + 8 * tile;
   MarchTile<R> w;
-  w.i0 = T[0];
-  w.j0 = T[1];
-  w.k0 = T[2];
-  w.k1 = T[3];
-  const int xlo = T[4], xhi = T[5], mid = T[6];
+  w.i0 = __builtin_amdgcn_readfirstlane(T[0]);
+  w.j0 = __builtin_amdgcn_readfirstlane(T[1]);
+  w.k0 = __builtin_amdgcn_readfirstlane(T[2]);
+  w.k1 = __builtin_amdgcn_readfirstlane(T[3]);
+  const int xlo = __builtin_amdgcn_readfirstlane(T[4]), xhi = __builtin_amdgcn_readfirstlane(T[5]);
+  const int mid = __builtin_amdgcn_readfirstlane(T[6]);
   PlainCoef<real> q;
   {
     const Vec4<real> cf = a.coef[mid], gx = a.gaxe[mid];
@@ -1077,48 +1098,58 @@ __global__ __launch_bounds__(256) void k_march_plain(FieldArgs<real> a, MarchArg
     }
     q.r = cf.v[3];
   }
+  constexpr uint32_t ws = sizeof(real);
+  const uint32_t pxb = (uint32_t)a.px * ws;
   // lanes xlo..xhi are owned; lane xhi+1 supplies the new E after the
   // range (the next cell, or the wrapped cell 1)
-  w.ip = march_map(w.i0 + lane, a.nx, a.per[0], w.lane_live);
+  w.ip = march_map<PER>(w.i0 + lane, a.nx, a.per[0], w.lane_live);
   w.lane_live = w.lane_live && w.i0 + lane >= xlo && w.i0 + lane <= xhi + 1;
   w.lane_own = w.i0 + lane >= xlo && w.i0 + lane <= xhi;
+  const uint32_t ib = (uint32_t)w.ip * ws;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    w.jrow[r] = march_map(w.j0 + r, a.ny, a.per[1], w.row_live[r]);
+    w.jrow[r] = march_map<PER>(w.j0 + r, a.ny, a.per[1], w.row_live[r]);
     w.row_own[r] = w.j0 + r <= a.ny;
+    w.o[r] = ib + pxb * (uint32_t)w.jrow[r];
   }
+  w.oyl = ib + pxb * (uint32_t)(w.j0 - 1);
   // halo row j0+R: needed when the last tile row is owned
   w.yh_need = w.j0 + R - 1 <= a.ny;
-  w.jyh = march_map(w.j0 + R, a.ny, a.per[1], w.yh_live);
+  w.jyh = march_map<PER>(w.j0 + R, a.ny, a.per[1], w.yh_live);
+  w.oyh = ib + pxb * (uint32_t)w.jyh;
   // halo column i0+64: needed when lane 63 is owned
   w.xh_need = xhi == w.i0 + 63;
   bool xh_live;
-  w.ixh = march_map(w.i0 + 64, a.nx, a.per[0], xh_live);
+  const int ixh = march_map<PER>(w.i0 + 64, a.nx, a.per[0], xh_live);
   // gather rows: column i0+64 lane q -> row j0-1+q (q = 0..R; lane 0 only
   // supplies Hx), column i0-1 lane q -> tile row q (q < R) or the halo row
   {
     const int g = min(lane, R);
     bool lv;
-    w.jxg = g == 0 ? w.j0 - 1 : march_map(w.j0 + g - 1, a.ny, a.per[1], lv);
+    const int jxg = g == 0 ? w.j0 - 1 : march_map<PER>(w.j0 + g - 1, a.ny, a.per[1], lv);
     w.xg_live = xh_live && (g == 0 || lv);
-    w.jxl = march_map(w.j0 + g, a.ny, a.per[1], lv);
+    w.oxh = (uint32_t)ixh * ws + pxb * (uint32_t)jxg;
+    const int jxl = march_map<PER>(w.j0 + g, a.ny, a.per[1], lv);
+    w.oxl = (uint32_t)(w.i0 - 1) * ws + pxb * (uint32_t)jxl;
   }
+  w.ghosts = PER && ((a.per[0] && (xlo == 1 || xhi == a.nx)) || (a.per[1] && (w.j0 == 1 || w.j0 + R > a.ny)) ||
+             (a.per[2] && (w.k0 == 1 || w.k1 == a.nz)));
   PlainCarry<real, R> c;
   {
     // old Hx, Hy of plane k0-1 (a real plane or the ghost plane 0) for the
     // k-1 terms of plane k0
-    const int kb = a.pxy * (w.k0 - 1);
+    const int64_t kb = (int64_t)a.pxy * (w.k0 - 1);
+    const real *h0 = m.ho[0] + kb, *h1 = m.ho[1] + kb;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int cc = kb + w.ip + a.px * w.jrow[r];
-      c.hx[r] = m.ho[0][cc];
-      c.hy[r] = m.ho[1][cc];
+      c.hx[r] = ld_at(h0, w.o[r]);
+      c.hy[r] = ld_at(h1, w.o[r]);
       c.hz[r] = 0;
       c.ex[r] = c.ey[r] = c.ez[r] = 0;
     }
-    c.yh_hy = m.ho[1][kb + w.ip + a.px * w.jyh];
+    c.yh_hy = ld_at(h1, w.oyh);
     c.yh_ex = c.yh_ez = 0;
-    c.xh_hx = m.ho[0][kb + w.ixh + a.px * w.jxg];
+    c.xh_hx = ld_at(h0, w.oxh);
     c.xh_ey = c.xh_ez = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) c.ph_yx[r] = c.ph_zx[r] = 0;
@@ -1128,7 +1159,7 @@ __global__ __launch_bounds__(256) void k_march_plain(FieldArgs<real> a, MarchArg
   XfLane<real> xl{};
   if constexpr (XF) {
     const int i = w.ip;
-    xl.on = T[7] != 0 && (i <= x.Px || i > a.nx - x.Px);
+    xl.on = __builtin_amdgcn_readfirstlane(T[7]) != 0 && (i <= x.Px || i > a.nx - x.Px);
     if (xl.on) {
       const bool hi = i > x.Px;  // as pml_index (the slabs never overlap: 2 Px <= nx)
       xl.sb = x.base + (hi ? x.hioff + (i - (a.nx - x.Px + 1)) : i - 1);
@@ -1141,15 +1172,15 @@ __global__ __launch_bounds__(256) void k_march_plain(FieldArgs<real> a, MarchArg
   PlainPlane<real, R> A, B;
   plain_load<real, R, XF>(a, m, x, xl, w, w.k0, A);
   for (int k = w.k0; k <= w.k1 + 1; k += 2) {
-    plain_plane<real, R, XF>(a, m, x, xl, src, nsrc, q, w, lane, k, A, B, c);
-    if (k + 1 <= w.k1 + 1) plain_plane<real, R, XF>(a, m, x, xl, src, nsrc, q, w, lane, k + 1, B, A, c);
+    plain_plane<real, R, XF, PER>(a, m, x, xl, src, nsrc, q, w, lane, k, A, B, c);
+    if (k + 1 <= w.k1 + 1) plain_plane<real, R, XF, PER>(a, m, x, xl, src, nsrc, q, w, lane, k + 1, B, A, c);
   }
 }
 
 // General work: workgroup = 256 threads over cells x0..x1 x j0..j1 of
 // planes k0..k1 (list entry: x0, x1, j0, j1, k0, width, k1, face), 64 x 4 cells
 // (a wavefront is one row), 32 x 8 or 16 x 16 (narrow boxes: the x edges),
-// the fused cell updates over the two copies.  k_gen_e reads the old H and
+// the fused cell updates over the two copies.  gen_e_block reads the old H and
 // E and writes the new E, one cell per thread, a workgroup per plane (the
 // planes of an entry dealt to neighbouring workgroups, so a plane's
 // neighbour below is still in L2);
@@ -1161,34 +1192,33 @@ __global__ __launch_bounds__(256) void k_march_plain(FieldArgs<real> a, MarchArg
 // cell per thread; the E update marched so holds too many registers and
 // runs slower).
 template <typename real>
-__device__ __forceinline__ bool gen_cell(const FieldArgs<real>& a, const MarchArgs<real>& m, int& i, int& j, int& k0,
+__device__ __forceinline__ bool gen_cell(const FieldArgs<real>& a, const TileList& tl, int b, int& i, int& j, int& jb, int& k0,
                                          int& k1, bool& wide, int& pl, int& face) {
-  const int b = blockIdx.x;
-  int lb = a.xcdmap ? (b & 7) * m.tper + (b >> 3) : b;
-  if (lb >= m.ntiles * m.nsplit) return false;
-  pl = lb % m.nsplit;
-  lb /= m.nsplit;
-  const int32_t* T = m.tiles + 8 * lb;
+  int lb = deal(b, tl.tper, a.xcdmap);
+  if (lb >= tl.n * tl.nsplit) return false;
+  pl = lb % tl.nsplit;
+  lb /= tl.nsplit;
+  const int32_t* T = tl.tiles + 8 * lb;
   const int bw = T[5];
   wide = bw == 64;
   const int t = (int)threadIdx.x;
   i = T[0] + (t & (bw - 1));
-  j = T[2] + (wide ? __builtin_amdgcn_readfirstlane(t >> 6) : t / bw);
+  jb = T[2];
+  j = jb + (wide ? __builtin_amdgcn_readfirstlane(t >> 6) : t / bw);
   k0 = T[4];
   k1 = T[6];
   face = T[7];
   return i <= T[1] && j <= T[3];
 }
 
-// FP32: eight wavefronts per SIMD (the compiler keeps some kernel arguments
-// in vector registers to fit), 8 % faster than the seven its register use
-// otherwise allows; the kernel waits on memory for most of its life
+// a.h: the old H, a.e: the new E
 template <typename real>
-__global__ __launch_bounds__(256, sizeof(real) == 4 ? 8 : 5) void k_gen_e(FieldArgs<real> a, PmlArgs<real> p, PmlArgs<real> pw,
-                                               MarchArgs<real> m, SrcArgs<real> src, int nsrc) {
-  int i, j, k0, k1, pl, face;
+__device__ __forceinline__ void gen_e_block(const FieldArgs<real>& a, const PmlArgs<real>& p, const PmlArgs<real>& pw,
+                                            const MarchArgs<real>& m, const TileList& tl, const SrcArgs<real>& src,
+                                            int nsrc, int b) {
+  int i, j, jb, k0, k1, pl, face;
   bool wide;
-  if (!gen_cell(a, m, i, j, k0, k1, wide, pl, face)) return;
+  if (!gen_cell(a, tl, b, i, j, jb, k0, k1, wide, pl, face)) return;
   const int k = k0 + pl;
   if (k > k1) return;
   real sv[3] = {0, 0, 0};
@@ -1221,32 +1251,31 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 8 : 5) void k_gen_e(FieldA
 // one (i, j) column of planes k0..k1, pipelined by hand (see above)
 template <typename real, int FACE>
 __device__ __forceinline__ void gen_h_column(const FieldArgs<real>& a, const PmlArgs<real>& p, const PmlArgs<real>& pw,
-                                             const MarchArgs<real>& m, int i, int j, int k0, int k1) {
-  const DftFuse<real> df{};
+                                             const MarchArgs<real>& m, int i, int j, int jb, int k0, int k1) {
   HCellIn<real> cur, nxt;
-  h_cell_load<real, FACE>(a, p, i, j, k0, false, (real)0, (real)0, a.e[0], a.e[1], a.e[2], m.ho[0], m.ho[1],
+  h_cell_load<real, FACE>(a, p, i, j, k0, jb, false, (real)0, (real)0, a.e[0], a.e[1], a.e[2], m.ho[0], m.ho[1],
                           m.ho[2], cur);
   for (int k = k0; k <= k1; ++k) {
     const int kn = min(k + 1, k1);
-    h_cell_load<real, FACE>(a, p, i, j, kn, kn > k, cur.ex_kp, cur.ey_kp, a.e[0], a.e[1], a.e[2], m.ho[0],
+    h_cell_load<real, FACE>(a, p, i, j, kn, jb, kn > k, cur.ex_kp, cur.ey_kp, a.e[0], a.e[1], a.e[2], m.ho[0],
                             m.ho[1], m.ho[2], nxt);
-    h_cell_store(a, pw, df, i, j, k, cur, a.h[0], a.h[1], a.h[2]);
+    h_cell_store(a, pw, i, j, k, cur, a.h[0], a.h[1], a.h[2]);
     cur = nxt;
   }
 }
 
 template <typename real>
 __global__ __launch_bounds__(256) void k_gen_h(FieldArgs<real> a, PmlArgs<real> p, PmlArgs<real> pw,
-                                               MarchArgs<real> m) {
-  int i, j, k0, k1, pl, face;
+                                               MarchArgs<real> m, TileList tl) {
+  int i, j, jb, k0, k1, pl, face;
   bool wide;
-  if (!gen_cell(a, m, i, j, k0, k1, wide, pl, face)) return;
+  if (!gen_cell(a, tl, (int)blockIdx.x, i, j, jb, k0, k1, wide, pl, face)) return;
   if (face == 2)
-    gen_h_column<real, 2>(a, p, pw, m, i, j, k0, k1);
+    gen_h_column<real, 2>(a, p, pw, m, i, j, jb, k0, k1);
   else if (face == 1)
-    gen_h_column<real, 1>(a, p, pw, m, i, j, k0, k1);
+    gen_h_column<real, 1>(a, p, pw, m, i, j, jb, k0, k1);
   else
-    gen_h_column<real, 0>(a, p, pw, m, i, j, k0, k1);
+    gen_h_column<real, 0>(a, p, pw, m, i, j, jb, k0, k1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1348,9 +1377,11 @@ __global__ __launch_bounds__(256) void k_ade(FieldArgs<real> a, AdeCoef<double> 
   ade_cell<real, FUSED>(a, co, cells, masks, state, n, src, nsrc, e);
 }
 
-// Several groups in one launch (the one-pass step): group q takes blocks
-// blk[q] .. blk[q+1]-1.  A small group alone is a short launch that leaves
-// most of the GPU idle, and every launch boundary costs a drain.
+// Up to kAdeMulti Drude/CP/Raman groups as a part of an E launch: group q
+// takes blocks blk[q] .. blk[q+1]-1.  The FUSED forms advance D here and
+// write components no other part writes.  The coefficients come as kernel
+// arguments: read through a pointer, they were loaded again after every store
+// of the state (11 -> 21 us for one 9,000-cell group alone).
 constexpr int kAdeMulti = 4;
 struct AdeMulti {
   int32_t ng;
@@ -1363,13 +1394,19 @@ struct AdeMulti {
 };
 
 template <typename real>
-__global__ __launch_bounds__(256) void k_ade_multi(FieldArgs<real> a, AdeMulti g, SrcArgs<real> src, int nsrc) {
-  const int b = (int)blockIdx.x;
+__device__ __forceinline__ void ade_block(const FieldArgs<real>& a, const AdeMulti& g, const SrcArgs<real>& src,
+                                          int nsrc, int b) {
   int q = 0;
   while (q + 1 < g.ng && b >= g.blk[q + 1]) ++q;
-  const int64_t e = (int64_t)(b - g.blk[q]) * blockDim.x + threadIdx.x;
+  const int64_t e = (int64_t)(b - g.blk[q]) * 256 + threadIdx.x;
   if (e >= g.n[q]) return;
   ade_cell<real, true>(a, g.co[q], g.cells[q], g.masks[q], g.state[q], g.n[q], src, nsrc, e);
+}
+
+// groups past the first kAdeMulti
+template <typename real>
+__global__ __launch_bounds__(256) void k_ade_multi(FieldArgs<real> a, AdeMulti g, SrcArgs<real> src, int nsrc) {
+  ade_block(a, g, src, nsrc, (int)blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1715,19 +1752,21 @@ __global__ __launch_bounds__(256) void k_ref_pml_h(FieldArgs<real> a, RefPmlArgs
 // every gated step copies the plane's selected components into a ring of
 // kDftBlock samples; a flush adds dt * sum_b cos/sin(w t_b) F_b, t_b =
 // (n_b - 1) dt, to the FP64 accumulators [slot][re|im][m][v][u].
-// Every monitor of a step in one launch (each kernel boundary costs about
-// 9 us on this GPU): the samples of up to kMonPlanes DFT planes, each laid
-// out as samples[slot][v][u] (u, v the plane's two free axes in x, y, z
-// order), then the probes.  Plane q owns blocks blk[q] .. blk[q+1]-1,
-// (np+255)/256 per sampled component; the blocks from blk[nplanes] on write
-// the probes.
+// The samples of up to kMonPlanes DFT planes, each laid out as
+// samples[slot][v][u] (u, v the plane's two free axes in x, y, z order), then
+// the probes, as a part of a launch that leaves the fields they read alone
+// (or a launch of their own at the end of a call or a DFT block).  Plane q
+// owns blocks blk[q] .. blk[q+1]-1, (np+255)/256 per sampled component; the
+// blocks from blk[nplanes] on write the probes.  The two-kernel step samples
+// E in its H launch and H in the next step's E launch.
 constexpr int kMonPlanes = 8;
 template <typename real>
 struct MonList {
-  int32_t nplanes, nprobe;
+  int32_t nplanes, nprobe, nblk;
+  int32_t part;            // probes: 1 the time and E, 2 H, 3 all
   int32_t axis[kMonPlanes], index[kMonPlanes], n1[kMonPlanes];
   int64_t np[kMonPlanes];
-  int32_t comp[kMonPlanes][6];
+  uint64_t sel[kMonPlanes];  // byte q: component | slot << 4 of the plane's q-th sample
   real* dst[kMonPlanes];
   int32_t blk[kMonPlanes + 1];
   const int32_t* ppos;
@@ -1735,20 +1774,21 @@ struct MonList {
   double tn;
 };
 
-template <typename real>
-__global__ __launch_bounds__(256) void k_monitors(FieldArgs<real> a, MonList<real> m) {
-  const int b = blockIdx.x;
+// F(c): array of component c (0..2 E, 3..5 H)
+template <typename real, typename Fields>
+__device__ __forceinline__ void mon_block(const MonList<real>& m, int px, int pxy, int b, const Fields& F) {
+  if (b >= m.nblk) return;
   if (b >= m.blk[m.nplanes]) {  // probes (incident-line probes are written by k_tfsf_h)
-    for (int p = (b - m.blk[m.nplanes]) * 256 + (int)threadIdx.x; p < m.nprobe; p += 256 * (int)gridDim.x) {
-      if (m.ppos[3 * p] < 0) continue;
-      const int64_t c = m.ppos[3 * p] + a.px * m.ppos[3 * p + 1] + a.pxy * m.ppos[3 * p + 2];
-      double* r = m.pout + 7 * p;
+    const int p = (b - m.blk[m.nplanes]) * 256 + (int)threadIdx.x;
+    if (p >= m.nprobe || m.ppos[3 * p] < 0) return;
+    const int64_t c = m.ppos[3 * p] + px * m.ppos[3 * p + 1] + pxy * m.ppos[3 * p + 2];
+    double* r = m.pout + 7 * p;
+    if (m.part & 1) {
       r[0] = m.tn;
-      for (int q = 0; q < 3; ++q) {
-        r[1 + q] = (double)a.e[q][c];
-        r[4 + q] = (double)a.h[q][c];
-      }
+      for (int q = 0; q < 3; ++q) r[1 + q] = (double)F(q)[c];
     }
+    if (m.part & 2)
+      for (int q = 3; q < 6; ++q) r[1 + q] = (double)F(q)[c];
     return;
   }
   int q = 0;
@@ -1756,8 +1796,8 @@ __global__ __launch_bounds__(256) void k_monitors(FieldArgs<real> a, MonList<rea
   const int64_t np = m.np[q];
   const int nbx = (int)((np + 255) / 256);
   const int lb = b - m.blk[q];
-  const int slot = lb / nbx;
-  const int64_t o = (int64_t)(lb - slot * nbx) * 256 + threadIdx.x;
+  const int e = lb / nbx;
+  const int64_t o = (int64_t)(lb - e * nbx) * 256 + threadIdx.x;
   if (o >= np) return;
   const int n1 = m.n1[q], axis = m.axis[q];
   const int u = (int)(o % n1) + 1, v = (int)(o / n1) + 1;
@@ -1766,10 +1806,138 @@ __global__ __launch_bounds__(256) void k_monitors(FieldArgs<real> a, MonList<rea
   pc[axis] = m.index[q];
   pc[a1] = u;
   pc[a2] = v;
-  const int64_t c = pc[0] + a.px * pc[1] + a.pxy * pc[2];
-  const int comp = m.comp[q][slot];
-  const real* F = comp < 3 ? a.e[comp] : a.h[comp - 3];
-  m.dst[q][(int64_t)slot * np + o] = F[c];
+  const int64_t c = pc[0] + px * pc[1] + pxy * pc[2];
+  const int sel = (int)(m.sel[q] >> (8 * e)) & 0xff;
+  m.dst[q][(int64_t)(sel >> 4) * np + o] = F(sel & 7)[c];
+}
+
+template <typename real>
+__global__ __launch_bounds__(256) void k_monitors(FieldArgs<real> a, MonList<real> m) {
+  mon_block(m, a.px, a.pxy, (int)blockIdx.x, [&](int c) -> const real* { return c < 3 ? a.e[c] : a.h[c - 3]; });
+}
+
+// ---------------------------------------------------------------------------
+// Launches of the FUSED engine.  Each is a list of parts, every part a range
+// of workgroups, none of which reads what another part of the launch writes:
+// a launch of its own costs a part 4-9 us however little it does (the start
+// of its first wavefronts and the drain of its last ones), which is most of
+// the step on small grids.  Measured with the parts as launches of their own
+// (profiling runs them so, that each has its time) and in two launches a
+// step, the two-kernel form, us a step: 64^3 FP32 25.2 / 14.9, 96^3 FP32
+// 40.0 / 28.4, 96^3 FP64 55.5 / 40.3, 150 x 137 x 211 FP32 periodic under a
+// TFSF wave 103 / 84, 160^3 FP32 91 / 80.
+struct Parts {
+  int32_t mon, ade, mix, xf, plain, gen;  // blocks of each part (0: not in this launch)
+};
+
+// The kernel arguments a cell update needs, loaded in one batch: left to the
+// compiler, each is loaded where it is first used and waited for there, a
+// chain of a dozen scalar loads before the first field load.  No instruction
+// beyond the loads.  FP32 H, 160^3: 36.5 -> 35.0 us; the E update and FP64
+// lose more to the registers it takes (160^3 E 48 -> 54 us).
+template <typename real>
+__device__ __forceinline__ void load_args(const FieldArgs<real>& a, const PmlArgs<real>& p) {
+  asm volatile("" ::"s"(a.e[0]), "s"(a.e[1]), "s"(a.e[2]), "s"(a.h[0]), "s"(a.h[1]), "s"(a.h[2]), "s"(a.nx), "s"(a.ny),
+               "s"(a.nz), "s"(a.px), "s"(a.pxy), "s"(p.P[0]), "s"(p.P[1]), "s"(p.P[2]), "s"(a.per[0]), "s"(a.per[1]),
+               "s"(a.per[2]));
+}
+
+// Two-kernel step, E half: monitors of the step before (H), dispersive
+// cells, rows that mix materials, and the rows with one material id (the
+// table entry is then a wave-uniform scalar load).  A wavefront of the
+// latter marches its 64 columns through KZ planes, carrying H of the plane
+// below in registers (KZ = 1: one plane, nothing carried).
+template <typename real, int KZ, bool LISTS>
+__global__ __launch_bounds__(256) void k_step_e(FieldArgs<real> a, PmlArgs<real> p, SrcArgs<real> src, int nsrc,
+                                                Parts pt, MonList<real> mon, AdeMulti ade, const int32_t* mix,
+                                                SegGrid gm, SegGrid gt) {
+  int b = (int)blockIdx.x;
+  if constexpr (LISTS) {
+    if (b < pt.mon) {
+      mon_block(mon, a.px, a.pxy, b, [&](int c) -> const real* { return c < 3 ? a.e[c] : a.h[c - 3]; });
+      return;
+    }
+    b -= pt.mon;
+    if (b < round8(pt.ade)) {
+      if (b < pt.ade) ade_block(a, ade, src, nsrc, b);
+      return;
+    }
+    b -= round8(pt.ade);
+    if (b < pt.mix) {
+      e_mixed_block(a, p, src, nsrc, mix, gm, b);
+      return;
+    }
+    b -= pt.mix;
+  }
+  int tx, r;
+  if (!seg_of(gt, b, a.xcdmap, tx, r)) return;
+  const int i = tx * 64 + ((int)threadIdx.x & 63) + 1;
+  const int tz = fast_quot(gt.ny, r), j = r - tz * gt.ny.d + 1;
+  if (i > a.nx) return;
+  e_column<real, KZ>(a, p, src, nsrc, i, j, tz, a.h[0], a.h[1], a.h[2], a.e[0], a.e[1], a.e[2]);
+}
+
+// Two-kernel step, H half: monitors of this step (E), every cell.
+template <typename real, int KZ>
+__global__ __launch_bounds__(256) void k_step_h(FieldArgs<real> a, PmlArgs<real> p, Parts pt, MonList<real> mon,
+                                                SegGrid gt) {
+  int b = (int)blockIdx.x;
+  if (b < pt.mon) {
+    mon_block(mon, a.px, a.pxy, b, [&](int c) -> const real* { return c < 3 ? a.e[c] : a.h[c - 3]; });
+    return;
+  }
+  b -= pt.mon;
+  if constexpr (sizeof(real) == 4) load_args(a, p);
+  int tx, r;
+  if (!seg_of(gt, b, a.xcdmap, tx, r)) return;
+  const int i = tx * 64 + ((int)threadIdx.x & 63) + 1;
+  const int tz = fast_quot(gt.ny, r), j = r - tz * gt.ny.d + 1;
+  if (i > a.nx) return;
+  h_column<real, KZ>(a, p, i, j, tz, a.e[0], a.e[1], a.e[2], a.h[0], a.h[1], a.h[2]);
+}
+
+// One-pass step: what reads the old copies and writes the new ones goes in
+// two launches by the registers it needs: the x-face tiles and the plain
+// tiles (the longest workgroups first), then the monitors of the step before,
+// dispersive cells and E of the general cells; H of the general cells
+// (k_gen_h) follows, since it reads E that other workgroups write.
+template <typename real, int R, bool PER>
+__global__ __launch_bounds__(256) void k_march(FieldArgs<real> a, MarchArgs<real> m, SrcArgs<real> src, int nsrc,
+                                               Parts pt, TileList xf, TileList plain, XfArgs<real> x) {
+  int b = (int)blockIdx.x;
+  if (b < pt.xf) {
+    if constexpr (kXface<real>) march_block<real, 2, true, PER>(a, m, xf, src, nsrc, x, b);
+    return;
+  }
+  b -= pt.xf;
+  march_block<real, R, false, PER>(a, m, plain, src, nsrc, x, b);
+}
+
+// a.h: the old H, a.e: the new E.  FP32 runs at eight wavefronts per SIMD
+// (the compiler keeps some kernel arguments in vector registers to fit): the
+// general cells wait on memory for most of their life.
+template <typename real>
+__global__ __launch_bounds__(256, sizeof(real) == 4 ? 8 : 4) void k_gen_e(
+    FieldArgs<real> a, MarchArgs<real> m, PmlArgs<real> p, PmlArgs<real> pw, SrcArgs<real> src, int nsrc, Parts pt,
+    MonList<real> mon, AdeMulti ade, TileList gen) {
+  int b = (int)blockIdx.x;
+  if (b < pt.mon) {
+    mon_block(mon, a.px, a.pxy, b, [&](int c) -> const real* { return c < 3 ? m.eo[c] : m.ho[c - 3]; });
+    return;
+  }
+  b -= pt.mon;
+  if (b < round8(pt.ade)) {
+    if (b < pt.ade) ade_block(a, ade, src, nsrc, b);
+    return;
+  }
+  gen_e_block(a, p, pw, m, gen, src, nsrc, b - round8(pt.ade));
+}
+
+// x-face tiles of 4 rows (FDTD_XFACE_BY=4)
+template <typename real, bool PER>
+__global__ __launch_bounds__(256) void k_xface4(FieldArgs<real> a, MarchArgs<real> m, SrcArgs<real> src, int nsrc,
+                                                TileList xf, XfArgs<real> x) {
+  march_block<real, 4, true, PER>(a, m, xf, src, nsrc, x, (int)blockIdx.x);
 }
 
 // cos/sin table of one block of samples: tab[(b*nfreq + m)*2 + {0,1}]
@@ -1988,7 +2156,7 @@ __global__ __launch_bounds__(256) void k_tfsf_h(FieldArgs<real> a, PmlArgs<real>
   real hv;
   if (all_faces && in_pml(p.P, i, j, k, a.nx, a.ny, a.nz)) {
     // the part of H_q along the axis takes the value; with both parts of
-    // H_q stored, H_q = the two summed as k_fused_h sums them (Hxy+Hxz,
+    // H_q stored, H_q = the two summed as h_cell_store sums them (Hxy+Hxz,
     // Hyz+Hyx, Hzx+Hzy), otherwise H_q takes the value itself (a part not
     // stored is H_q less the other part)
     const int sa = q == 0 ? (L.axis == 1 ? S_HXY : S_HXZ)
@@ -2117,11 +2285,6 @@ FieldArgs<real> field_args(Sim* s) {
   a.px = (int32_t)s->px;
   a.pxy = (int32_t)s->pxy;
   a.ku = (real)s->ku;
-  a.ntx = (s->nx + s->bx - 1) / s->bx;
-  a.nty = (s->ny + s->by - 1) / s->by;
-  a.ntz = s->nz;
-  const int tiles = a.ntx * a.nty * a.ntz;
-  a.tper = (tiles + 7) / 8;
   a.xcdmap = s->xcdmap;
   return a;
 }
@@ -2188,13 +2351,85 @@ struct Timer {
   }
 };
 
-template <typename real>
-inline dim3 tile_grid(const FieldArgs<real>& a) {
-  const int tiles = a.ntx * a.nty * a.ntz;
-  return dim3((unsigned)(a.xcdmap ? 8 * a.tper : tiles));
+// From this many workgroups of plain rows on, the lists of a two-kernel E
+// launch have a launch of their own: beside them the rows' kernel holds the
+// registers of the dispersive update (FP32: seven wavefronts a SIMD instead of
+// eight), which costs more than a launch once the rows fill the GPU many
+// times over.  FP32 cubes with a gold sphere, one launch against two, us a
+// step: 128 cells a side 46 / 52, 160: 89 / 92, 203: 195 / 192, 256: 361 / 356.
+constexpr int kListsApart = 32768;
+
+// the segment grid of `rows` rows of nx cells (SegGrid) and its blocks
+inline SegGrid seg_grid(int nx, int ny, int64_t rows, int* blocks) {
+  SegGrid g;
+  g.ntx = fast_div((nx + 63) / 64);
+  g.ny = fast_div(ny);
+  g.n = (int32_t)(g.ntx.d * rows);
+  const int nb = (g.n + 3) / 4;  // four wavefronts a workgroup
+  g.tper = (nb + 7) / 8;
+  *blocks = 8 * g.tper;
+  return g;
 }
 
-// 8 XCD runs of `per` blocks of 4 wavefronts (seg_work undoes the dealing)
+// ---- monitors ----------------------------------------------------------------
+// What is still to be sampled of the last step made: its DFT planes (the
+// components `sel` names) and its probes.
+template <typename real>
+void mon_add(MonList<real>& m, const MonPend& q) {
+  const int n = m.nplanes++;
+  m.axis[n] = q.axis;
+  m.index[n] = q.index;
+  m.n1[n] = q.n1;
+  m.np[n] = q.np;
+  m.sel[n] = q.sel;
+  m.dst[n] = (real*)q.dst;
+  m.blk[n + 1] = m.blk[n] + (int32_t)((q.np + 255) / 256) * q.nsel;
+}
+template <typename real>
+void mon_probes(Sim* s, MonList<real>& m, double* out, double tn, int part) {
+  m.nprobe = (int)s->probes.size();
+  m.ppos = (const int32_t*)s->d_probe_pos;
+  m.pout = out;
+  m.tn = tn;
+  m.part = part;
+}
+template <typename real>
+void mon_close(MonList<real>& m) {
+  m.nblk = m.blk[m.nplanes] + (m.nprobe > 0 ? (m.nprobe + 255) / 256 : 0);
+}
+
+template <typename real>
+void launch_monitors(Sim* s, MonList<real>& m) {
+  mon_close(m);
+  if (!m.nblk) return;
+  Timer tm(s, FDTD_K_MON);
+  hipLaunchKernelGGL(k_monitors<real>, dim3((unsigned)m.nblk), dim3(256), 0, s->stream, field_args<real>(s), m);
+}
+
+// The pending samples as a list a launch can take along; the planes that do
+// not fit the list are sampled by launches of their own.
+template <typename real>
+MonList<real> take_pending(Sim* s) {
+  MonList<real> m{};
+  size_t q = 0;
+  for (; s->mon_pend.size() - q > (size_t)kMonPlanes;) {
+    MonList<real> o{};
+    for (int e = 0; e < kMonPlanes; ++e) mon_add(o, s->mon_pend[q++]);
+    launch_monitors(s, o);
+  }
+  for (; q < s->mon_pend.size(); ++q) mon_add(m, s->mon_pend[q]);
+  if (s->probe_part) mon_probes(s, m, s->probe_out, s->probe_tn, s->probe_part);
+  s->mon_pend.clear();
+  s->probe_part = 0;
+  mon_close(m);
+  return m;
+}
+
+template <typename real>
+void flush_pending(Sim* s) {
+  MonList<real> m = take_pending<real>(s);
+  launch_monitors(s, m);
+}
 
 inline dim3 cell_grid(int nx, int nrows, int nz, dim3 blk) {
   return dim3((unsigned)((nx + blk.x - 1) / blk.x), (unsigned)((nrows + blk.y - 1) / blk.y), (unsigned)nz);
@@ -2245,6 +2480,7 @@ SrcArgs<real> source_args(Sim* s, int n, int* nsrc) {
 template <typename real>
 void dft_flush_plane(Sim* s, DftPlane& d) {
   if (d.nbuf == 0) return;
+  flush_pending<real>(s);
   const int64_t np = (int64_t)d.n1 * d.n2;
   Timer tm(s, FDTD_K_MON);
   const int nt = d.nfreq * d.nbuf;
@@ -2261,7 +2497,6 @@ void dft_flush_plane(Sim* s, DftPlane& d) {
 template <typename real>
 int step_impl(Sim* s) {
   const int n = s->n_done + 1;
-  const double t = (double)(n - 1) * s->dt;
   FieldArgs<real> a = field_args<real>(s);
   int nsrc = 0;
   SrcArgs<real> src = source_args<real>(s, n, &nsrc);
@@ -2277,6 +2512,38 @@ int step_impl(Sim* s) {
     LordCoef c = g.ld;
     c.ku = s->ku;
     return c;
+  };
+
+  // the Drude/CP/Raman groups, kAdeMulti at a time: the first list goes with
+  // an E launch (their blocks in *blocks), the others have launches of their own
+  auto ade_lists = [&](const FieldArgs<real>& af, int* blocks) {
+    AdeMulti first{}, g{};
+    bool have = false;
+    auto done = [&]() {
+      if (!g.ng) return;
+      if (!have) {
+        first = g;
+        have = true;
+      } else {
+        Timer tm(s, FDTD_K_ADE);
+        hipLaunchKernelGGL(k_ade_multi<real>, dim3((unsigned)g.blk[g.ng]), dim3(256), 0, st, af, g, src, nsrc);
+      }
+      g = AdeMulti{};
+    };
+    for (auto& G : s->groups) {
+      if (G.kind != 0 || !G.ncells) continue;
+      const int q = g.ng++;
+      g.co[q] = ade_coef(G);
+      g.cells[q] = G.d_cells;
+      g.masks[q] = G.d_mask;
+      g.state[q] = (double*)G.d_state;
+      g.n[q] = G.ncells;
+      g.blk[q + 1] = g.blk[q] + (int32_t)((G.ncells + 255) / 256);
+      if (g.ng == kAdeMulti) done();
+    }
+    done();
+    *blocks = first.blk[first.ng];
+    return first;
   };
 
   // TFSF lines: E half step after the main E stage (the D terms above read
@@ -2308,30 +2575,41 @@ int step_impl(Sim* s) {
                          (double)n * s->dt, n1, n2);
     }
   };
-  // FP32 two-kernel steps: this step's monitor samples are written by the
-  // H kernel (not with a TFSF wave: its H correction follows it); dry steps
-  // write them too, into the ring slot the next real step overwrites
-  auto fused_monitors = [&]() {
-    DftFuse<real> df{};
-    if (kFuseDftReal<real> && s->dft_fuse && s->tfsfs.empty()) {
-      for (auto& d : s->dfts) {
-        if (df.n == kFuseDft) break;
-        if (n < d.n_begin || (d.n_end > 0 && n > d.n_end)) continue;
-        const int q = df.n++;
-        int ns = 0;
-        for (int c = 0; c < 6; ++c)
-          if (d.mask & (1 << c)) df.comp[q][ns++] = c;
-        df.axis[q] = d.axis;
-        df.index[q] = d.index;
-        df.n1[q] = d.n1;
-        df.ns[q] = ns;
-        df.np[q] = (int64_t)d.n1 * d.n2;
-        df.dst[q] = (real*)d.d_samp + (int64_t)d.nbuf * ns * df.np[q];
-        d.fused_now = true;
+  // this step's samples: the planes open at step n with their ring slots
+  // (dry steps write them too, into the slot the next real step overwrites);
+  // comps bit c selects component c
+  auto sample = [&](int comps, auto&& take) {
+    for (auto& d : s->dfts) {
+      if (n < d.n_begin || (d.n_end > 0 && n > d.n_end)) continue;
+      MonPend q{};
+      int slot = 0;
+      for (int c = 0; c < 6; ++c) {
+        if (!(d.mask & (1 << c))) continue;
+        if (comps & (1 << c)) q.sel |= (uint64_t)(c | slot << 4) << (8 * q.nsel++);
+        ++slot;
       }
+      if (!q.nsel) continue;
+      q.axis = d.axis;
+      q.index = d.index;
+      q.n1 = d.n1;
+      q.np = (int64_t)d.n1 * d.n2;
+      q.dst = (real*)d.d_samp + (int64_t)d.nbuf * slot * q.np;
+      take(q);
     }
-    return df;
   };
+  const bool probes_on = !s->probes.empty() && !s->dry;
+  double* probe_row =
+      probes_on ? s->d_probe + (int64_t)7 * (int64_t)s->probes.size() * (s->probe_row0 + (n - 1 - s->call_base)) : nullptr;
+  auto pend = [&](int comps, int part) {  // left to the next step's first launch, or the end of the call
+    sample(comps, [&](const MonPend& q) { s->mon_pend.push_back(q); });
+    if (probes_on) {
+      s->probe_part = part;
+      s->probe_out = probe_row;
+      s->probe_tn = (double)n * s->dt;
+    }
+  };
+  // profiling: every part a launch of its own, timed
+  const bool apart = s->profiling;
   if (s->engine == FDTD_ENGINE_FUSED && s->onepass) {
     // new fields go to the second copies, then the copies swap roles
     FieldArgs<real> an = a;
@@ -2339,35 +2617,13 @@ int step_impl(Sim* s) {
       an.e[q] = (real*)s->E2[q];
       an.h[q] = (real*)s->H2[q];
     }
-    {
-      FieldArgs<real> ad = a;  // D form from the old H into the new E
-      for (int q = 0; q < 3; ++q) ad.e[q] = an.e[q];
-      AdeMulti gm{};
-      auto launch_multi = [&]() {
-        if (!gm.ng) return;
-        Timer tm(s, FDTD_K_ADE);
-        hipLaunchKernelGGL(k_ade_multi<real>, dim3((unsigned)gm.blk[gm.ng]), dim3(256), 0, st, ad, gm, src, nsrc);
-        gm = AdeMulti{};
-      };
-      for (auto& g : s->groups) {
-        if (!g.ncells) continue;
-        if (g.kind == 2) {
-          Timer tm(s, FDTD_K_ADE);
-          hipLaunchKernelGGL((k_lord<real, true>), dim3((unsigned)((g.ncells + 255) / 256)), dim3(256), 0, st, ad,
-                             lord_coef(g), g.d_cells, g.d_mask, (double*)g.d_state, g.ncells, src, nsrc);
-          continue;
-        }
-        const int q = gm.ng;
-        gm.co[q] = ade_coef(g);
-        gm.cells[q] = g.d_cells;
-        gm.masks[q] = g.d_mask;
-        gm.state[q] = (double*)g.d_state;
-        gm.n[q] = g.ncells;
-        gm.blk[q + 1] = gm.blk[q] + (int32_t)((g.ncells + 255) / 256);
-        gm.ng = q + 1;
-        if (gm.ng == kAdeMulti) launch_multi();
-      }
-      launch_multi();
+    FieldArgs<real> ae = an;  // E of dispersive and general cells: the old H in, the new E out
+    for (int q = 0; q < 3; ++q) ae.h[q] = a.h[q];
+    for (auto& g : s->groups) {
+      if (g.kind != 2 || !g.ncells) continue;
+      Timer tm(s, FDTD_K_ADE);
+      hipLaunchKernelGGL((k_lord<real, true>), dim3((unsigned)((g.ncells + 255) / 256)), dim3(256), 0, st, ae,
+                         lord_coef(g), g.d_cells, g.d_mask, (double*)g.d_state, g.ncells, src, nsrc);
     }
     {
       int rc = build_march_tiles(s, s->op_by, s->op_kc);
@@ -2377,95 +2633,110 @@ int step_impl(Sim* s) {
     PmlArgs<real> pw = p;                 // new splits
     for (int q = 0; q < S_N; ++q)
       pw.s[q] = s->d_split2 ? (real*)s->d_split2 + (int64_t)q * s->npml_cells : nullptr;
-    MarchArgs<real> mg{};
+    MarchArgs<real> m{};
     for (int q = 0; q < 3; ++q) {
-      mg.eo[q] = a.e[q];
-      mg.ho[q] = a.h[q];
+      m.eo[q] = a.e[q];
+      m.ho[q] = a.h[q];
     }
     const int R = s->op_by;
-    // monitor samples: the separate sample kernel (written from the march
-    // instead, they cost the plain tiles more than the launches they save)
-    if (s->n_tl_plain || s->n_tl_xf) {
-      // x-face tiles (FP32 only, build_march_tiles): the split parts of
-      // the x slabs, old (p) and new (pw), and the x profiles
-      XfArgs<real> xa{};
-      if (s->n_tl_xf) {
-        const int Px = p.P[0], Py = p.P[1], Pz = p.P[2];
-        xa.eo[0] = p.s[S_EYX];
-        xa.eo[1] = p.s[S_EZX];
-        xa.ho[0] = p.s[S_HYX];
-        xa.ho[1] = p.s[S_HZX];
-        xa.en[0] = pw.s[S_EYX];
-        xa.en[1] = pw.s[S_EZX];
-        xa.hn[0] = pw.s[S_HYX];
-        xa.hn[1] = pw.s[S_HZX];
-        xa.f1 = p.f1[0];
-        xa.f2 = p.f2[0];
-        xa.g1 = p.g1[0];
-        xa.g2 = p.g2[0];
-        xa.kup = p.kup;
-        xa.Px = Px;
-        xa.Py = Py;
-        xa.Pz = Pz;
-        xa.nym = s->ny - 2 * Py;
-        xa.nzm = s->nz - 2 * Pz;
-        xa.base = 2 * Pz * s->nx * s->ny + (s->nz - 2 * Pz) * 2 * Py * s->nx;
-        xa.hioff = (s->nz - 2 * Pz) * xa.nym * Px;
+    const bool per = a.per[0] || a.per[1] || a.per[2];
+    // x-face tiles: the split parts of the x slabs, old (p) and new (pw),
+    // and the x profiles
+    XfArgs<real> xa{};
+    if (s->n_tl_xf) {
+      const int Px = p.P[0], Py = p.P[1], Pz = p.P[2];
+      xa.eo[0] = p.s[S_EYX];
+      xa.eo[1] = p.s[S_EZX];
+      xa.ho[0] = p.s[S_HYX];
+      xa.ho[1] = p.s[S_HZX];
+      xa.en[0] = pw.s[S_EYX];
+      xa.en[1] = pw.s[S_EZX];
+      xa.hn[0] = pw.s[S_HYX];
+      xa.hn[1] = pw.s[S_HZX];
+      xa.f1 = p.f1[0];
+      xa.f2 = p.f2[0];
+      xa.g1 = p.g1[0];
+      xa.g2 = p.g2[0];
+      xa.kup = p.kup;
+      xa.Px = Px;
+      xa.Py = Py;
+      xa.Pz = Pz;
+      xa.nym = s->ny - 2 * Py;
+      xa.nzm = s->nz - 2 * Pz;
+      xa.base = 2 * Pz * s->nx * s->ny + (s->nz - 2 * Pz) * 2 * Py * s->nx;
+      xa.hioff = (s->nz - 2 * Pz) * xa.nym * Px;
+    }
+    // four wavefronts (tiles) a workgroup
+    auto tile_list = [&](const int32_t* tiles, int ntl, int per_block, int nsplit, int* blocks) {
+      TileList t{tiles, ntl, 0, nsplit};
+      const int nb = (ntl * nsplit + per_block - 1) / per_block;
+      t.tper = (nb + 7) / 8;
+      *blocks = 8 * t.tper;
+      return t;
+    };
+    Parts all{};
+    const TileList tp = tile_list(s->d_tl_plain, s->n_tl_plain, 4, 1, &all.plain);
+    TileList tx = tile_list(s->d_tl_plain + 8 * (int64_t)s->n_tl_plain, s->n_tl_xf, 4, 1, &all.xf);
+    const TileList te = tile_list(s->d_tl_gen, s->n_tl_gen, 1, s->tl_gkc, &all.gen);  // a workgroup per plane
+    const AdeMulti ade = ade_lists(ae, &all.ade);
+    MonList<real> mon{};
+    if (!apart) mon = take_pending<real>(s);
+    all.mon = round8(mon.nblk);
+    auto march = [&](const Parts& pt) {
+      const int nb = pt.xf + pt.plain;
+      if (!nb) return;
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(256), 0, st, an, m, src, nsrc, pt, tx, tp, xa);
+      };
+      if (R == 2)
+        per ? go(k_march<real, 2, true>) : go(k_march<real, 2, false>);
+      else if (R == 4)
+        per ? go(k_march<real, 4, true>) : go(k_march<real, 4, false>);
+      else if constexpr (sizeof(real) == 4)  // FP64 tiles stop at 4 rows (8 would spill)
+        per ? go(k_march<real, 8, true>) : go(k_march<real, 8, false>);
+    };
+    auto gen_e = [&](const Parts& pt) {
+      const int nb = pt.mon + round8(pt.ade) + pt.gen;
+      if (nb)
+        hipLaunchKernelGGL(k_gen_e<real>, dim3((unsigned)nb), dim3(256), 0, st, ae, m, p, pw, src, nsrc, pt, mon,
+                           ade, te);
+    };
+    auto launch_xf4 = [&]() {
+      if constexpr (kXface<real>) {
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3((unsigned)all.xf), dim3(256), 0, st, an, m, src, nsrc, tx, xa);
+        };
+        per ? go(k_xface4<real, true>) : go(k_xface4<real, false>);
       }
-      // the plain tiles, then the x-face tiles (their own launch, tiles of
-      // tl_bx rows, the kernel with the split update)
+    };
+    const bool xf4 = s->n_tl_xf && s->tl_bx == 4;
+    if (apart) {
+      if (all.ade) {
+        Timer tm(s, FDTD_K_ADE);
+        gen_e(Parts{0, all.ade, 0, 0, 0, 0});
+      }
       if (s->n_tl_plain) {
         Timer tm(s, FDTD_K_E);
-        mg.tiles = s->d_tl_plain;
-        mg.ntiles = s->n_tl_plain;
-        const int blocks = (mg.ntiles + 3) / 4;  // four wavefronts per workgroup
-        mg.tper = (blocks + 7) / 8;
-        const dim3 grid((unsigned)(an.xcdmap ? 8 * mg.tper : blocks));
-        if (R == 2) {
-          hipLaunchKernelGGL((k_march_plain<real, 2, false>), grid, dim3(256), 0, st, an, mg, src, nsrc, xa);
-        } else if (R == 4) {
-          hipLaunchKernelGGL((k_march_plain<real, 4, false>), grid, dim3(256), 0, st, an, mg, src, nsrc, xa);
-        } else {
-          if constexpr (sizeof(real) == 4)  // FP64 tiles stop at 4 rows (8 would spill)
-            hipLaunchKernelGGL((k_march_plain<real, 8, false>), grid, dim3(256), 0, st, an, mg, src, nsrc, xa);
-        }
+        march(Parts{0, 0, 0, 0, all.plain, 0});
       }
-      if constexpr (sizeof(real) == 4) {
-        if (s->n_tl_xf) {
-          Timer tm(s, FDTD_K_XF);
-          MarchArgs<real> mx = mg;
-          mx.tiles = s->d_tl_plain + 8 * (int64_t)s->n_tl_plain;
-          mx.ntiles = s->n_tl_xf;
-          const int blocks = (mx.ntiles + 3) / 4;
-          mx.tper = (blocks + 7) / 8;
-          const dim3 grid((unsigned)(an.xcdmap ? 8 * mx.tper : blocks));
-          if (s->tl_bx == 4)
-            hipLaunchKernelGGL((k_march_plain<real, 4, true>), grid, dim3(256), 0, st, an, mx, src, nsrc, xa);
-          else
-            hipLaunchKernelGGL((k_march_plain<real, 2, true>), grid, dim3(256), 0, st, an, mx, src, nsrc, xa);
-        }
+      if (s->n_tl_xf) {
+        Timer tm(s, FDTD_K_XF);
+        xf4 ? launch_xf4() : march(Parts{0, 0, 0, all.xf, 0, 0});
       }
+      if (s->n_tl_gen) {
+        Timer tm(s, FDTD_K_GEN_E);
+        gen_e(Parts{0, 0, 0, 0, 0, all.gen});
+      }
+    } else {
+      if (xf4) launch_xf4();
+      march(Parts{0, 0, 0, xf4 ? 0 : all.xf, all.plain, 0});
+      gen_e(Parts{all.mon, all.ade, 0, 0, 0, all.gen});
     }
     if (s->n_tl_gen) {
-      mg.tiles = s->d_tl_gen;
-      mg.ntiles = s->n_tl_gen;  // E: a workgroup per plane of each; H: one each
-      FieldArgs<real> ae = an;  // E: old H in, new E out
-      for (int q = 0; q < 3; ++q) ae.h[q] = a.h[q];
-      {
-        MarchArgs<real> me = mg;
-        me.nsplit = s->tl_gkc;
-        me.tper = (me.ntiles * me.nsplit + 7) / 8;
-        const dim3 ge((unsigned)(an.xcdmap ? 8 * me.tper : me.ntiles * me.nsplit));
-        Timer tm(s, FDTD_K_GEN_E);
-        hipLaunchKernelGGL(k_gen_e<real>, ge, dim3(256), 0, st, ae, p, pw, me, src, nsrc);
-      }
-      mg.nsplit = 1;
-      mg.tper = (mg.ntiles + 7) / 8;
-      const dim3 grid((unsigned)(an.xcdmap ? 8 * mg.tper : mg.ntiles));
-      {
-        Timer tm(s, FDTD_K_GEN_H);
-        hipLaunchKernelGGL(k_gen_h<real>, grid, dim3(256), 0, st, an, p, pw, mg);
-      }
+      int nb = 0;
+      const TileList th = tile_list(s->d_tl_gen, s->n_tl_gen, 1, 1, &nb);
+      Timer tm(s, FDTD_K_GEN_H);
+      hipLaunchKernelGGL(k_gen_h<real>, dim3((unsigned)nb), dim3(256), 0, st, an, p, pw, m, th);
     }
     for (int q = 0; q < 3; ++q) {
       std::swap(s->E[q], s->E2[q]);
@@ -2475,28 +2746,54 @@ int step_impl(Sim* s) {
     a = field_args<real>(s);
     tfsf_e(st);
     tfsf_h(st, pml_args<real>(s), 1);
+    pend(63, 3);
   } else if (s->engine == FDTD_ENGINE_FUSED) {
     PmlArgs<real> p = pml_args<real>(s);
-    // tiles of zm planes, each thread marching its column through them
-    FieldArgs<real> az = a;
-    az.ntz = (s->nz + s->zm - 1) / s->zm;
-    az.tper = (az.ntx * az.nty * az.ntz + 7) / 8;
-    const dim3 gz = tile_grid(az);
-    {
-      Timer tm(s, FDTD_K_E);
+    Parts all{};
+    int tiles = 0;
+    const SegGrid gt = seg_grid(s->nx, s->ny, (int64_t)s->ny * ((s->nz + s->zm - 1) / s->zm), &tiles);
+    const SegGrid gm = seg_grid(s->nx, s->ny, s->nmix, &all.mix);
+    const AdeMulti ade = ade_lists(a, &all.ade);
+    auto by_zm = [&](auto&& go) {
       if (s->zm == 8)
-        hipLaunchKernelGGL((k_fused_e<real, 8>), gz, blk, 0, st, az, p, src, nsrc);
+        go(std::integral_constant<int, 8>{});
       else if (s->zm == 4)
-        hipLaunchKernelGGL((k_fused_e<real, 4>), gz, blk, 0, st, az, p, src, nsrc);
+        go(std::integral_constant<int, 4>{});
       else if (s->zm == 2)
-        hipLaunchKernelGGL((k_fused_e<real, 2>), gz, blk, 0, st, az, p, src, nsrc);
+        go(std::integral_constant<int, 2>{});
       else
-        hipLaunchKernelGGL((k_fused_e<real, 1>), gz, blk, 0, st, az, p, src, nsrc);
-      if (s->nmix) {
-        const int bm = std::min(256, (s->nx + 63) / 64 * 64);
-        const int ntx = (s->nx + bm - 1) / bm;
-        hipLaunchKernelGGL(k_fused_e_mixed<real>, dim3((unsigned)(s->nmix * ntx)), dim3((unsigned)bm), 0, st, a, p,
-                           src, nsrc, (const int32_t*)s->d_mixrows, ntx);
+        go(std::integral_constant<int, 1>{});
+    };
+    {
+      MonList<real> mon{};
+      if (!apart) mon = take_pending<real>(s);
+      all.mon = round8(mon.nblk);
+      auto launch = [&](const Parts& pt, int ntile) {
+        const int lists = pt.mon + round8(pt.ade) + pt.mix, nb = lists + ntile;
+        if (!nb) return;
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(256), 0, st, a, p, src, nsrc, pt, mon, ade,
+                             (const int32_t*)s->d_mixrows, gm, gt);
+        };
+        by_zm([&](auto kz) {
+          lists ? go(k_step_e<real, decltype(kz)::value, true>) : go(k_step_e<real, decltype(kz)::value, false>);
+        });
+      };
+      if (apart) {
+        {
+          Timer tm(s, FDTD_K_E);
+          launch(Parts{}, tiles);
+          launch(Parts{0, 0, all.mix, 0, 0, 0}, 0);
+        }
+        if (all.ade) {
+          Timer tm(s, FDTD_K_ADE);
+          launch(Parts{0, all.ade, 0, 0, 0, 0}, 0);
+        }
+      } else if (tiles < kListsApart) {
+        launch(all, tiles);
+      } else {
+        launch(Parts{}, tiles);
+        launch(all, 0);
       }
     }
     for (auto& g : s->groups) {
@@ -2508,24 +2805,35 @@ int step_impl(Sim* s) {
       else if (g.kind == 2)
         hipLaunchKernelGGL((k_lord<real, true>), dim3((unsigned)((g.ncells + 255) / 256)), dim3(256), 0, st, a,
                            lord_coef(g), g.d_cells, g.d_mask, (double*)g.d_state, g.ncells, src, nsrc);
-      else
-        hipLaunchKernelGGL((k_ade<real, true>), dim3((unsigned)((g.ncells + 255) / 256)), dim3(256), 0, st, a,
-                           ade_coef(g), g.d_cells, g.d_mask, (double*)g.d_state, g.ncells, src, nsrc);
     }
     tfsf_e(st);
-    const DftFuse<real> df = fused_monitors();
     {
+      // E is final here and H is not: this launch samples E, the next
+      // step's first one samples H
+      MonList<real> mon{};
+      if (!apart) {
+        std::vector<MonPend> eq;
+        sample(7, [&](const MonPend& q) { eq.push_back(q); });
+        for (size_t q = 0; q < eq.size(); ++q) {
+          if (mon.nplanes == kMonPlanes) {
+            launch_monitors(s, mon);
+            mon = MonList<real>{};
+          }
+          mon_add(mon, eq[q]);
+        }
+        if (probes_on) mon_probes(s, mon, probe_row, (double)n * s->dt, 1);
+        mon_close(mon);
+      }
+      Parts pt{};
+      pt.mon = round8(mon.nblk);
       Timer tm(s, FDTD_K_H);
-      if (s->zm == 8)
-        hipLaunchKernelGGL((k_fused_h<real, 8>), gz, blk, 0, st, az, p, df);
-      else if (s->zm == 4)
-        hipLaunchKernelGGL((k_fused_h<real, 4>), gz, blk, 0, st, az, p, df);
-      else if (s->zm == 2)
-        hipLaunchKernelGGL((k_fused_h<real, 2>), gz, blk, 0, st, az, p, df);
-      else
-        hipLaunchKernelGGL((k_fused_h<real, 1>), gz, blk, 0, st, az, p, df);
+      by_zm([&](auto kz) {
+        hipLaunchKernelGGL((k_step_h<real, decltype(kz)::value>), dim3((unsigned)(pt.mon + tiles)), dim3(256), 0, st,
+                           a, p, pt, mon, gt);
+      });
     }
     tfsf_h(st, p, 1);
+    apart ? pend(63, 3) : pend(56, 2);
   } else {
     const bool refy = s->pml_mode == FDTD_PML_REF_Y;
     const int P = refy ? s->pml.npml[1] : 0;
@@ -2576,91 +2884,22 @@ int step_impl(Sim* s) {
     }
     tfsf_h(st, PmlArgs<real>{}, 0);
   }
-  // monitors: buffer this step's plane samples, fold a full block.  Dry
-  // steps (the autotuner's) sample into the ring slot the next real step
+  if (s->engine == FDTD_ENGINE_STAGED) pend(63, 3);
+  if (s->engine == FDTD_ENGINE_STAGED || apart) flush_pending<real>(s);
+  // dry steps (the autotuner's) sample into the ring slot the next real step
   // overwrites, so each step form is timed with its sampling cost, and
-  // neither advance the ring, fold nor record probes.
-  (void)t;
-  // the planes this step samples with the monitor kernel (the others were
-  // written by the H kernel), with their ring slots
-  MonList<real> ml{};
-  auto launch_monitors = [&]() -> int {
-    int nb = 0;
-    for (int q = 0; q < ml.nplanes; ++q) {
-      ml.blk[q] = nb;
-      int ns = 0;
-      while (ns < 6 && ml.comp[q][ns] >= 0) ++ns;
-      nb += (int)((ml.np[q] + 255) / 256) * ns;
-    }
-    ml.blk[ml.nplanes] = nb;
-    const int pb = ml.nprobe > 0 ? (ml.nprobe + 255) / 256 : 0;
-    if (nb + pb == 0) return 0;
-    Timer tm(s, FDTD_K_MON);
-    hipLaunchKernelGGL(k_monitors<real>, dim3((unsigned)(nb + pb)), dim3(256), 0, st, a, ml);
-    ml = MonList<real>{};
-    return 0;
-  };
-  auto add_plane = [&](DftPlane& d, real* dst) -> int {
-    if (ml.nplanes == kMonPlanes) {
-      int rc = launch_monitors();
-      if (rc) return rc;
-    }
-    const int q = ml.nplanes++;
-    int ns = 0;
-    for (int c = 0; c < 6; ++c) ml.comp[q][c] = -1;
-    for (int c = 0; c < 6; ++c)
-      if (d.mask & (1 << c)) ml.comp[q][ns++] = c;
-    ml.axis[q] = d.axis;
-    ml.index[q] = d.index;
-    ml.n1[q] = d.n1;
-    ml.np[q] = (int64_t)d.n1 * d.n2;
-    ml.dst[q] = dst;
-    return 0;
-  };
-  if (s->dry) {
-    for (auto& d : s->dfts) {
-      if (!d.fused_now && !(n < d.n_begin || (d.n_end > 0 && n > d.n_end))) {
-        int ns = 0;
-        for (int c = 0; c < 6; ++c) ns += (d.mask >> c) & 1;
-        int rc = add_plane(d, (real*)d.d_samp + (int64_t)d.nbuf * ns * d.n1 * d.n2);
-        if (rc) return rc;
-      }
-      d.fused_now = false;
-    }
-    return launch_monitors();
-  }
-  std::vector<DftPlane*> active;
-  for (auto& d : s->dfts) {
-    if (n < d.n_begin) continue;
-    if (d.n_end > 0 && n > d.n_end) continue;
-    int ns = 0;
-    for (int c = 0; c < 6; ++c) ns += (d.mask >> c) & 1;
-    if (d.nbuf == 0) d.n_first = n;
-    if (!d.fused_now) {
-      int rc = add_plane(d, (real*)d.d_samp + (int64_t)d.nbuf * ns * d.n1 * d.n2);
-      if (rc) return rc;
-    }
-    d.fused_now = false;
-    active.push_back(&d);
-  }
-  if (!s->probes.empty()) {
-    ml.nprobe = (int)s->probes.size();
-    ml.ppos = (const int32_t*)s->d_probe_pos;
-    ml.pout = s->d_probe + (int64_t)7 * ml.nprobe * (s->probe_row0 + (n - 1 - s->call_base));
-    ml.tn = (double)n * s->dt;
-  }
-  {
-    int rc = launch_monitors();
-    if (rc) return rc;
-  }
+  // neither advance the ring, fold nor record probes
+  if (s->dry) return 0;
   // fold after this step's samples are written, when the ring is full or
   // the step is a multiple of kDftBlock: the blocks then end at the same
   // steps however the calls that make the steps are cut (a call folds what
   // it buffered at its end), so runs stepped in chunks of kDftBlock
   // multiples, or resumed from a checkpoint, equal runs stepped at once
-  for (DftPlane* d : active) {
-    d->nbuf += 1;
-    if (d->nbuf == kDftBlock || n % kDftBlock == 0) dft_flush_plane<real>(s, *d);
+  for (auto& d : s->dfts) {
+    if (n < d.n_begin || (d.n_end > 0 && n > d.n_end)) continue;
+    if (d.nbuf == 0) d.n_first = n;
+    d.nbuf += 1;
+    if (d.nbuf == kDftBlock || n % kDftBlock == 0) dft_flush_plane<real>(s, d);
   }
   return 0;
 }
@@ -2680,6 +2919,11 @@ int launch_step(Sim* s) {
 }
 
 int launch_dft_flush(Sim* s) {
+  // the last step's samples and probes, whether or not a plane has a block open
+  if (s->prec == FDTD_FP32)
+    flush_pending<float>(s);
+  else
+    flush_pending<double>(s);
   for (auto& d : s->dfts) {
     if (s->prec == FDTD_FP32)
       dft_flush_plane<float>(s, d);

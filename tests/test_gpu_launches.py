@@ -1,0 +1,111 @@
+"""The FUSED engine's launches at the sizes where their parts end: more
+dispersive groups and monitor planes than a launch takes along, calls of
+one step, grids whose lists leave the E launch, and the parts together
+(no profiling) against each in a launch of its own (profiling)."""
+import numpy as np
+import pytest
+
+from conftest import check, relerr
+
+pytestmark = pytest.mark.gpu
+
+
+def _spec(n=(41, 36, 34), groups=6, planes=11, nsteps=90):
+    """Gold-like boxes of `groups` different parameter sets, `planes` DFT
+    planes over the three axes with unlike gates, probes in and beside them."""
+    from fdtd_amd import box, gold_params_dict, workloads
+
+    spec = workloads.c1_gold_sphere(nsteps=nsteps, n=32)
+    spec["grid"].update(nx=n[0], ny=n[1], nz=n[2])
+    spec["pml"]["npml"] = [5, 4, 6]
+    mats = [{"type": "dielectric", "region": box((1, 1, 1), n), "eps": 1.0},
+            {"type": "dielectric", "region": box((1, 1, n[2] - 9), n), "eps": 2.25}]
+    for g in range(groups):
+        q = gold_params_dict()
+        q["gamma"] *= 1.0 + 0.1 * g
+        lo = (8 + 4 * g, 10 + g, 12)
+        mats.append({"type": "drude2cp", "region": box(lo, (lo[0] + 2, lo[1] + 8, 20)), "params": q})
+    spec["materials"] = mats
+    spec["sources"][0]["index"] = 9
+    om = spec["dft"][0]["omega"][:3]
+    spec["dft"] = [{"axis": q % 3, "index": 8 + q, "omega": om, "n_begin": 1 + 7 * (q % 4),
+                    "comps": [[1, 2, 4, 5], [0, 2, 3, 5], [0, 1, 3, 4], [2, 3]][q % 4] if q % 4 < 3 else [2, 3]}
+                   for q in range(planes)]
+    spec["probes"] = [[9, 12, 15], [1, 1, 1], list(n), [20, 18, 10]]
+    return spec
+
+
+def _run(spec, precision, steps, profiling=False):
+    import fdtd_amd
+
+    sim, ids, pids = fdtd_amd.make_simulation(spec, precision=precision, engine="fused")
+    sim.set_profiling(profiling)
+    for n in steps:
+        sim.step(n)
+    return sim, ids, pids
+
+
+def _same(a, ia, pa, b, ib, pb, spec):
+    for c in range(6):
+        assert np.array_equal(a.field(c), b.field(c)), c
+    for x, y, d in zip(ia, ib, spec["dft"]):
+        for c in d["comps"]:
+            for u, v in zip(a.dft(x, c), b.dft(y, c)):
+                assert np.array_equal(u, v)
+    for x, y in zip(pa, pb):
+        assert np.array_equal(a.probe(x), b.probe(y))
+
+
+@pytest.mark.parametrize("form", [{"FDTD_ONEPASS": "0"}, {"FDTD_ONEPASS": "0", "FDTD_ZMARCH": "4"},
+                                  {"FDTD_ONEPASS": "1", "FDTD_ONEPASS_BY": "2", "FDTD_ONEPASS_KC": "8"}])
+def test_groups_and_planes_past_one_list(form, monkeypatch):
+    """Six dispersive groups (a launch takes four), eleven planes (a launch
+    takes eight), calls of 1, 63, 1 and 25 steps across a DFT block: FP64
+    against the oracle at the parity bar, and bit for bit the run whose
+    parts are launches of their own."""
+    import oracle
+
+    for k, v in form.items():
+        monkeypatch.setenv(k, v)
+    spec = _spec()
+    steps = (1, 63, 1, 25)
+    a, ia, pa = _run(spec, "fp64", steps)
+    b, ib, pb = _run(spec, "fp64", steps, profiling=True)
+    _same(a, ia, pa, b, ib, pb, spec)
+    o, io, po = oracle.make_simulation(spec)
+    for n in steps:
+        o.step(n)
+    for c in range(6):
+        check(f"lists field {c}", relerr(a.field(c), o.field(c)), 1e-12)
+    for x, y, d in zip(ia, io, spec["dft"]):
+        for c in d["comps"]:
+            for u, v in zip(a.dft(x, c), o.dft(y, c)):
+                check(f"lists dft {c}", relerr(u, v), 1e-12)
+    for x, y in zip(pa, po):
+        check("lists probe", relerr(a.probe(x), o.probe(y)), 1e-12)
+    for s in (a, b, o):
+        s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("n,apart", [((9, 362, 362), False), ((9, 363, 363), True)])
+def test_lists_beside_the_rows_and_apart(n, apart, precision, monkeypatch):
+    """Grids on both sides of the line from which the lists of the two-kernel
+    E half have a launch of their own (32,768 workgroups of rows; 9 cells a
+    row leave lanes idle): the same bits as the one-pass step."""
+    assert (n[1] * n[2] >= 4 * 32768) == apart
+    spec = _spec(n, groups=0, planes=2, nsteps=6)
+    spec["pml"]["npml"] = [2, 6, 6]
+    spec["probes"] = [[5, 110, 15], [1, 1, 1], list(n)]
+    monkeypatch.setenv("FDTD_ONEPASS", "0")
+    from fdtd_amd import box, gold_params_dict
+
+    spec["materials"].append({"type": "drude2cp", "region": box((4, 100, 9), (6, 140, 30)),
+                              "params": gold_params_dict()})
+    spec["dft"] = [{"axis": 2, "index": 12, "omega": spec["dft"][0]["omega"], "comps": [0, 1, 3, 4]}]
+    a, ia, pa = _run(spec, precision, (6,))
+    monkeypatch.setenv("FDTD_ONEPASS", "1")
+    b, ib, pb = _run(spec, precision, (6,))
+    _same(a, ia, pa, b, ib, pb, spec)
+    a.close()
+    b.close()
