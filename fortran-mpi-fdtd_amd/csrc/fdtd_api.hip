@@ -488,6 +488,8 @@ void* upload_table(Sim* s) {
     }
     coef[q].v[3] = (real)m.pgax;
     gaxe[q].v[3] = (real)m.eps;
+    // STAGED: bit 8+c, the dispersive cells' part advances D_c
+    if (s->engine == FDTD_ENGINE_STAGED) fl |= (uint32_t)m.pad << 8;
     flags[q] = fl;
   }
   std::vector<uint8_t> blob(n * (2 * sizeof(Vec4<real>) + sizeof(uint32_t)));
@@ -718,6 +720,7 @@ int commit_impl(Sim* s) {
         t.coef[c] = s->ku;
       } else {
         t.act[c] = ACT_ADE;
+        if (m.type == 1 || m.type == 2) t.pad |= 1 << c;
       }
     }
     t.pgax = key[3] >= 0 ? (s->mats[key[3]].eps_r == 0.0 ? 0.0 : 1.0 / s->mats[key[3]].eps_r) : 1.0;
@@ -727,7 +730,6 @@ int commit_impl(Sim* s) {
     } else {
       t.eps = 1.0;
     }
-    t.pad = 0;
   }
   s->ntab = (int)s->tab.size();
   s->d_mattab = s->prec == FDTD_FP32 ? upload_table<float>(s) : upload_table<double>(s);

@@ -31,7 +31,7 @@ struct alignas(16) MatEntry {
   real gax[3];
   real eps;
   int32_t act[3];
-  int32_t pad;
+  int32_t pad;  // bit q: E_q is written by a Drude/CP/Raman group
 };
 
 // Device form of the material table: coef = (Ku*gax x,y,z, PML medium gax),

@@ -24,40 +24,6 @@
 
 namespace fdtd {
 
-template <typename real>
-struct FieldArgs {
-  real* e[3];
-  real* h[3];
-  real* d[3];
-  const uint8_t* matid;
-  const Vec4<real>* coef;   // Ku*gax x,y,z, PML medium gax
-  const Vec4<real>* gaxe;   // gax x,y,z, energy eps
-  const uint32_t* flags;    // bit q: a dielectric writes E_q
-  const int32_t* rowmat;    // per ghosted (j,k) row: uniform id or -1 (dword: scalar loads)
-  int32_t nx, ny, nz;
-  int32_t per[3];
-  int32_t px, pxy;          // offsets fit 32 bits (checked at commit)
-  real ku;
-  int32_t xcdmap;  // deal blocks to the 8 XCDs (one L2 each) in contiguous runs
-};
-
-// element at byte offset `off` of the row or plane that starts at p; with p
-// wave-uniform the access takes a scalar address and the 32-bit offset, and
-// no address arithmetic per access
-template <typename real>
-__device__ __forceinline__ real ld_at(const real* p, uint32_t off) {
-  return *(const real*)((const char*)p + off);
-}
-template <typename real>
-__device__ __forceinline__ void st_at(real* p, uint32_t off, real v) {
-  *(real*)((char*)p + off) = v;
-}
-
-// A launch of several parts gives each a whole number of rounds over the
-// XCDs, so that the dealing of a part's blocks does not depend on the parts
-// before it.
-__host__ __device__ __forceinline__ int round8(int n) { return (n + 7) & ~7; }
-
 // Exact quotient by a divisor known on the host, of any 31-bit number (m =
 // ceil(2^(31+s) / d), s = ceil(log2 d): Granlund and Montgomery, "Division by
 // invariant integers using multiplication", 1994): a scalar multiply and a
@@ -79,6 +45,41 @@ inline FastDiv fast_div(int d) {
 __device__ __forceinline__ int fast_quot(const FastDiv& f, int v) {
   return (int)(((uint64_t)(uint32_t)v * f.m) >> f.sh);
 }
+
+template <typename real>
+struct FieldArgs {
+  real* e[3];
+  real* h[3];
+  real* d[3];
+  const uint8_t* matid;
+  const Vec4<real>* coef;   // Ku*gax x,y,z, PML medium gax
+  const Vec4<real>* gaxe;   // gax x,y,z, energy eps
+  const uint32_t* flags;    // bit q: a dielectric writes E_q
+  const int32_t* rowmat;    // per ghosted (j,k) row: uniform id or -1 (dword: scalar loads)
+  int32_t nx, ny, nz;
+  int32_t per[3];
+  int32_t px, pxy;          // offsets fit 31 bits (checked at commit)
+  FastDiv by_px, by_pxy;    // i, j, k of an offset
+  real ku;
+  int32_t xcdmap;  // deal blocks to the 8 XCDs (one L2 each) in contiguous runs
+};
+
+// element at byte offset `off` of the row or plane that starts at p; with p
+// wave-uniform the access takes a scalar address and the 32-bit offset, and
+// no address arithmetic per access
+template <typename real>
+__device__ __forceinline__ real ld_at(const real* p, uint32_t off) {
+  return *(const real*)((const char*)p + off);
+}
+template <typename real>
+__device__ __forceinline__ void st_at(real* p, uint32_t off, real v) {
+  *(real*)((char*)p + off) = v;
+}
+
+// A launch of several parts gives each a whole number of rounds over the
+// XCDs, so that the dealing of a part's blocks does not depend on the parts
+// before it.
+__host__ __device__ __forceinline__ int round8(int n) { return (n + 7) & ~7; }
 
 // Logical block of block b of a part of nb blocks (padded to 8 * tper):
 // each XCD takes a contiguous run of tper.
@@ -103,6 +104,15 @@ struct RefPmlArgs {
   const real* prof[2];  // 12 profiles per slab, stride ps
   int32_t ps;
 };
+
+// i, j, k of offset c
+template <typename real>
+__device__ __forceinline__ void cell_of(const FieldArgs<real>& a, int c, int& i, int& j, int& k) {
+  k = fast_quot(a.by_pxy, c);
+  const int r = c - k * a.pxy;
+  j = fast_quot(a.by_px, r);
+  i = r - j * a.px;
+}
 
 // ---------------------------------------------------------------------------
 // ghost maintenance for periodic axes
@@ -1287,18 +1297,62 @@ __global__ __launch_bounds__(256) void k_gen_h(FieldArgs<real> a, PmlArgs<real> 
 // the small difference of the large D and I, which FP32 would cancel away
 // (an FP32 state gave 6e-5 relative spectra error on the 16-disk case);
 // E is stored in field precision.
+// STAGED rows: D advances on rows j0..j1 (updateD between the y slabs); on
+// the slabs' inner rows ja and jb the split fields write Ex and Ez (0: no
+// such row).
+struct StagedRows {
+  int32_t j0, j1, ja, jb;
+  __device__ __forceinline__ bool main(int j) const { return j >= j0 && j <= j1; }
+  __device__ __forceinline__ bool pml_writes(int j, int q) const { return q != 1 && (j == ja || j == jb); }
+};
+
+// New D of a cell: updateD, sim3/include/myfdtd_func.f90:19-41, on the main
+// rows, then the plane sources through it one after the other,
+// sim3/program.f90:396-406 (the TFSF consistency terms among them).  False:
+// D stays as it is.
+template <typename real>
+__device__ __forceinline__ bool staged_d(const FieldArgs<real>& a, const SrcArgs<real>& src, int nsrc,
+                                         const StagedRows& rows, int i, int j, int k, int c, real* d) {
+  d[0] = a.d[0][c];
+  d[1] = a.d[1][c];
+  d[2] = a.d[2][c];
+  bool wrote = rows.main(j);
+  if (wrote) {
+    const real hx = a.h[0][c], hy = a.h[1][c], hz = a.h[2][c];
+    const real curlhzy = hz - a.h[2][c - a.px];
+    const real curlhyz = -hy + a.h[1][c - a.pxy];
+    const real curlhxz = hx - a.h[0][c - a.pxy];
+    const real curlhzx = -hz + a.h[2][c - 1];
+    const real curlhyx = hy - a.h[1][c - 1];
+    const real curlhxy = -hx + a.h[0][c - a.px];
+    d[0] = d[0] + a.ku * (curlhzy + curlhyz);
+    d[1] = d[1] + a.ku * (curlhxz + curlhzx);
+    d[2] = d[2] + a.ku * (curlhyx + curlhxy);
+  }
+  for (int q = 0; q < nsrc; ++q) {
+    const int pos = src.axis[q] == 0 ? i : (src.axis[q] == 1 ? j : k);
+    if (pos != src.index[q]) continue;
+    wrote = true;
+    const int cq = src.comp[q];
+    const real v = src_value(src, q);
+    if (cq == 0) d[0] = d[0] + v;
+    else if (cq == 1) d[1] = d[1] + v;
+    else d[2] = d[2] + v;
+  }
+  return wrote;
+}
+
 template <typename real, bool FUSED>
 __device__ __forceinline__ void ade_cell(const FieldArgs<real>& a, const AdeCoef<double>& co, const int32_t* cells,
                                          const uint8_t* masks, double* state, int64_t n, const SrcArgs<real>& src,
-                                         int nsrc, int64_t e) {
-  const int64_t c = cells[e];
+                                         int nsrc, int64_t e, const StagedRows& rows) {
+  const int c = cells[e];
   const int mask = masks[e];
-  const int k = (int)(c / a.pxy);
-  const int64_t rem = c - (int64_t)k * a.pxy;
-  const int j = (int)(rem / a.px);
-  const int i = (int)(rem - (int64_t)j * a.px);
+  int i, j, k;
+  cell_of(a, c, i, j, k);
   double cur[3] = {0, 0, 0};
   double sv[3] = {0, 0, 0};
+  real dn[3];
   if (FUSED) {
     const double hx = a.h[0][c], hy = a.h[1][c], hz = a.h[2][c];
     cur[0] = (hz - (double)a.h[2][c - a.px]) + (-hy + (double)a.h[1][c - a.pxy]);
@@ -1308,6 +1362,8 @@ __device__ __forceinline__ void ade_cell(const FieldArgs<real>& a, const AdeCoef
       const int pos = src.axis[q] == 0 ? i : (src.axis[q] == 1 ? j : k);
       if (pos == src.index[q]) sv[src.comp[q]] += (double)src_value(src, q);
     }
+  } else {
+    staged_d(a, src, nsrc, rows, i, j, k, c, dn);
   }
   const int w0 = FUSED ? 1 : 0;  // word offset of I
   const int ncp = co.ncp;
@@ -1321,7 +1377,8 @@ __device__ __forceinline__ void ade_cell(const FieldArgs<real>& a, const AdeCoef
       dv = dv + sv[q];
       *dp = dv;
     } else {
-      dv = a.d[q][c];
+      a.d[q][c] = dn[q];  // the rows' part leaves these components' D to this one
+      dv = dn[q];
     }
     double* Ip = state + (int64_t)((w0 + 0) * 3 + q) * n + e;
     double* Sp = state + (int64_t)((w0 + 1) * 3 + q) * n + e;
@@ -1349,8 +1406,10 @@ __device__ __forceinline__ void ade_cell(const FieldArgs<real>& a, const AdeCoef
     // E = Re[X / (ga + sn)]
     const double dr = co.gar + snv, di = co.gai;
     const double ev = (xr * dr + xi * di) / (dr * dr + di * di);
-    a.e[q][c] = (real)ev;
-    put_e_ghost(a.e[q], (real)ev, i, j, k, c, a);
+    if (FUSED || !rows.pml_writes(j, q)) {
+      a.e[q][c] = (real)ev;
+      put_e_ghost(a.e[q], (real)ev, i, j, k, c, a);
+    }
     if (co.raman) {
       const double nsn = co.r1 * snv + co.r2 * snm2 + co.r0 * (ev * ev);
       *snm2p = snv;
@@ -1366,15 +1425,6 @@ __device__ __forceinline__ void ade_cell(const FieldArgs<real>& a, const AdeCoef
           (co.gbr[pp] * gi[pp] + co.gbi[pp] * gr[pp]) + co.gci[pp] * ev;
     }
   }
-}
-
-template <typename real, bool FUSED>
-__global__ __launch_bounds__(256) void k_ade(FieldArgs<real> a, AdeCoef<double> co, const int32_t* cells,
-                                             const uint8_t* masks, double* state, int64_t n, SrcArgs<real> src,
-                                             int nsrc) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  ade_cell<real, FUSED>(a, co, cells, masks, state, n, src, nsrc, e);
 }
 
 // Up to kAdeMulti Drude/CP/Raman groups as a part of an E launch: group q
@@ -1393,20 +1443,21 @@ struct AdeMulti {
   int64_t n[kAdeMulti];
 };
 
-template <typename real>
+template <typename real, bool FUSED>
 __device__ __forceinline__ void ade_block(const FieldArgs<real>& a, const AdeMulti& g, const SrcArgs<real>& src,
-                                          int nsrc, int b) {
+                                          int nsrc, int b, const StagedRows& rows = StagedRows{}) {
   int q = 0;
   while (q + 1 < g.ng && b >= g.blk[q + 1]) ++q;
   const int64_t e = (int64_t)(b - g.blk[q]) * 256 + threadIdx.x;
   if (e >= g.n[q]) return;
-  ade_cell<real, true>(a, g.co[q], g.cells[q], g.masks[q], g.state[q], g.n[q], src, nsrc, e);
+  ade_cell<real, FUSED>(a, g.co[q], g.cells[q], g.masks[q], g.state[q], g.n[q], src, nsrc, e, rows);
 }
 
 // groups past the first kAdeMulti
-template <typename real>
-__global__ __launch_bounds__(256) void k_ade_multi(FieldArgs<real> a, AdeMulti g, SrcArgs<real> src, int nsrc) {
-  ade_block(a, g, src, nsrc, (int)blockIdx.x);
+template <typename real, bool FUSED>
+__global__ __launch_bounds__(256) void k_ade_multi(FieldArgs<real> a, AdeMulti g, SrcArgs<real> src, int nsrc,
+                                                   StagedRows rows) {
+  ade_block<real, FUSED>(a, g, src, nsrc, (int)blockIdx.x, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -1423,12 +1474,10 @@ __global__ __launch_bounds__(256) void k_lord(FieldArgs<real> a, LordCoef co, co
                                               int nsrc) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
-  const int64_t c = cells[e];
+  const int c = cells[e];
   const int mask = masks[e];
-  const int k = (int)(c / a.pxy);
-  const int64_t rem = c - (int64_t)k * a.pxy;
-  const int j = (int)(rem / a.px);
-  const int i = (int)(rem - (int64_t)j * a.px);
+  int i, j, k;
+  cell_of(a, c, i, j, k);
   double cur[3] = {0, 0, 0};
   double sv[3] = {0, 0, 0};
   if (FUSED) {
@@ -1490,12 +1539,10 @@ __global__ __launch_bounds__(256) void k_ljp(FieldArgs<real> a, LjpCoef<double> 
                                              int nsrc) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
-  const int64_t c = cells[e];
+  const int c = cells[e];
   const int mask = masks[e];
-  const int k = (int)(c / a.pxy);
-  const int64_t rem = c - (int64_t)k * a.pxy;
-  const int j = (int)(rem / a.px);
-  const int i = (int)(rem - (int64_t)j * a.px);
+  int i, j, k;
+  cell_of(a, c, i, j, k);
   const real hx = a.h[0][c], hy = a.h[1][c], hz = a.h[2][c];
   const real cur[3] = {(hz - a.h[2][c - a.px]) + (-hy + a.h[1][c - a.pxy]),   // curlhzy + curlhyz
                        (hx - a.h[0][c - a.pxy]) + (-hz + a.h[2][c - 1]),     // curlhxz + curlhzx
@@ -1554,75 +1601,35 @@ __global__ __launch_bounds__(256) void k_ljp(FieldArgs<real> a, LjpCoef<double> 
 }
 
 // ---------------------------------------------------------------------------
-// STAGED engine
-// updateD, sim3/include/myfdtd_func.f90:19-41, over rows [j0, j1]
-template <typename real>
-__global__ __launch_bounds__(256) void k_staged_d(FieldArgs<real> a, int j0, int j1) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y + j0;
-  const int k = blockIdx.z + 1;
-  if (i > a.nx || j > j1) return;
-  const int64_t c = i + a.px * j + a.pxy * k;
-  const real hx = a.h[0][c], hy = a.h[1][c], hz = a.h[2][c];
-  const real curlhzy = hz - a.h[2][c - a.px];
-  const real curlhyz = -hy + a.h[1][c - a.pxy];
-  const real curlhxz = hx - a.h[0][c - a.pxy];
-  const real curlhzx = -hz + a.h[2][c - 1];
-  const real curlhyx = hy - a.h[1][c - 1];
-  const real curlhxy = -hx + a.h[0][c - a.px];
-  a.d[0][c] = a.d[0][c] + a.ku * (curlhzy + curlhyz);
-  a.d[1][c] = a.d[1][c] + a.ku * (curlhxz + curlhzx);
-  a.d[2][c] = a.d[2][c] + a.ku * (curlhyx + curlhxy);
-}
-
-// plane source, sim3/program.f90:396-406 (dval: value dscale * *dval read
-// here, the TFSF consistency terms)
-template <typename real>
-__global__ void k_staged_src(FieldArgs<real> a, int axis, int index, int comp, real val, const double* dval,
-                             double dscale) {
-  if (dval) val = (real)(dscale * *dval);
-  const int u = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int v = blockIdx.y + 1;
-  int p[3];
-  const int a1 = axis == 0 ? 1 : 0, a2 = axis == 2 ? 1 : 2;
-  const int n[3] = {a.nx, a.ny, a.nz};
-  if (u > n[a1]) return;
-  p[axis] = index;
-  p[a1] = u;
-  p[a2] = v;
-  const int64_t c = p[0] + a.px * p[1] + a.pxy * p[2];
-  a.d[comp][c] = a.d[comp][c] + val;
-}
-
+// STAGED engine: updateD, the sources and update_E of one cell in one pass
+// (each cell's D and E depend on H alone), as the reference's stages compute
+// it; E of the dispersive materials and the split fields are other parts of
+// the same launch (k_staged_e).
+//
 // ConstantDielectric%update_E for every cell/component whose last writer is
-// a dielectric (mod3/simpledielectric_mod.f90:181-183).
+// a dielectric (mod3/simpledielectric_mod.f90:181-183).  flags bit 8+q: the
+// dispersive cells' part advances D_q.
 template <typename real>
-__global__ __launch_bounds__(256) void k_staged_mat(FieldArgs<real> a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-  const int k = blockIdx.z + 1;
-  if (i > a.nx || j > a.ny) return;
+__device__ __forceinline__ void staged_e_cell(const FieldArgs<real>& a, const SrcArgs<real>& src, int nsrc,
+                                              const StagedRows& rows, int i, int j, int k, uint32_t fl,
+                                              const Vec4<real>& gx) {
   const int c = i + a.px * j + a.pxy * k;
-  const unsigned id = a.matid[c];
-  const uint32_t fl = a.flags[id];
-  const Vec4<real> gx = a.gaxe[id];
+  real d[3];
+  const bool wrote = staged_d(a, src, nsrc, rows, i, j, k, c, d);
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    if (!(fl & (1u << q))) continue;
-    const real ev = a.d[q][c] * gx.v[q];
+    if (wrote && !(fl & (256u << q))) a.d[q][c] = d[q];
+    if (!(fl & (1u << q)) || rows.pml_writes(j, q)) continue;
+    const real ev = d[q] * gx.v[q];
     a.e[q][c] = ev;
     put_e_ghost(a.e[q], ev, i, j, k, c, a);
   }
 }
 
-// updateH, sim3/include/myfdtd_func.f90:45-64, over rows [j0, j1]
+// updateH, sim3/include/myfdtd_func.f90:45-64, of one main-row cell
 template <typename real>
-__global__ __launch_bounds__(256) void k_staged_h(FieldArgs<real> a, int j0, int j1) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y + j0;
-  const int k = blockIdx.z + 1;
-  if (i > a.nx || j > j1) return;
-  const int64_t c = i + a.px * j + a.pxy * k;
+__device__ __forceinline__ void staged_h_cell(const FieldArgs<real>& a, int i, int j, int k) {
+  const int c = i + a.px * j + a.pxy * k;
   const real ex = a.e[0][c], ey = a.e[1][c], ez = a.e[2][c];
   const real curleyz = a.e[1][c + a.pxy] - ey;
   const real curlezy = -a.e[2][c + a.px] + ez;
@@ -1643,13 +1650,15 @@ __global__ __launch_bounds__(256) void k_staged_h(FieldArgs<real> a, int j0, int
 
 // Reference y-slab PML, E: updateEs (mod3/BERpmly_mod.f90:117-159) driven by
 // split H only, then setboundayEya/Eyb (:200-225,255-278).  Slab 0 holds
-// rows 0..P+1, slab 1 rows jb-1..ny+1; split ghosts stay zero.
+// rows 0..P+1, slab 1 rows jb-1..ny+1; split ghosts stay zero.  The module
+// copies the main fields of the row beyond a slab's inner one into the
+// slab's ghost row (E and H of rows P+1 and jb-1); the only reads of those
+// copies are E of row P+1 in the H update of row P and H of row jb-1 in the E
+// update of row jb, which take the main fields here, so that the slab's
+// cells need nothing another workgroup of the launch writes.
 template <typename real>
-__global__ __launch_bounds__(256) void k_ref_pml_e(FieldArgs<real> a, RefPmlArgs<real> p) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int jr = blockIdx.y * blockDim.y + threadIdx.y;  // 0..2P-1
-  const int k = blockIdx.z + 1;
-  if (i > a.nx || jr >= 2 * p.P) return;
+__device__ __forceinline__ void ref_pml_e_cell(const FieldArgs<real>& a, const RefPmlArgs<real>& p, int i, int jr,
+                                               int k) {
   const int sl = jr < p.P ? 0 : 1;
   const int j = sl == 0 ? jr + 1 : p.jb + (jr - p.P);
   const int jl = sl == 0 ? j : j - (p.jb - 1);
@@ -1658,8 +1667,10 @@ __global__ __launch_bounds__(256) void k_ref_pml_e(FieldArgs<real> a, RefPmlArgs
   const int ps = p.ps;
   const int64_t o = i + p.sx * jl + p.sxy * k;
   const int64_t ojm = o - p.sx, okm = o - p.sxy, oim = o - 1;
+  const int c = i + a.px * j + a.pxy * k;
+  const bool edge = sl == 1 && j == p.jb;  // the row below is the main one jb-1
   const real curlHzy_p = S[S_HZX][o] + S[S_HZY][o];
-  const real curlHzy_m = -S[S_HZX][ojm] - S[S_HZY][ojm];
+  const real curlHzy_m = edge ? -a.h[2][c - a.px] : -S[S_HZX][ojm] - S[S_HZY][ojm];
   const real curlHyz_p = -S[S_HYZ][o] - S[S_HYX][o];
   const real curlHyz_m = S[S_HYZ][okm] + S[S_HYX][okm];
   const real curlHxz_p = S[S_HXY][o] + S[S_HXZ][o];
@@ -1669,7 +1680,7 @@ __global__ __launch_bounds__(256) void k_ref_pml_e(FieldArgs<real> a, RefPmlArgs
   const real curlHyx_p = S[S_HYZ][o] + S[S_HYX][o];
   const real curlHyx_m = -S[S_HYZ][oim] - S[S_HYX][oim];
   const real curlHxy_p = -S[S_HXY][o] - S[S_HXZ][o];
-  const real curlHxy_m = S[S_HXY][ojm] + S[S_HXZ][ojm];
+  const real curlHxy_m = edge ? a.h[0][c - a.px] : S[S_HXY][ojm] + S[S_HXZ][ojm];
   const real f1x = pr[0 * ps + i], f2x = pr[1 * ps + i];
   const real f1y = pr[2 * ps + j], f2y = pr[3 * ps + j];
   const real f1z = pr[4 * ps + k], f2z = pr[5 * ps + k];
@@ -1681,15 +1692,7 @@ __global__ __launch_bounds__(256) void k_ref_pml_e(FieldArgs<real> a, RefPmlArgs
   S[S_EZY][o] = ezy;
   S[S_EXZ][o] = f1z * S[S_EXZ][o] + f2z * (curlHyz_p + curlHyz_m);
   S[S_EYZ][o] = f1z * S[S_EYZ][o] + f2z * (curlHxz_p + curlHxz_m);
-  const int64_t c = i + a.px * j + a.pxy * k;
-  if (sl == 0 && j == p.P) {
-    S[S_EXY][o + p.sx] = a.e[0][c + a.px];
-    S[S_EZY][o + p.sx] = a.e[2][c + a.px];
-    a.e[0][c] = exy;
-    a.e[2][c] = ezy;
-  } else if (sl == 1 && j == p.jb) {
-    S[S_EXY][o - p.sx] = a.e[0][c - a.px];
-    S[S_EZY][o - p.sx] = a.e[2][c - a.px];
+  if (sl == 0 ? j == p.P : j == p.jb) {
     a.e[0][c] = exy;
     a.e[2][c] = ezy;
   }
@@ -1697,11 +1700,8 @@ __global__ __launch_bounds__(256) void k_ref_pml_e(FieldArgs<real> a, RefPmlArgs
 
 // Reference y-slab PML, H: updateHs (:161-195) and setboundayHya/Hyb.
 template <typename real>
-__global__ __launch_bounds__(256) void k_ref_pml_h(FieldArgs<real> a, RefPmlArgs<real> p) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int jr = blockIdx.y * blockDim.y + threadIdx.y;
-  const int k = blockIdx.z + 1;
-  if (i > a.nx || jr >= 2 * p.P) return;
+__device__ __forceinline__ void ref_pml_h_cell(const FieldArgs<real>& a, const RefPmlArgs<real>& p, int i, int jr,
+                                               int k) {
   const int sl = jr < p.P ? 0 : 1;
   const int j = sl == 0 ? jr + 1 : p.jb + (jr - p.P);
   const int jl = sl == 0 ? j : j - (p.jb - 1);
@@ -1710,7 +1710,9 @@ __global__ __launch_bounds__(256) void k_ref_pml_h(FieldArgs<real> a, RefPmlArgs
   const int ps = p.ps;
   const int64_t o = i + p.sx * jl + p.sxy * k;
   const int64_t ojp = o + p.sx, okp = o + p.sxy, oip = o + 1;
-  const real curlEzy_p = -S[S_EZX][ojp] - S[S_EZY][ojp];
+  const int c = i + a.px * j + a.pxy * k;
+  const bool edge = sl == 0 && j == p.P;  // the row above is the main one P+1
+  const real curlEzy_p = edge ? -a.e[2][c + a.px] : -S[S_EZX][ojp] - S[S_EZY][ojp];
   const real curlEzy_m = S[S_EZX][o] + S[S_EZY][o];
   const real curlEyz_p = S[S_EYZ][okp] + S[S_EYX][okp];
   const real curlEyz_m = -S[S_EYZ][o] - S[S_EYX][o];
@@ -1720,7 +1722,7 @@ __global__ __launch_bounds__(256) void k_ref_pml_h(FieldArgs<real> a, RefPmlArgs
   const real curlEzx_m = -S[S_EZX][o] - S[S_EZY][o];
   const real curlEyx_p = -S[S_EYZ][oip] - S[S_EYX][oip];
   const real curlEyx_m = S[S_EYZ][o] + S[S_EYX][o];
-  const real curlExy_p = S[S_EXY][ojp] + S[S_EXZ][ojp];
+  const real curlExy_p = edge ? a.e[0][c + a.px] : S[S_EXY][ojp] + S[S_EXZ][ojp];
   const real curlExy_m = -S[S_EXY][o] - S[S_EXZ][o];
   const real g1x = pr[6 * ps + i], g2x = pr[7 * ps + i];
   const real g1y = pr[8 * ps + j], g2y = pr[9 * ps + j];
@@ -1733,15 +1735,7 @@ __global__ __launch_bounds__(256) void k_ref_pml_h(FieldArgs<real> a, RefPmlArgs
   S[S_HZY][o] = hzy;
   S[S_HXZ][o] = g1z * S[S_HXZ][o] + g2z * (curlEyz_m + curlEyz_p);
   S[S_HYZ][o] = g1z * S[S_HYZ][o] + g2z * (curlExz_m + curlExz_p);
-  const int64_t c = i + a.px * j + a.pxy * k;
-  if (sl == 0 && j == p.P) {
-    S[S_HXY][o + p.sx] = a.h[0][c + a.px];
-    S[S_HZY][o + p.sx] = a.h[2][c + a.px];
-    a.h[0][c] = hxy;
-    a.h[2][c] = hzy;
-  } else if (sl == 1 && j == p.jb) {
-    S[S_HXY][o - p.sx] = a.h[0][c - a.px];
-    S[S_HZY][o - p.sx] = a.h[2][c - a.px];
+  if (sl == 0 ? j == p.P : j == p.jb) {
     a.h[0][c] = hxy;
     a.h[2][c] = hzy;
   }
@@ -1859,7 +1853,7 @@ __global__ __launch_bounds__(256) void k_step_e(FieldArgs<real> a, PmlArgs<real>
     }
     b -= pt.mon;
     if (b < round8(pt.ade)) {
-      if (b < pt.ade) ade_block(a, ade, src, nsrc, b);
+      if (b < pt.ade) ade_block<real, true>(a, ade, src, nsrc, b);
       return;
     }
     b -= round8(pt.ade);
@@ -1927,10 +1921,77 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 8 : 4) void k_gen_e(
   }
   b -= pt.mon;
   if (b < round8(pt.ade)) {
-    if (b < pt.ade) ade_block(a, ade, src, nsrc, b);
+    if (b < pt.ade) ade_block<real, true>(a, ade, src, nsrc, b);
     return;
   }
   gen_e_block(a, p, pw, m, gen, src, nsrc, b - round8(pt.ade));
+}
+
+// STAGED step, E half: monitors of the step before (H), the dispersive cells,
+// the y slabs' split E (mix: their blocks), then D, sources and dielectric E
+// of every row; H half: monitors (E), split H, H of the main rows.  A row's
+// material entry is a scalar load where the row has one id.  The reference
+// keeps these as seven loops; as launches of their own they cost the shipped
+// case (125 x 1266 x 25, FP64) 174 us a step, D and E alone 52 + 36 us at 15
+// words a cell where one pass moves 12; together @STAGED@ us.
+template <typename real>
+__global__ __launch_bounds__(256) void k_staged_e(FieldArgs<real> a, RefPmlArgs<real> rp, SrcArgs<real> src, int nsrc,
+                                                  StagedRows rows, Parts pt, MonList<real> mon, AdeMulti ade,
+                                                  SegGrid gs, SegGrid gt) {
+  int b = (int)blockIdx.x;
+  if (b < pt.mon) {
+    mon_block(mon, a.px, a.pxy, b, [&](int c) -> const real* { return c < 3 ? a.e[c] : a.h[c - 3]; });
+    return;
+  }
+  b -= pt.mon;
+  if (b < round8(pt.ade)) {
+    if (b < pt.ade) ade_block<real, false>(a, ade, src, nsrc, b, rows);
+    return;
+  }
+  b -= round8(pt.ade);
+  int tx, r;
+  if (b < pt.mix) {
+    if (!seg_of(gs, b, a.xcdmap, tx, r)) return;
+    const int i = tx * 64 + ((int)threadIdx.x & 63) + 1, kz = fast_quot(gs.ny, r);
+    if (i <= a.nx) ref_pml_e_cell(a, rp, i, r - kz * gs.ny.d, kz + 1);
+    return;
+  }
+  if (!seg_of(gt, b - pt.mix, a.xcdmap, tx, r)) return;
+  const int i = tx * 64 + ((int)threadIdx.x & 63) + 1, kz = fast_quot(gt.ny, r);
+  const int j = r - kz * gt.ny.d + 1, k = kz + 1;
+  if (i > a.nx) return;
+  const int rm = a.rowmat[j + (a.ny + 2) * k];
+  if (rm >= 0) {
+    const uint32_t fl = a.flags[rm];
+    bool any = rows.main(j) || (fl & 7u);
+    for (int q = 0; q < nsrc; ++q) any |= src.axis[q] != 1 || src.index[q] == j;
+    if (!any) return;  // a slab row that nothing here writes
+    staged_e_cell(a, src, nsrc, rows, i, j, k, fl, a.gaxe[rm]);
+  } else {
+    const unsigned id = a.matid[i + a.px * j + a.pxy * k];
+    staged_e_cell(a, src, nsrc, rows, i, j, k, a.flags[id], a.gaxe[id]);
+  }
+}
+
+template <typename real>
+__global__ __launch_bounds__(256) void k_staged_h(FieldArgs<real> a, RefPmlArgs<real> rp, StagedRows rows, Parts pt,
+                                                  MonList<real> mon, SegGrid gs, SegGrid gt) {
+  int b = (int)blockIdx.x;
+  if (b < pt.mon) {
+    mon_block(mon, a.px, a.pxy, b, [&](int c) -> const real* { return c < 3 ? a.e[c] : a.h[c - 3]; });
+    return;
+  }
+  b -= pt.mon;
+  int tx, r;
+  if (b < pt.mix) {
+    if (!seg_of(gs, b, a.xcdmap, tx, r)) return;
+    const int i = tx * 64 + ((int)threadIdx.x & 63) + 1, kz = fast_quot(gs.ny, r);
+    if (i <= a.nx) ref_pml_h_cell(a, rp, i, r - kz * gs.ny.d, kz + 1);
+    return;
+  }
+  if (!seg_of(gt, b - pt.mix, a.xcdmap, tx, r)) return;
+  const int i = tx * 64 + ((int)threadIdx.x & 63) + 1, kz = fast_quot(gt.ny, r);
+  if (i <= a.nx) staged_h_cell(a, i, r - kz * gt.ny.d + rows.j0, kz + 1);
 }
 
 // x-face tiles of 4 rows (FDTD_XFACE_BY=4)
@@ -2284,6 +2345,8 @@ FieldArgs<real> field_args(Sim* s) {
   for (int q = 0; q < 3; ++q) a.per[q] = s->g.periodic[q] ? 1 : 0;
   a.px = (int32_t)s->px;
   a.pxy = (int32_t)s->pxy;
+  a.by_px = fast_div(a.px);
+  a.by_pxy = fast_div(a.pxy);
   a.ku = (real)s->ku;
   a.xcdmap = s->xcdmap;
   return a;
@@ -2514,6 +2577,9 @@ int step_impl(Sim* s) {
     return c;
   };
 
+  const bool refy = s->pml_mode == FDTD_PML_REF_Y;
+  const int Py = refy ? s->pml.npml[1] : 0;
+  const StagedRows rows{1 + Py, s->ny - Py, refy ? Py : 0, refy ? s->ny - Py + 1 : 0};
   // the Drude/CP/Raman groups, kAdeMulti at a time: the first list goes with
   // an E launch (their blocks in *blocks), the others have launches of their own
   auto ade_lists = [&](const FieldArgs<real>& af, int* blocks) {
@@ -2526,7 +2592,12 @@ int step_impl(Sim* s) {
         have = true;
       } else {
         Timer tm(s, FDTD_K_ADE);
-        hipLaunchKernelGGL(k_ade_multi<real>, dim3((unsigned)g.blk[g.ng]), dim3(256), 0, st, af, g, src, nsrc);
+        if (s->engine == FDTD_ENGINE_FUSED)
+          hipLaunchKernelGGL((k_ade_multi<real, true>), dim3((unsigned)g.blk[g.ng]), dim3(256), 0, st, af, g, src, nsrc,
+                             rows);
+        else
+          hipLaunchKernelGGL((k_ade_multi<real, false>), dim3((unsigned)g.blk[g.ng]), dim3(256), 0, st, af, g, src,
+                             nsrc, rows);
       }
       g = AdeMulti{};
     };
@@ -2610,6 +2681,22 @@ int step_impl(Sim* s) {
   };
   // profiling: every part a launch of its own, timed
   const bool apart = s->profiling;
+  // in the H launch E is final and H is not: it samples E, the next step's
+  // first launch H
+  auto e_samples = [&]() {
+    MonList<real> mon{};
+    if (apart) return mon;
+    sample(7, [&](const MonPend& q) {
+      if (mon.nplanes == kMonPlanes) {
+        launch_monitors(s, mon);
+        mon = MonList<real>{};
+      }
+      mon_add(mon, q);
+    });
+    if (probes_on) mon_probes(s, mon, probe_row, (double)n * s->dt, 1);
+    mon_close(mon);
+    return mon;
+  };
   if (s->engine == FDTD_ENGINE_FUSED && s->onepass) {
     // new fields go to the second copies, then the copies swap roles
     FieldArgs<real> an = a;
@@ -2808,22 +2895,7 @@ int step_impl(Sim* s) {
     }
     tfsf_e(st);
     {
-      // E is final here and H is not: this launch samples E, the next
-      // step's first one samples H
-      MonList<real> mon{};
-      if (!apart) {
-        std::vector<MonPend> eq;
-        sample(7, [&](const MonPend& q) { eq.push_back(q); });
-        for (size_t q = 0; q < eq.size(); ++q) {
-          if (mon.nplanes == kMonPlanes) {
-            launch_monitors(s, mon);
-            mon = MonList<real>{};
-          }
-          mon_add(mon, eq[q]);
-        }
-        if (probes_on) mon_probes(s, mon, probe_row, (double)n * s->dt, 1);
-        mon_close(mon);
-      }
+      const MonList<real> mon = e_samples();
       Parts pt{};
       pt.mon = round8(mon.nblk);
       Timer tm(s, FDTD_K_H);
@@ -2835,24 +2907,42 @@ int step_impl(Sim* s) {
     tfsf_h(st, p, 1);
     apart ? pend(63, 3) : pend(56, 2);
   } else {
-    const bool refy = s->pml_mode == FDTD_PML_REF_Y;
-    const int P = refy ? s->pml.npml[1] : 0;
-    const int j0 = 1 + P, j1 = s->ny - P;
+    RefPmlArgs<real> rp{};
+    if (refy) rp = ref_pml_args<real>(s);
+    Parts all{};
+    int tiles = 0, main_tiles = 0;
+    const SegGrid gt = seg_grid(s->nx, s->ny, (int64_t)s->ny * s->nz, &tiles);
+    const SegGrid gh = seg_grid(s->nx, s->ny - 2 * Py, (int64_t)(s->ny - 2 * Py) * s->nz, &main_tiles);
+    const SegGrid gs = seg_grid(s->nx, std::max(1, 2 * Py), (int64_t)2 * Py * s->nz, &all.mix);
+    const AdeMulti ade = ade_lists(a, &all.ade);
+    // the Lorentz cells' launches read E or the new D, and write E the split
+    // fields then replace: the slabs' part comes after them
+    bool lorentz = false;
+    for (const auto& g : s->groups) lorentz |= g.kind != 0 && g.ncells;
     {
-      Timer tm(s, FDTD_K_E);
-      hipLaunchKernelGGL(k_staged_d<real>, cell_grid(s->nx, j1 - j0 + 1, s->nz, blk), blk, 0, st, a, j0, j1);
-    }
-    for (int q = 0; q < nsrc; ++q) {
-      const int ax = src.axis[q];
-      const int a1 = ax == 0 ? 1 : 0, a2 = ax == 2 ? 1 : 2;
-      const int nn[3] = {s->nx, s->ny, s->nz};
-      Timer tm(s, FDTD_K_MAT);
-      hipLaunchKernelGGL(k_staged_src<real>, dim3((unsigned)((nn[a1] + 63) / 64), (unsigned)nn[a2]), dim3(64), 0, st,
-                         a, ax, src.index[q], src.comp[q], src.val[q], src.dval[q], src.dscale[q]);
-    }
-    {
-      Timer tm(s, FDTD_K_MAT);
-      hipLaunchKernelGGL(k_staged_mat<real>, cell_grid(s->nx, s->ny, s->nz, blk), blk, 0, st, a);
+      MonList<real> mon{};
+      if (!apart) mon = take_pending<real>(s);
+      all.mon = round8(mon.nblk);
+      auto launch = [&](const Parts& pt, int ntile) {
+        const int nb = pt.mon + round8(pt.ade) + pt.mix + ntile;
+        if (nb)
+          hipLaunchKernelGGL(k_staged_e<real>, dim3((unsigned)nb), dim3(256), 0, st, a, rp, src, nsrc, rows, pt, mon,
+                             ade, gs, gt);
+      };
+      if (apart) {
+        {
+          Timer tm(s, FDTD_K_E);
+          launch(Parts{}, tiles);
+        }
+        if (all.ade) {
+          Timer tm(s, FDTD_K_ADE);
+          launch(Parts{0, all.ade, 0, 0, 0, 0}, 0);
+        }
+      } else if (lorentz) {
+        launch(Parts{all.mon, all.ade, 0, 0, 0, 0}, tiles);
+      } else {
+        launch(all, tiles);
+      }
     }
     for (auto& g : s->groups) {
       if (!g.ncells) continue;
@@ -2863,29 +2953,37 @@ int step_impl(Sim* s) {
       else if (g.kind == 2)
         hipLaunchKernelGGL((k_lord<real, false>), dim3((unsigned)((g.ncells + 255) / 256)), dim3(256), 0, st, a,
                            lord_coef(g), g.d_cells, g.d_mask, (double*)g.d_state, g.ncells, src, 0);
-      else
-        hipLaunchKernelGGL((k_ade<real, false>), dim3((unsigned)((g.ncells + 255) / 256)), dim3(256), 0, st, a,
-                           ade_coef(g), g.d_cells, g.d_mask, (double*)g.d_state, g.ncells, src, 0);
     }
-    RefPmlArgs<real> rp{};
-    if (refy) {
-      rp = ref_pml_args<real>(s);
+    if (refy && (apart || lorentz)) {
       Timer tm(s, FDTD_K_PML_E);
-      hipLaunchKernelGGL(k_ref_pml_e<real>, cell_grid(s->nx, 2 * P, s->nz, blk), blk, 0, st, a, rp);
+      hipLaunchKernelGGL(k_staged_e<real>, dim3((unsigned)all.mix), dim3(256), 0, st, a, rp, src, nsrc, rows,
+                         Parts{0, 0, all.mix, 0, 0, 0}, MonList<real>{}, AdeMulti{}, gs, gt);
     }
     tfsf_e(st);
     {
-      Timer tm(s, FDTD_K_H);
-      hipLaunchKernelGGL(k_staged_h<real>, cell_grid(s->nx, j1 - j0 + 1, s->nz, blk), blk, 0, st, a, j0, j1);
-    }
-    if (refy) {
-      Timer tm(s, FDTD_K_PML_H);
-      hipLaunchKernelGGL(k_ref_pml_h<real>, cell_grid(s->nx, 2 * P, s->nz, blk), blk, 0, st, a, rp);
+      const MonList<real> mon = e_samples();
+      auto launch = [&](const Parts& pt, const MonList<real>& m, int ntile) {
+        const int nb = pt.mon + pt.mix + ntile;
+        if (nb)
+          hipLaunchKernelGGL(k_staged_h<real>, dim3((unsigned)nb), dim3(256), 0, st, a, rp, rows, pt, m, gs, gh);
+      };
+      if (apart) {
+        {
+          Timer tm(s, FDTD_K_H);
+          launch(Parts{}, mon, main_tiles);
+        }
+        if (refy) {
+          Timer tm(s, FDTD_K_PML_H);
+          launch(Parts{0, 0, all.mix, 0, 0, 0}, mon, 0);
+        }
+      } else {
+        launch(Parts{round8(mon.nblk), 0, all.mix, 0, 0, 0}, mon, main_tiles);
+      }
     }
     tfsf_h(st, PmlArgs<real>{}, 0);
+    apart ? pend(63, 3) : pend(56, 2);
   }
-  if (s->engine == FDTD_ENGINE_STAGED) pend(63, 3);
-  if (s->engine == FDTD_ENGINE_STAGED || apart) flush_pending<real>(s);
+  if (apart) flush_pending<real>(s);
   // dry steps (the autotuner's) sample into the ring slot the next real step
   // overwrites, so each step form is timed with its sampling cost, and
   // neither advance the ring, fold nor record probes
