@@ -466,6 +466,23 @@ int setup_ref_y(Sim* s) {
 // plane: grids of wider planes keep the two-kernel step.
 bool onepass_fits(const Sim* s) { return (uint64_t)s->pxy * s->wsize < ((uint64_t)1 << 32); }
 
+// Whether a step that goes once through `arrays` field arrays marks what it
+// will not read again within the step as nontemporal: the arrays of a
+// pass together take more than 7/8 of the 256 MiB memory-side cache, so such
+// lines would leave it before the next step and only push out lines that a
+// neighbour still reads.  Below the line the next step finds them there.
+// us per step, marked against not, one pass of 12 arrays (its stores): FP32
+// 128^3 (124 MiB) 67.6 : 64.3, 150 x 137 x 211 (217 MiB) 109 : 106, 160^3
+// (231 MiB) 92.3 : 94.8, 203^3 176 : 189, 384^3 725 : 748, 512^3 1852 : 1913,
+// FP64 320^3 1003 : 1031; STAGED FP64, 9 arrays (D, read and written): 100 x
+// 800 x 25 74 : 67, 110 x 1000 x 25 (208 MiB) 94 : 84, 125 x 1100 x 25 (261
+// MiB) 113 : 126, 125 x 1266 x 25 125 : 143.  Marked loads of the fields that
+// neighbouring tiles share lose everywhere.
+bool streams_past_llc(const Sim* s, int arrays) {
+  if (const char* e = std::getenv("FDTD_NT")) return std::atoi(e) != 0;
+  return (uint64_t)s->ncell_alloc * s->wsize * arrays > ((uint64_t)256 << 20) / 8 * 7;
+}
+
 inline bool cell_in_pml(const Sim* s, int i, int j, int k) {
   if (s->pml_mode != FDTD_PML_ALL_FACES) return false;
   const int* P = s->P;
@@ -546,6 +563,8 @@ int commit_impl(Sim* s) {
   // one-pass step: FUSED engine without Lorentz-Jp materials (their E form
   // reads the previous E in place); FDTD_ONEPASS=0 keeps the two-kernel step
   s->onepass = 0;
+  s->nt_march = streams_past_llc(s, 12);
+  s->nt_d = streams_past_llc(s, 9);
   if (s->engine == FDTD_ENGINE_FUSED) {
     bool ljp = false;
     for (const auto& m : s->mats) ljp |= m.type == 3;

@@ -231,6 +231,7 @@ struct Sim {
   // whether fused kernels deal tiles to XCDs in contiguous runs
   int bx = 64, by = 4;
   int xcdmap = 1;
+  bool nt_march = false, nt_d = false;  // streams_past_llc of the one-pass fields, of STAGED D
   // one-pass step (FUSED engine): E and H of a step read from one copy of
   // the fields and written to the other (E2/H2/d_split2 hold the second
   // copy).  The grid is cut into tiles of 64 x op_by cells (op_by in

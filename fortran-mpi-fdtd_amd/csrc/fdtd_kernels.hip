@@ -75,6 +75,14 @@ template <typename real>
 __device__ __forceinline__ void st_at(real* p, uint32_t off, real v) {
   *(real*)((char*)p + off) = v;
 }
+// NT: a nontemporal store (streams_past_llc)
+template <bool NT, typename real>
+__device__ __forceinline__ void put(real* p, real v) {
+  if constexpr (NT)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
 
 // A launch of several parts gives each a whole number of rounds over the
 // XCDs, so that the dealing of a part's blocks does not depend on the parts
@@ -873,7 +881,7 @@ __device__ __forceinline__ real plain_e(const PlainCoef<real>& q, int c, real e0
   return ev;
 }
 
-template <typename real, int R, bool XF, bool PER>
+template <typename real, int R, bool XF, bool PER, bool NT>
 __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const MarchArgs<real>& m,
                                             const XfArgs<real>& x, const XfLane<real>& xl,
                                             const SrcArgs<real>& src, int nsrc, PlainCoef<real> q,
@@ -987,9 +995,9 @@ __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const Marc
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (!w.row_own[r]) continue;
-      st_at(e0, w.o[r], exn[r]);
-      st_at(e1, w.o[r], eyn[r]);
-      st_at(e2, w.o[r], ezn[r]);
+      put<NT>((real*)((char*)e0 + w.o[r]), exn[r]);
+      put<NT>((real*)((char*)e1 + w.o[r]), eyn[r]);
+      put<NT>((real*)((char*)e2 + w.o[r]), ezn[r]);
       if (PER && w.ghosts) {
         const int64_t cc = w.ip + a.px * w.jrow[r] + kb;
         put_e_ghost(a.e[0], exn[r], w.ip, w.jrow[r], kk, cc, a);
@@ -1041,9 +1049,9 @@ __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const Marc
           x.hn[1][sc] = n[1];
         }
       }
-      st_at(h0, w.o[r], hx);
-      st_at(h1, w.o[r], hy);
-      st_at(h2, w.o[r], hz);
+      put<NT>((real*)((char*)h0 + w.o[r]), hx);
+      put<NT>((real*)((char*)h1 + w.o[r]), hy);
+      put<NT>((real*)((char*)h2 + w.o[r]), hz);
       if (PER && w.ghosts) {
         const int64_t cc = w.ip + a.px * w.jrow[r] + kb;
         put_h_ghost(a.h[0], hx, w.ip, w.jrow[r], kh, cc, a);
@@ -1085,7 +1093,7 @@ __device__ __forceinline__ void plain_plane(const FieldArgs<real>& a, const Marc
 // E).  No LDS and no barrier.  PER: some axis is periodic (the ghost stores
 // and the wrapped maps cost registers and scalar branches per row and plane,
 // so the handles without a periodic axis run a kernel without them).
-template <typename real, int R, bool XF, bool PER>
+template <typename real, int R, bool XF, bool PER, bool NT>
 __device__ __forceinline__ void march_block(const FieldArgs<real>& a, const MarchArgs<real>& m, const TileList& tl,
                                             const SrcArgs<real>& src, int nsrc, const XfArgs<real>& x, int b) {
   const int lane = threadIdx.x & 63;
@@ -1182,8 +1190,8 @@ __device__ __forceinline__ void march_block(const FieldArgs<real>& a, const Marc
   PlainPlane<real, R> A, B;
   plain_load<real, R, XF>(a, m, x, xl, w, w.k0, A);
   for (int k = w.k0; k <= w.k1 + 1; k += 2) {
-    plain_plane<real, R, XF, PER>(a, m, x, xl, src, nsrc, q, w, lane, k, A, B, c);
-    if (k + 1 <= w.k1 + 1) plain_plane<real, R, XF, PER>(a, m, x, xl, src, nsrc, q, w, lane, k + 1, B, A, c);
+    plain_plane<real, R, XF, PER, NT>(a, m, x, xl, src, nsrc, q, w, lane, k, A, B, c);
+    if (k + 1 <= w.k1 + 1) plain_plane<real, R, XF, PER, NT>(a, m, x, xl, src, nsrc, q, w, lane, k + 1, B, A, c);
   }
 }
 
@@ -1310,12 +1318,16 @@ struct StagedRows {
 // rows, then the plane sources through it one after the other,
 // sim3/program.f90:396-406 (the TFSF consistency terms among them).  False:
 // D stays as it is.
-template <typename real>
+template <typename real, bool NT = false>
 __device__ __forceinline__ bool staged_d(const FieldArgs<real>& a, const SrcArgs<real>& src, int nsrc,
                                          const StagedRows& rows, int i, int j, int k, int c, real* d) {
-  d[0] = a.d[0][c];
-  d[1] = a.d[1][c];
-  d[2] = a.d[2][c];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    if constexpr (NT)
+      d[q] = __builtin_nontemporal_load(a.d[q] + c);
+    else
+      d[q] = a.d[q][c];
+  }
   bool wrote = rows.main(j);
   if (wrote) {
     const real hx = a.h[0][c], hy = a.h[1][c], hz = a.h[2][c];
@@ -1609,16 +1621,16 @@ __global__ __launch_bounds__(256) void k_ljp(FieldArgs<real> a, LjpCoef<double> 
 // ConstantDielectric%update_E for every cell/component whose last writer is
 // a dielectric (mod3/simpledielectric_mod.f90:181-183).  flags bit 8+q: the
 // dispersive cells' part advances D_q.
-template <typename real>
+template <typename real, bool NT>
 __device__ __forceinline__ void staged_e_cell(const FieldArgs<real>& a, const SrcArgs<real>& src, int nsrc,
                                               const StagedRows& rows, int i, int j, int k, uint32_t fl,
                                               const Vec4<real>& gx) {
   const int c = i + a.px * j + a.pxy * k;
   real d[3];
-  const bool wrote = staged_d(a, src, nsrc, rows, i, j, k, c, d);
+  const bool wrote = staged_d<real, NT>(a, src, nsrc, rows, i, j, k, c, d);
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    if (wrote && !(fl & (256u << q))) a.d[q][c] = d[q];
+    if (wrote && !(fl & (256u << q))) put<NT>(a.d[q] + c, d[q]);
     if (!(fl & (1u << q)) || rows.pml_writes(j, q)) continue;
     const real ev = d[q] * gx.v[q];
     a.e[q][c] = ev;
@@ -1894,17 +1906,18 @@ __global__ __launch_bounds__(256) void k_step_h(FieldArgs<real> a, PmlArgs<real>
 // two launches by the registers it needs: the x-face tiles and the plain
 // tiles (the longest workgroups first), then the monitors of the step before,
 // dispersive cells and E of the general cells; H of the general cells
-// (k_gen_h) follows, since it reads E that other workgroups write.
-template <typename real, int R, bool PER>
+// (k_gen_h) follows, since it reads E that other workgroups write.  NT: the
+// marching tiles' stores nontemporal (streams_past_llc).
+template <typename real, int R, bool PER, bool NT>
 __global__ __launch_bounds__(256) void k_march(FieldArgs<real> a, MarchArgs<real> m, SrcArgs<real> src, int nsrc,
                                                Parts pt, TileList xf, TileList plain, XfArgs<real> x) {
   int b = (int)blockIdx.x;
   if (b < pt.xf) {
-    if constexpr (kXface<real>) march_block<real, 2, true, PER>(a, m, xf, src, nsrc, x, b);
+    if constexpr (kXface<real>) march_block<real, 2, true, PER, NT>(a, m, xf, src, nsrc, x, b);
     return;
   }
   b -= pt.xf;
-  march_block<real, R, false, PER>(a, m, plain, src, nsrc, x, b);
+  march_block<real, R, false, PER, NT>(a, m, plain, src, nsrc, x, b);
 }
 
 // a.h: the old H, a.e: the new E.  FP32 runs at eight wavefronts per SIMD
@@ -1933,8 +1946,11 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 8 : 4) void k_gen_e(
 // material entry is a scalar load where the row has one id.  The reference
 // keeps these as seven loops; as launches of their own they cost the shipped
 // case (125 x 1266 x 25, FP64) 174 us a step, D and E alone 52 + 36 us at 15
-// words a cell where one pass moves 12; together @STAGED@ us.
-template <typename real>
+// words a cell where one pass moves 12; together 148 us.  NT: D, which nothing
+// else of the step reads, marked nontemporal on grids past the memory-side
+// cache (streams_past_llc), where E and H, 6 of the 9 arrays, then mostly stay
+// in it: 126 us.
+template <typename real, bool NT>
 __global__ __launch_bounds__(256) void k_staged_e(FieldArgs<real> a, RefPmlArgs<real> rp, SrcArgs<real> src, int nsrc,
                                                   StagedRows rows, Parts pt, MonList<real> mon, AdeMulti ade,
                                                   SegGrid gs, SegGrid gt) {
@@ -1966,10 +1982,10 @@ __global__ __launch_bounds__(256) void k_staged_e(FieldArgs<real> a, RefPmlArgs<
     bool any = rows.main(j) || (fl & 7u);
     for (int q = 0; q < nsrc; ++q) any |= src.axis[q] != 1 || src.index[q] == j;
     if (!any) return;  // a slab row that nothing here writes
-    staged_e_cell(a, src, nsrc, rows, i, j, k, fl, a.gaxe[rm]);
+    staged_e_cell<real, NT>(a, src, nsrc, rows, i, j, k, fl, a.gaxe[rm]);
   } else {
     const unsigned id = a.matid[i + a.px * j + a.pxy * k];
-    staged_e_cell(a, src, nsrc, rows, i, j, k, a.flags[id], a.gaxe[id]);
+    staged_e_cell<real, NT>(a, src, nsrc, rows, i, j, k, a.flags[id], a.gaxe[id]);
   }
 }
 
@@ -1998,7 +2014,7 @@ __global__ __launch_bounds__(256) void k_staged_h(FieldArgs<real> a, RefPmlArgs<
 template <typename real, bool PER>
 __global__ __launch_bounds__(256) void k_xface4(FieldArgs<real> a, MarchArgs<real> m, SrcArgs<real> src, int nsrc,
                                                 TileList xf, XfArgs<real> x) {
-  march_block<real, 4, true, PER>(a, m, xf, src, nsrc, x, (int)blockIdx.x);
+  march_block<real, 4, true, PER, false>(a, m, xf, src, nsrc, x, (int)blockIdx.x);
 }
 
 // cos/sin table of one block of samples: tab[(b*nfreq + m)*2 + {0,1}]
@@ -2775,12 +2791,19 @@ int step_impl(Sim* s) {
       auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(256), 0, st, an, m, src, nsrc, pt, tx, tp, xa);
       };
-      if (R == 2)
-        per ? go(k_march<real, 2, true>) : go(k_march<real, 2, false>);
-      else if (R == 4)
-        per ? go(k_march<real, 4, true>) : go(k_march<real, 4, false>);
-      else if constexpr (sizeof(real) == 4)  // FP64 tiles stop at 4 rows (8 would spill)
-        per ? go(k_march<real, 8, true>) : go(k_march<real, 8, false>);
+      auto by_rows = [&](auto prd, auto nt) {
+        constexpr bool PER = decltype(prd)::value, NT = decltype(nt)::value;
+        if (R == 2)
+          go(k_march<real, 2, PER, NT>);
+        else if (R == 4)
+          go(k_march<real, 4, PER, NT>);
+        else if constexpr (sizeof(real) == 4)  // FP64 tiles stop at 4 rows (8 would spill)
+          go(k_march<real, 8, PER, NT>);
+      };
+      auto by_store = [&](auto prd) {
+        s->nt_march ? by_rows(prd, std::true_type{}) : by_rows(prd, std::false_type{});
+      };
+      per ? by_store(std::true_type{}) : by_store(std::false_type{});
     };
     auto gen_e = [&](const Parts& pt) {
       const int nb = pt.mon + round8(pt.ade) + pt.gen;
@@ -2925,9 +2948,10 @@ int step_impl(Sim* s) {
       all.mon = round8(mon.nblk);
       auto launch = [&](const Parts& pt, int ntile) {
         const int nb = pt.mon + round8(pt.ade) + pt.mix + ntile;
-        if (nb)
-          hipLaunchKernelGGL(k_staged_e<real>, dim3((unsigned)nb), dim3(256), 0, st, a, rp, src, nsrc, rows, pt, mon,
-                             ade, gs, gt);
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(256), 0, st, a, rp, src, nsrc, rows, pt, mon, ade, gs, gt);
+        };
+        if (nb) s->nt_d ? go(k_staged_e<real, true>) : go(k_staged_e<real, false>);
       };
       if (apart) {
         {
@@ -2956,7 +2980,7 @@ int step_impl(Sim* s) {
     }
     if (refy && (apart || lorentz)) {
       Timer tm(s, FDTD_K_PML_E);
-      hipLaunchKernelGGL(k_staged_e<real>, dim3((unsigned)all.mix), dim3(256), 0, st, a, rp, src, nsrc, rows,
+      hipLaunchKernelGGL((k_staged_e<real, false>), dim3((unsigned)all.mix), dim3(256), 0, st, a, rp, src, nsrc, rows,
                          Parts{0, 0, all.mix, 0, 0, 0}, MonList<real>{}, AdeMulti{}, gs, gt);
     }
     tfsf_e(st);

@@ -109,3 +109,36 @@ def test_lists_beside_the_rows_and_apart(n, apart, precision, monkeypatch):
     _same(a, ia, pa, b, ib, pb, spec)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("by", ["2", "4", "8"])
+@pytest.mark.parametrize("case", ["gold_sphere", "periodic_box"])
+def test_marked_stores_of_the_march(case, by, precision, monkeypatch):
+    """The one-pass step with its stores marked nontemporal (what a grid past
+    the memory-side cache runs; FDTD_NT forces a side): the same bits."""
+    from test_gpu_onepass import _cases, _run as run, _same as same
+
+    spec = _cases()[case]
+    env = {"FDTD_ONEPASS": "1", "FDTD_ONEPASS_BY": by, "FDTD_ONEPASS_KC": "16"}
+    got = [run(spec, precision, dict(env, FDTD_NT=nt), monkeypatch) for nt in "01"]
+    same(*got[0], *got[1])
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("case", ["ref_graphene_small", "periodic_box"])
+def test_marked_d_of_the_reference_order(case, precision, golden, monkeypatch):
+    """The same of the staged engine's D, y-slab PML and periodic axes."""
+    import fdtd_amd
+    from test_gpu_onepass import _cases
+
+    spec = _cases()[case] if case == "periodic_box" else golden(case)[0]
+    got = []
+    for nt in "01":
+        monkeypatch.setenv("FDTD_NT", nt)
+        sim, _, _ = fdtd_amd.make_simulation(spec, precision=precision, engine="staged")
+        sim.step(min(spec["nsteps"], 130))
+        got.append(sim)
+    assert np.abs(got[0].field(0)).max() > 0
+    for c in range(9):
+        assert np.array_equal(got[0].field(c), got[1].field(c)), c
