@@ -966,7 +966,7 @@ void* field_ptr(Sim* s, int comp) {
 }  // namespace
 
 // Tile lists of the one-pass step for tiles of 64 x by cells (x from 1 in
-// steps of 64, y from 1 in steps of by) and z ranges of at most kc planes;
+// steps of 64, y from 1 in steps of by) and z ranges of at most kc/4 planes;
 // 8 words per tile: i0, j0, k0, k1, xlo, xhi, then (plain tiles) the
 // material id and 1 for an x-face tile (0 otherwise).
 //
@@ -1003,8 +1003,16 @@ int build_march_tiles(Sim* s, int by, int kc) {
   const int Px = af ? s->P[0] : 0, Py = af ? s->P[1] : 0, Pz = af ? s->P[2] : 0;
   const int pers[3] = {s->g.periodic[0] ? 1 : 0, s->g.periodic[1] ? 1 : 0, s->g.periodic[2] ? 1 : 0};
   std::vector<std::pair<int, int>> zr;
+  // planes a wavefront marches: kc planes are four wavefronts' work.  Short
+  // ranges recompute one plane's E in four, but put four times the wavefronts
+  // in flight, and a tile that one metal cell makes general is a quarter as
+  // large.  us per step at kc = 16 against one wavefront over 16 planes:
+  // 128^3 FP32 54 : 68, 150 x 137 x 211 100 : 110, 203^3 163 : 178, 256^3 285 :
+  // 304, 384^3 disks 651 : 690, 512^3 1686 : 1730 (4 rows); 96^3 FP64 45 : 61,
+  // 320^3 FP64 1021 : 1018 (kc = 32, 8 planes: 1009).
+  const int kw = (kc + 3) / 4;
   auto segment = [&](int a, int b) {
-    for (int k = a; k <= b; k += kc) zr.push_back({k, std::min(b, k + kc - 1)});
+    for (int k = a; k <= b; k += kw) zr.push_back({k, std::min(b, k + kw - 1)});
   };
   if (Pz > 0) {
     segment(1, Pz);
@@ -1685,7 +1693,7 @@ int fdtd_autotune(fdtd_sim* s, int steps, int* out_by, int* out_kc) {
     return set_error(FDTD_ERR_STATE, "autotune runs before the first step, on untouched fields");
   FDTD_HIP(hipSetDevice(s->device));
   // candidates: the two-kernel step (by = 0) and one-pass tiles of 64 x by
-  // cells marching kc planes
+  // cells, kc planes cut among four wavefronts
   std::vector<std::pair<int, int>> cand;
   bool ljp = false;
   for (const auto& m : s->mats) ljp |= m.type == 3;

@@ -235,7 +235,7 @@ struct Sim {
   // one-pass step (FUSED engine): E and H of a step read from one copy of
   // the fields and written to the other (E2/H2/d_split2 hold the second
   // copy).  The grid is cut into tiles of 64 x op_by cells (op_by in
-  // {2, 4, 8}) and z ranges of at most op_kc planes (broken at the z PML
+  // {2, 4, 8}) and z ranges of at most op_kc/4 planes (broken at the z PML
   // slabs).  Plain tiles (one dielectric material, no PML, no x- or
   // y-normal source plane) are marched through their planes by one
   // wavefront each, E and H in one pass; the other tiles run the fused

@@ -624,7 +624,7 @@ constexpr bool kXface = sizeof(real) == 4;
 // read from one copy of the fields and written to the other (old: m.eo,
 // m.ho and the splits p.s; new: a.e, a.h and pw.s), so no cell reads a value
 // another workgroup has already replaced, whatever order they run in.  The
-// grid is cut into tiles of 64 x R cells over z ranges of at most kc planes
+// grid is cut into tiles of 64 x R cells over z ranges of at most kc/4 planes
 // (lists built on the host, fdtd_api.hip build_march_tiles):
 //
 //  plain tiles (one dielectric material, no PML cell among the cells they

@@ -337,9 +337,9 @@ int fdtd_commit(fdtd_sim* sim);
 /* Optional, no reference counterpart: pick the FUSED engine's step form by
  * timing `steps` steps of each candidate on this handle -- the two-kernel
  * step with tiles of kc = 1, 2, 4 or 8 planes (each thread marching its
- * column) and the one-pass step, each wavefront marching a tile of 64 x by
- * cells through kc planes (by in {2, 4, 8}, FP64 {2, 4}; kc in {16, 32,
- * 64, 128}).  The timed steps run without sources on the untouched (zero)
+ * column) and the one-pass step, four wavefronts sharing kc planes of a tile
+ * of 64 x by cells (by in {2, 4, 8}, FP64 {2, 4}; kc in {16, 32, 64,
+ * 128}).  The timed steps run without sources on the untouched (zero)
  * fields and leave them zero; they sample the DFT planes as real steps do
  * (into a buffer slot the first real step overwrites) but fold nothing and
  * record no probes.  Call it after set-up and before the first fdtd_step

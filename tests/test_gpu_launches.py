@@ -112,15 +112,16 @@ def test_lists_beside_the_rows_and_apart(n, apart, precision, monkeypatch):
 
 
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
-@pytest.mark.parametrize("by", ["2", "4", "8"])
+@pytest.mark.parametrize("by,kc", [("2", "16"), ("4", "200"), ("8", "2")])
 @pytest.mark.parametrize("case", ["gold_sphere", "periodic_box"])
-def test_marked_stores_of_the_march(case, by, precision, monkeypatch):
+def test_marked_stores_of_the_march(case, by, kc, precision, monkeypatch):
     """The one-pass step with its stores marked nontemporal (what a grid past
-    the memory-side cache runs; FDTD_NT forces a side): the same bits."""
+    the memory-side cache runs; FDTD_NT forces a side), a wavefront marching
+    4 planes, all of the grid's, or 1: the same bits."""
     from test_gpu_onepass import _cases, _run as run, _same as same
 
     spec = _cases()[case]
-    env = {"FDTD_ONEPASS": "1", "FDTD_ONEPASS_BY": by, "FDTD_ONEPASS_KC": "16"}
+    env = {"FDTD_ONEPASS": "1", "FDTD_ONEPASS_BY": by, "FDTD_ONEPASS_KC": kc}
     got = [run(spec, precision, dict(env, FDTD_NT=nt), monkeypatch) for nt in "01"]
     same(*got[0], *got[1])
 
