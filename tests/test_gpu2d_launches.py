@@ -71,3 +71,25 @@ def test_dispersive_cells_and_monitors_on_shared_rows(polarization, tfsf):
         check(f"rows probe {polarization} {tfsf}", relerr(gs.probe(a), os_.probe(b)), 1e-12)
     gs.close()
     os_.close()
+
+
+@pytest.mark.parametrize("polarization", ["tez", "tmz"])
+@pytest.mark.parametrize("nx,nfreq", [(96, 1), (511, 3), (512, 70), (513, 2), (1030, 5)])
+def test_flux_is_the_sum_of_the_read_spectra(polarization, nx, nfreq):
+    """A line's flux, bit for bit the products of its two spectra added cell
+    after cell from zero in FP64: rows below, at and past the 512 cells a
+    wavefront takes at a time."""
+    from fdtd_amd import sim2d
+
+    spec = sim2d.sweep_instance(np.random.default_rng(nx), side=96, nsteps=101, nfreq=nfreq, polarization=polarization)
+    spec["grid"]["nx"] = nx
+    s, ids, _ = sim2d.make_simulation2d(spec, precision="fp32")
+    s.step(101)
+    e, h, sign = (sim2d.EZ2, sim2d.HX2, 1.0) if polarization == "tmz" else (sim2d.EX2, sim2d.HZ2, -1.0)
+    for a in ids:
+        (er, ei), (hr, hi) = s.dft(a, e), s.dft(a, h)
+        p = sign * ((hr * er + hi * ei) * spec["grid"]["ds"])
+        want = np.cumsum(np.concatenate([np.zeros((1, nfreq)), p]), axis=0)[-1]
+        assert np.any(want != 0)
+        assert np.array_equal(s.flux(a), want)
+    s.close()
