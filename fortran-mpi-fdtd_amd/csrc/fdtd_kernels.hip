@@ -2048,6 +2048,72 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int kDftTabRow = 65;  // double2 entries a sample row of the staged table (64 + 1 pad)
 constexpr int kDftFoldGroups = 512;  // workgroups of a fold: two a CU
 
+// One wavefront's share: 16 cells of a slot, NT tiles of 16 frequencies from
+// m0.  Every load -- the block's samples, then the accumulators -- is issued
+// before the first matrix instruction and without a branch: rows past the
+// block's samples, cells past the plane and frequencies past the last are
+// clamped to the last one (the table holds zeros for such samples; such cells
+// and frequencies are not stored).  Loaded under those tests each sample had a
+// wait of its own, and a tile's accumulators were not asked for until its sums
+// were done: a fold of 384 x 384 cells, 4 components, 128 frequencies (2.4 GB
+// read and written) 1000 us then, 638 us now; 150 x 137 cells, 32 frequencies
+// 62 and 35 us; FP64 320 x 320, 64 frequencies 241 and 224 us.  32 frequencies
+// a pass with three wavefronts a SIMD instead of two measured 692, 31 and 258.
+template <typename real, int NT>
+__device__ __forceinline__ void dft_fold_tile(const real* __restrict__ samp, const double2* lt, uint32_t np, int nslots,
+                                              int slot, int64_t cell, int nfreq, int m0, int count, double dt,
+                                              double* __restrict__ re, double* __restrict__ im, int jj, int kk) {
+  const bool cin = cell < (int64_t)np;
+  const int64_t cc = cin ? cell : (int64_t)np - 1;
+  real f[kDftBlock / 4];  // this lane's samples: b = 4 st + kk
+#pragma unroll
+  for (int st = 0; st < kDftBlock / 4; ++st) {
+    const int b = min(4 * st + kk, count - 1);
+    f[st] = samp[(uint64_t)(uint32_t)(b * nslots + slot) * np + cc];
+  }
+  __builtin_amdgcn_sched_barrier(0);  // the samples first: the sums wait for them alone
+  double ar[NT][4], ai[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const uint64_t o = (uint64_t)(uint32_t)min(m0 + 16 * t + kk + 4 * v, nfreq - 1) * np + cc;
+      ar[t][v] = re[o];
+      ai[t][v] = im[o];
+    }
+  // the samples are in, the accumulators still under way: without this the
+  // compiler moves each sample's load to the step below that uses it
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int st = 0; st < kDftBlock / 4; ++st) asm volatile("" : "+v"(f[st]));
+  v4d dc[NT], ds[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) dc[t] = ds[t] = (v4d){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int st = 0; st < kDftBlock / 4; ++st) {  // every lane: the matrix instructions need them all
+    if (4 * st >= count) break;
+    const double fv = (double)f[st];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const double2 cs = lt[(4 * st + kk) * kDftTabRow + 16 * t + jj];
+      dc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(cs.x, fv, dc[t], 0, 0, 0);
+      ds[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(cs.y, fv, ds[t], 0, 0, 0);
+    }
+  }
+  if (!cin) return;
+  asm volatile("" : "+v"(m0));  // the addresses again, not kept over the sums (registers)
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int m = m0 + 16 * t + kk + 4 * v;
+      if (m >= nfreq) continue;
+      const uint64_t o = (uint64_t)(uint32_t)m * np + cell;
+      re[o] = ar[t][v] + dc[t][v] * dt;
+      im[o] = ai[t][v] + ds[t][v] * dt;
+    }
+}
+
 template <typename real>
 __global__ __launch_bounds__(256, 2) void k_dft_accum(const real* __restrict__ samp, int64_t np, int nslots, int nfreq,
                                                    int count, const double* __restrict__ tab, double dt,
@@ -2067,52 +2133,24 @@ __global__ __launch_bounds__(256, 2) void k_dft_accum(const real* __restrict__ s
     __syncthreads();
     // wave tiles of 16 cells of one slot, strided over the grid (the loop
     // count is uniform per wavefront; no barrier inside)
+    const int nt = (min(64, nfreq - m0) + 15) / 16;
     for (int64_t wt = (int64_t)blockIdx.x * 4 + w; wt < nwt; wt += (int64_t)gridDim.x * 4) {
       const int slot = (int)(wt / ntile);
       const int64_t cell = (wt - (int64_t)slot * ntile) * 16 + jj;
-      const bool cin = cell < np;
-      double f[kDftBlock / 4];  // this lane's samples: b = 4 st + kk
-#pragma unroll
-      for (int st = 0; st < kDftBlock / 4; ++st) {
-        const int b = 4 * st + kk;
-        f[st] = (cin && b < count) ? (double)samp[((int64_t)b * nslots + slot) * np + cell] : 0.0;
-      }
-      v4d dc[4], ds[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) dc[t] = ds[t] = (v4d){0.0, 0.0, 0.0, 0.0};
-#pragma unroll 1
-      for (int st = 0; st < kDftBlock / 4; ++st) {  // every lane: the matrix instructions need them all
-        if (4 * st >= count) break;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const double2 cs = lt[(4 * st + kk) * kDftTabRow + 16 * t + jj];
-          dc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(cs.x, f[st], dc[t], 0, 0, 0);
-          ds[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(cs.y, f[st], ds[t], 0, 0, 0);
-        }
-      }
-      if (!cin) continue;  // cells past the plane's end: no accumulator
       double* re = acc + (int64_t)slot * 2 * nfreq * np;
       double* im = re + (int64_t)nfreq * np;
-      // accumulators: all loads of a tile pair before its stores
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        double ar[4], ai[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int m = m0 + 16 * t + kk + 4 * v;
-          const int64_t q = (int64_t)m * np + cell;
-          ar[v] = m < nfreq ? re[q] : 0.0;
-          ai[v] = m < nfreq ? im[q] : 0.0;
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int m = m0 + 16 * t + kk + 4 * v;
-          if (m >= nfreq) continue;
-          const int64_t q = (int64_t)m * np + cell;
-          re[q] = ar[v] + dc[t][v] * dt;
-          im[q] = ai[v] + ds[t][v] * dt;
-        }
-      }
+      auto go = [&](auto n) {
+        dft_fold_tile<real, decltype(n)::value>(samp, lt, (uint32_t)np, nslots, slot, cell, nfreq, m0, count, dt, re,
+                                                im, jj, kk);
+      };
+      if (nt == 4)
+        go(std::integral_constant<int, 4>{});
+      else if (nt == 3)
+        go(std::integral_constant<int, 3>{});
+      else if (nt == 2)
+        go(std::integral_constant<int, 2>{});
+      else
+        go(std::integral_constant<int, 1>{});
     }
   }
 }

@@ -143,3 +143,26 @@ def test_marked_d_of_the_reference_order(case, precision, golden, monkeypatch):
     assert np.abs(got[0].field(0)).max() > 0
     for c in range(9):
         assert np.array_equal(got[0].field(c), got[1].field(c)), c
+
+
+@pytest.mark.parametrize("nfreq", [1, 16, 17, 33, 49, 64, 65, 130])
+def test_fold_tiles(nfreq):
+    """Spectra at nfreq frequencies (16 a tile, 64 a pass) over planes whose
+    cells end inside a tile of 16, folded over blocks of 1, 3, 63, 64 and 5
+    samples: FP64 against the oracle at the parity bar."""
+    import oracle
+    from fdtd_amd import workloads
+
+    n = (33, 35, 38)
+    spec = _spec(n, groups=1, planes=3)
+    spec["pml"]["npml"] = [4, 4, 6]
+    om = workloads.wavelength_frequencies(400e-9, 900e-9, nfreq)
+    for d in spec["dft"]:
+        d.update(omega=list(om), n_begin=1)
+    a, ia, _ = _run(spec, "fp64", (1, 3, 63, 64, 5))
+    o, io, _ = oracle.make_simulation(spec)
+    o.step(136)
+    for x, y, d in zip(ia, io, spec["dft"]):
+        for c in d["comps"]:
+            for u, v in zip(a.dft(x, c), o.dft(y, c)):
+                check(f"fold {nfreq} {c}", relerr(u, v), 1e-12)
