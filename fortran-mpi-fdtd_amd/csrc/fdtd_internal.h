@@ -119,6 +119,14 @@ struct HostSource {
 // when the chunks are multiples of kDftBlock (the pool's 64, 256).
 constexpr int kDftBlock = 64;
 
+// Large result reads (read_back): from how many bytes, host threads, bytes of
+// each thread's two pinned slots (16 MiB a read), reads that may hold such
+// slots at once.
+constexpr size_t kReadRingFrom = (size_t)16 << 20;
+constexpr int kReadThreads = 4;
+constexpr size_t kReadSlot = (size_t)2 << 20;
+constexpr int kReadRings = 4;
+
 // Planes a general workgroup of the one-pass step marches through (at most).
 constexpr int kGenKc = 4;
 

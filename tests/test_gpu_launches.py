@@ -166,3 +166,49 @@ def test_fold_tiles(nfreq):
         for c in d["comps"]:
             for u, v in zip(a.dft(x, c), o.dft(y, c)):
                 check(f"fold {nfreq} {c}", relerr(u, v), 1e-12)
+
+
+@pytest.mark.parametrize("n", [(204, 205, 16), (409, 411, 16)])
+def test_large_reads_from_two_threads(n):
+    """Spectra of 10 and 43 MB an array, read through the pinned slots (from
+    16 MiB on, 2 MiB a slice, the last one short) by two threads from two
+    handles at once: the bytes of the same frequencies on planes of two
+    frequencies each, whose reads stay below the line."""
+    import threading
+
+    import fdtd_amd
+    from fdtd_amd import workloads
+
+    nf = 32
+    om = list(workloads.wavelength_frequencies(400e-9, 900e-9, nf))
+    sims = []
+    for q in range(2):
+        spec = workloads.c1_gold_sphere(nsteps=8, n=16)
+        spec["grid"].update(nx=n[0], ny=n[1], nz=n[2])
+        spec["pml"]["npml"] = [2, 2, 2]
+        spec["materials"] = [{"type": "dielectric", "region": fdtd_amd.box((1, 1, 1), n), "eps": 1.0 + q}]
+        spec["sources"][0]["index"] = 7
+        spec["dft"] = [{"axis": 2, "index": 8, "omega": w, "comps": [0, 4]}
+                       for w in [om] + [om[f:f + 2] for f in range(0, nf, 2)]]
+        spec["probes"] = []
+        s, i, _ = fdtd_amd.make_simulation(spec, precision="fp32", engine="fused")
+        s.step(8)
+        sims.append((s, i))
+    got = [None, None]
+
+    def read(q):
+        s, i = sims[q]
+        got[q] = [s.dft(i[0], c) for c in (0, 4)]
+
+    th = [threading.Thread(target=read, args=(q,)) for q in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for (s, i), g in zip(sims, got):
+        for c, parts in zip((0, 4), g):
+            assert np.any(parts[0] != 0) and np.any(parts[1] != 0)
+            for k in range(nf // 2):
+                for u, v in zip(parts, s.dft(i[1 + k], c)):
+                    assert np.array_equal(u[:, :, 2 * k:2 * k + 2], v)
+        s.close()
