@@ -126,6 +126,8 @@ constexpr size_t kReadRingFrom = (size_t)16 << 20;
 constexpr int kReadThreads = 4;
 constexpr size_t kReadSlot = (size_t)2 << 20;
 constexpr int kReadRings = 4;
+// Device buffer of a packed field read (at least one plane).
+constexpr size_t kPackBytes = (size_t)32 << 20;
 
 // Planes a general workgroup of the one-pass step marches through (at most).
 constexpr int kGenKc = 4;
@@ -230,7 +232,7 @@ struct Sim {
   int call_base = 0;  // steps done before the current fdtd_step call
   // reductions
   double* d_red = nullptr;
-  int red_cap = 0;
+  size_t red_cap = 0;
 
   std::vector<DevBuf> allocs;
   size_t dev_bytes = 0;
@@ -311,6 +313,7 @@ double* reduction_buffer(Sim* s, size_t bytes);  // reusable, grown with dev_all
 int launch_step(Sim* s);           // one full time step at s->n_done + 1
 int launch_dft_flush(Sim* s);      // fold every buffered DFT sample
 int launch_energy(Sim* s, double* we, double* wh);
+int launch_pack(Sim* s, const void* field, int k0, int planes, double* out);  // interior planes, FP64, x fastest
 int launch_flux(Sim* s, int id, double* S);
 int flux_check(Sim* s, int id);                            // the plane carries the four components
 int launch_flux_into(Sim* s, int id, double* dS, double* S);  // dS: nfreq doubles of device memory

@@ -3107,6 +3107,32 @@ int flux_check(Sim* s, int id) {
   return 0;
 }
 
+// Interior rows of planes k0.. of a field, as FP64 without the ghosts: a
+// wavefront 64 cells of a row, bound by its writes (8 B a cell).
+template <typename real>
+__global__ __launch_bounds__(256) void k_pack(const real* __restrict__ f, int nx, int ny, int64_t px, int64_t pxy,
+                                              int k0, int64_t rows, double* __restrict__ out) {
+  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= rows) return;
+  const int64_t k = r / ny, j = r - k * ny;
+  const real* row = f + px * (j + 1) + pxy * (k0 + k);
+  for (int i = (int)threadIdx.x & 63; i < nx; i += 64) out[r * nx + i] = (double)row[i + 1];
+}
+
+int launch_pack(Sim* s, const void* field, int k0, int planes, double* out) {
+  FDTD_HIP(hipSetDevice(s->device));
+  const int64_t rows = (int64_t)s->ny * planes;
+  const dim3 nb((unsigned)((rows + 3) / 4));
+  if (s->prec == FDTD_FP32)
+    hipLaunchKernelGGL(k_pack<float>, nb, dim3(256), 0, s->stream, (const float*)field, s->nx, s->ny, s->px, s->pxy,
+                       k0, rows, out);
+  else
+    hipLaunchKernelGGL(k_pack<double>, nb, dim3(256), 0, s->stream, (const double*)field, s->nx, s->ny, s->px, s->pxy,
+                       k0, rows, out);
+  FDTD_HIP(hipGetLastError());
+  return 0;
+}
+
 int launch_flux(Sim* s, int id, double* S) {
   int rc = flux_check(s, id);
   if (rc) return rc;

@@ -212,3 +212,20 @@ def test_large_reads_from_two_threads(n):
                 for u, v in zip(parts, s.dft(i[1 + k], c)):
                     assert np.array_equal(u[:, :, 2 * k:2 * k + 2], v)
         s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("n", [(1, 5, 3), (63, 7, 5), (64, 4, 9), (129, 3, 2), (2049, 1025, 3)])
+def test_packed_field_reads(n, precision):
+    """A field read back equals the field set: rows of 1, 63, 64 and 129
+    cells, and one plane a pass where two exceed the device's buffer (17 MB
+    a plane)."""
+    import fdtd_amd
+
+    sim = fdtd_amd.Simulation(n[0], n[1], n[2], 1e-9, 0.5, precision=precision, engine="fused")
+    rng = np.random.default_rng(n[0])
+    for c in (0, 4):
+        f = rng.standard_normal(n).astype(np.float32).astype(np.float64)
+        sim.set_field(c, f)
+        assert np.array_equal(sim.field(c), f), c
+    sim.close()
