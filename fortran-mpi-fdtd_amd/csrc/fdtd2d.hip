@@ -251,6 +251,7 @@ struct Batch {
   int prec = FDTD_FP64;
   int device = 0;
   hipStream_t stream = nullptr;
+  bool nt_d = false;  // the field arrays outgrow the memory-side cache (batch_build)
   void* d_inst = nullptr;
   int32_t* d_ctl = nullptr;  // [count][2]: steps done at the block's start, target
   int32_t* d_tile_inst = nullptr;
@@ -618,7 +619,23 @@ __device__ __forceinline__ void mon_cell(const Inst<real>& S, int i, int j, int 
     }
 }
 
-template <typename real>
+// D of a strip, which nothing else of the step reads; NT: nontemporal (k2_e)
+template <bool NT, typename real>
+__device__ __forceinline__ real get_d(const real* p) {
+  if constexpr (NT)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
+}
+template <bool NT, typename real>
+__device__ __forceinline__ void put_d(real* p, real v) {
+  if constexpr (NT)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+
+template <typename real, bool NT>
 __device__ __forceinline__ void e_tez_strip(const Inst<real>& S, int i, int j0) {
   constexpr int R = kRowsPerWave;
   const int px = S.px;
@@ -631,8 +648,8 @@ __device__ __forceinline__ void e_tez_strip(const Inst<real>& S, int i, int j0) 
     const int c = c0 + px * r;
     hz[r + 1] = S.hz[c];
     hzi[r] = S.hz[c - 1];
-    dx[r] = S.dx[c];
-    dy[r] = S.dy[c];
+    dx[r] = get_d<NT>(S.dx + c);
+    dy[r] = get_d<NT>(S.dy + c);
     id[r] = S.matid[c];
   }
   Mat<real> m[R];
@@ -643,8 +660,8 @@ __device__ __forceinline__ void e_tez_strip(const Inst<real>& S, int i, int j0) 
     const int c = c0 + px * r;
     const real dxv = dx[r] + S.ku * (hz[r + 1] - hz[r]);
     const real dyv = dy[r] - S.ku * (hz[r + 1] - hzi[r]);
-    if (m[r].act[1] != ACT_ADE) S.dy[c] = dyv;
-    if (m[r].act[0] != ACT_ADE) S.dx[c] = dxv;
+    if (m[r].act[1] != ACT_ADE) put_d<NT>(S.dy + c, dyv);
+    if (m[r].act[0] != ACT_ADE) put_d<NT>(S.dx + c, dxv);
     if (m[r].act[1] == ACT_DIEL) {
       const real ey = dyv * m[r].gax[1];
       S.ey[c] = ey;
@@ -681,7 +698,7 @@ __device__ __forceinline__ void h_tez_strip(const Inst<real>& S, int i, int j0) 
   }
 }
 
-template <typename real>
+template <typename real, bool NT>
 __device__ __forceinline__ void e_tmz_strip(const Inst<real>& S, int i, int j0) {
   constexpr int R = kRowsPerWave;
   const int px = S.px;
@@ -695,7 +712,7 @@ __device__ __forceinline__ void e_tmz_strip(const Inst<real>& S, int i, int j0) 
     hx[r + 1] = S.hx[c];
     hy[r] = S.hy[c];
     hyi[r] = S.hy[c - 1];
-    dz[r] = S.dz[c];
+    dz[r] = get_d<NT>(S.dz + c);
     id[r] = S.matid[c];
   }
   Mat<real> m[R];
@@ -705,7 +722,7 @@ __device__ __forceinline__ void e_tmz_strip(const Inst<real>& S, int i, int j0) 
   for (int r = 0; r < R; ++r) {
     const int c = c0 + px * r;
     const real d = dz[r] + S.ku * ((hy[r] - hyi[r]) + (-hx[r + 1] + hx[r]));
-    if (m[r].act[0] != ACT_ADE) S.dz[c] = d;
+    if (m[r].act[0] != ACT_ADE) put_d<NT>(S.dz + c, d);
     if (m[r].act[0] == ACT_DIEL) {
       const real ez = d * m[r].gax[0];
       S.ez[c] = ez;
@@ -839,8 +856,10 @@ __host__ __device__ __forceinline__ int list_blocks(int n) { return (n + 7) & ~7
 // while that does not pass its target ctl[2q+1].  The E launch starts with
 // the dispersive cells' work list (no cell reads what another of the launch
 // writes); they come first because a cell's 12-26 words of FP64 state take
-// longer than a tile.
-template <typename real>
+// longer than a tile.  NT: D nontemporal, for batches whose fields outgrow the
+// memory-side cache, where E and H, half of the arrays, then more often stay in
+// it from one half step to the next (batch_build).
+template <typename real, bool NT>
 __global__ __launch_bounds__(kTX * kWaves) void k2_e(const Inst<real>* __restrict__ I, const int32_t* __restrict__ ctl,
                                                      const int32_t* __restrict__ tile_inst, int ntiles,
                                                      const int4* __restrict__ ade, int nade, int st) {
@@ -865,9 +884,9 @@ __global__ __launch_bounds__(kTX * kWaves) void k2_e(const Inst<real>* __restric
     if (i > S.nx) continue;
     if (strip_plain(S, (lt % S.ntx) * kTX, j0, true)) {
       if (S.tmz)
-        e_tmz_strip(S, i, j0);
+        e_tmz_strip<real, NT>(S, i, j0);
       else
-        e_tez_strip(S, i, j0);
+        e_tez_strip<real, NT>(S, i, j0);
       continue;
     }
     real carry = 0;
@@ -1792,6 +1811,22 @@ int batch_build(Batch* b) {
   FDTD_HIP(hipSetDevice(b->device));
   hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e != hipSuccess) return hip_check(e, "hipStreamCreate");
+  {
+    // D is marked nontemporal (k2_e) where what a step goes through -- fields,
+    // material ids, dispersive state -- takes more than 3/4 of the 256 MiB
+    // memory-side cache: below, the next step finds it there.  us per step,
+    // marked against not, 16 simulations FP32: 640^2 (135 MiB) 62 : 57, 800^2
+    // (201 MiB) 86 : 91, 900^2 106 : 119, 1000^2 123 : 140, 1300^2 216 : 241; 256
+    // of 128^2 (191 MiB, most of it state) 80 : 81; 24 of 256-2048 cells a side
+    // (763 MiB) 352 : 367.
+    uint64_t bytes = 0;
+    for (const Sim* s : b->sims) {
+      bytes += (uint64_t)s->ncell * (s->wsize * (s->tmz ? 4 : 5) + 1);
+      for (const auto& g : s->groups) bytes += (uint64_t)g.ncells * g.nstate * 2 * sizeof(double);
+    }
+    const char* e = std::getenv("FDTD_NT");
+    b->nt_d = e ? std::atoi(e) != 0 : bytes > ((uint64_t)256 << 20) / 4 * 3;
+  }
   const size_t isz = b->prec == FDTD_FP32 ? sizeof(Inst<float>) : sizeof(Inst<double>);
   b->d_inst = alloc_in(b->allocs, nullptr, isz * count);
   b->d_ctl = (int32_t*)alloc_in(b->allocs, nullptr, sizeof(int32_t) * 2 * count);
@@ -1855,8 +1890,11 @@ void enqueue_block(Batch* b) {
     // the line's E half step may precede k2_e, which reads only the line's h
     if (b->ntf)
       hipLaunchKernelGGL(k2_tfsf_line<real>, dim3((unsigned)b->ntf), dim3(256), 0, st, I, ctl, b->d_tfl, b->ntf, 0, s);
-    hipLaunchKernelGGL(k2_e<real>, dim3(grid + (unsigned)list_blocks(b->nade)), dim3(kTX * kWaves), 0, st, I, ctl,
-                       b->d_tile_inst, b->ntiles, b->d_ade, b->nade, s);
+    auto go_e = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(grid + (unsigned)list_blocks(b->nade)), dim3(kTX * kWaves), 0, st, I, ctl,
+                         b->d_tile_inst, b->ntiles, b->d_ade, b->nade, s);
+    };
+    b->nt_d ? go_e(k2_e<real, true>) : go_e(k2_e<real, false>);
     if (b->nljp)
       hipLaunchKernelGGL(k2_ljp<real>, dim3((unsigned)b->nljp), dim3(kChunk), 0, st, I, ctl, b->d_ljp, b->nljp, s);
     hipLaunchKernelGGL(k2_h<real>, dim3(grid), dim3(kTX * kWaves), 0, st, I, ctl, b->d_tile_inst, b->ntiles, s);

@@ -93,3 +93,25 @@ def test_flux_is_the_sum_of_the_read_spectra(polarization, nx, nfreq):
         assert np.any(want != 0)
         assert np.array_equal(s.flux(a), want)
     s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("polarization", ["tez", "tmz"])
+def test_marked_d(polarization, precision, monkeypatch):
+    """The E launch with D marked nontemporal (what a batch past the
+    memory-side cache runs; FDTD_NT forces a side): the same bits."""
+    from fdtd_amd import sim2d
+
+    spec = sim2d.sweep_instance(np.random.default_rng(4), side=130, nsteps=150, polarization=polarization)
+    comps = (sim2d.EZ2, sim2d.HX2, sim2d.HY2, sim2d.DZ2) if polarization == "tmz" else \
+        (sim2d.EX2, sim2d.EY2, sim2d.HZ2, sim2d.DX2, sim2d.DY2)
+    got = []
+    for nt in "01":
+        monkeypatch.setenv("FDTD_NT", nt)
+        s, ids, _ = sim2d.make_simulation2d(spec, precision=precision)
+        s.step(150)
+        got.append([s.field(c) for c in comps] + [s.flux(a) for a in ids])
+        s.close()
+    assert np.any(got[0][0] != 0)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
