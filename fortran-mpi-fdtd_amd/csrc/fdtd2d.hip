@@ -18,7 +18,7 @@
 // sim2 = FDTDsimulations/2D/air-nanoAntennas_Si02-Sisubstrate/):
 //   E: rows j0..j1 (npmly..N_y-npmly): D += Ku curl Hz (include/
 //      myfdtd_2Dfunc.f90:16-32), line sources on Dx, E = D*gax of the last
-//      dielectric writer (dispersive cells: their own launch); in the y slabs
+//      dielectric writer (dispersive cells: beside the tiles); in the y slabs
 //      the split-field PML (mod2/BERpmly_HzExEy_mod.f90:96-123) with Ex
 //      handed to the main field on rows 1..ja and jb..N_y (:144-178);
 //      periodic x: the ghost columns of Ey follow (mympi_2Dfunc.f90).

@@ -534,26 +534,8 @@ int commit_impl(Sim* s) {
   s->engine = eng;
   if ((int)s->srcs.size() > kMaxSrc) return set_error(FDTD_ERR_ARG, "too many sources");
 
-  // launch shape: whole 64-lane wavefronts along x, 256 threads per block
-  {
-    const int r = (s->nx + 63) / 64 * 64;
-    s->bx = std::min(256, r);
-    s->by = 256 / s->bx;
-    // tuning overrides: FDTD_BLOCK_X in {64,128,256,512}, FDTD_BLOCK_Y in
-    // {1,2,4,8} (at most 512 threads), FDTD_XCD_MAP in {0,1}
-    if (const char* e = std::getenv("FDTD_BLOCK_X")) {
-      const int v = std::atoi(e);
-      if (v == 64 || v == 128 || v == 256 || v == 512) {
-        s->bx = v;
-        s->by = std::max(1, 256 / v);
-      }
-    }
-    if (const char* e = std::getenv("FDTD_BLOCK_Y")) {
-      const int v = std::atoi(e);
-      if ((v == 1 || v == 2 || v == 4 || v == 8) && v * s->bx <= 512) s->by = v;
-    }
-    if (const char* e = std::getenv("FDTD_XCD_MAP")) s->xcdmap = std::atoi(e) != 0;
-  }
+  // FDTD_XCD_MAP=0: blocks in launch order, not dealt to the XCDs
+  if (const char* e = std::getenv("FDTD_XCD_MAP")) s->xcdmap = std::atoi(e) != 0;
   // layout: rows are whole 128-byte lines and the first interior cell of
   // every row starts a line (the field pointer is offset by line-1 cells
   // inside its allocation), so each wavefront's 64 cells span the fewest lines
@@ -1254,7 +1236,7 @@ int build_march_tiles(Sim* s, int by, int kc) {
   std::vector<int> ys, zs;
   // pass 0: the plain tiles of by rows; pass 1 (x-face tiles only): the
   // tiles with lanes in an x slab, bx rows each (FDTD_XFACE_BY, 2 or 4),
-  // listed after the others and marched by their own launch
+  // listed after the others
   const char* xb_env = std::getenv("FDTD_XFACE_BY");
   const int bx = xb_env && std::atoi(xb_env) == 4 ? 4 : 2;
   for (int pass = 0; pass < (xface ? 2 : 1); ++pass) {
@@ -2275,8 +2257,8 @@ int fdtd_algorithmic_bytes(fdtd_sim* s, int kernel, double* bytes) {
     const int P = s->pml_mode == FDTD_PML_REF_Y ? s->pml.npml[1] : 0;
     const double Nm = (double)s->nx * (s->ny - 2 * P) * s->nz;
     const double Ns = (double)s->nx * 2 * P * s->nz;
-    if (kernel == FDTD_K_E || kernel == FDTD_K_H) b = w * 9.0 * Nm;
-    if (kernel == FDTD_K_MAT) b = w * 6.0 * N;
+    if (kernel == FDTD_K_E) b = w * (9.0 * Nm + 3.0 * N);  // E from the D just advanced: written only
+    if (kernel == FDTD_K_H) b = w * 9.0 * Nm;
     if (kernel == FDTD_K_PML_E || kernel == FDTD_K_PML_H) b = w * 24.0 * Ns;
     if (kernel == FDTD_K_ADE)
       for (auto& g : s->groups) b += (w * 6.0 + 8.0 * 2.0 * 3.0 * g.nstate) * (double)g.ncells;

@@ -237,9 +237,7 @@ struct Sim {
   std::vector<DevBuf> allocs;
   size_t dev_bytes = 0;
 
-  // launch shape of the cell-parallel kernels (x threads, y threads) and
-  // whether fused kernels deal tiles to XCDs in contiguous runs
-  int bx = 64, by = 4;
+  // whether tiles are dealt to XCDs in contiguous runs
   int xcdmap = 1;
   bool nt_march = false, nt_d = false;  // streams_past_llc of the one-pass fields, of STAGED D
   // one-pass step (FUSED engine): E and H of a step read from one copy of

@@ -2548,10 +2548,6 @@ void flush_pending(Sim* s) {
   launch_monitors(s, m);
 }
 
-inline dim3 cell_grid(int nx, int nrows, int nz, dim3 blk) {
-  return dim3((unsigned)((nx + blk.x - 1) / blk.x), (unsigned)((nrows + blk.y - 1) / blk.y), (unsigned)nz);
-}
-
 template <typename real>
 SrcArgs<real> source_args(Sim* s, int n, int* nsrc) {
   SrcArgs<real> sa{};
@@ -2618,7 +2614,6 @@ int step_impl(Sim* s) {
   int nsrc = 0;
   SrcArgs<real> src = source_args<real>(s, n, &nsrc);
   if (s->dry) nsrc = 0;
-  const dim3 blk((unsigned)s->bx, (unsigned)s->by, 1);
   hipStream_t st = s->stream;
   auto ade_coef = [&](const AdeGroup& g) {  // FP64 in both precisions
     AdeCoef<double> c = g.coef;

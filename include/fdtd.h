@@ -83,19 +83,20 @@ enum {
 /* Stepping engines (fdtd_grid.engine). */
 enum {
   FDTD_ENGINE_AUTO = 0,   /* STAGED for REF_Y, FUSED otherwise                  */
-  FDTD_ENGINE_STAGED = 1, /* one kernel per reference stage, D kept everywhere  */
+  FDTD_ENGINE_STAGED = 1, /* the reference's stages in order, D kept everywhere */
   FDTD_ENGINE_FUSED = 2   /* fused E / H kernels, D kept only in ADE cells      */
 };
 
 /* Kernel ids for fdtd_kernel_stats. */
 enum {
-  FDTD_K_E = 0,       /* E half step (fused), updateD (staged), or the
-                         one-pass step over its plain tiles            */
+  FDTD_K_E = 0,       /* E half step (fused), updateD, sources and
+                         dielectric E (staged), or the one-pass step over
+                         its plain tiles                               */
   FDTD_K_H = 1,       /* H half step (fused) or updateH (staged)   */
   FDTD_K_ADE = 2,     /* dispersive cells (gold, graphene)         */
   FDTD_K_PML_E = 3,   /* staged split-field E                       */
   FDTD_K_PML_H = 4,   /* staged split-field H                       */
-  FDTD_K_MAT = 5,     /* staged dielectric E = D*gax + source       */
+  FDTD_K_MAT = 5,     /* TFSF: incident line, H corrections         */
   FDTD_K_MON = 6,     /* DFT monitors and probes                    */
   FDTD_K_GEN_E = 7,   /* one-pass step: E of its general tiles      */
   FDTD_K_GEN_H = 8,   /* one-pass step: H of its general tiles      */
@@ -413,7 +414,10 @@ int fdtd_energy(fdtd_sim* sim, double* we, double* wh);
 /* ---- introspection -------------------------------------------------------- */
 int fdtd_memory_bytes(fdtd_sim* sim, size_t* bytes);
 /* HIP-event timing of every kernel launch while enabled (adds events to the
- * handle's stream; off by default).                                        */
+ * handle's stream; off by default).  While it is on, the parts that share a
+ * launch otherwise (tiles, dispersive cells, monitors, PML slabs) have
+ * launches of their own, so that each has its time: a step then takes longer,
+ * with the same results.                                                   */
 int fdtd_set_profiling(fdtd_sim* sim, int on);
 int fdtd_kernel_stats(fdtd_sim* sim, int kernel, double* total_ms,
                       int64_t* launches);
