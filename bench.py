@@ -6,9 +6,11 @@ One "step" is one full time step of the workload (E half step with the
 dispersive cells and the PML, H half step, DFT monitors and probes) over the
 whole 512^3 grid; inputs are resident in HBM before the timed region.
 
-Prints ONE JSON line.  ``roofline`` is measured live: HIP events around every
-launch of the dominant kernel (the fused E update) on the handle's stream,
-its algorithmic bytes per launch divided by its mean duration.
+Prints ONE JSON line.  ``roofline`` is measured live, in up to 20 steps after
+the timed ones: HIP events around every launch of the dominant kernel (the
+one-pass march, or the E half step) on the handle's stream, its algorithmic
+bytes per launch divided by its mean duration.  (With the events on, what
+shares a launch in the timed steps has launches of its own.)
 ``cpu_baseline`` times the FP64 CPU oracle (OpenMP) on 60 steps of the
 same 512^3 workload on this host.  ``served_stream`` replays a seeded
 Poisson stream of smaller gold jobs (64-320 cells a side) through the
@@ -40,11 +42,14 @@ def run_gpu(spec, precision, steps, warmup):
     setup_s = time.time() - t0
     sim.step(warmup)
     sim.sync()
-    sim.set_profiling(True)
     t1 = time.perf_counter()
     sim.step(steps)
     sim.sync()
     elapsed = time.perf_counter() - t1
+    flux = [float(v) for v in sim.flux(ids[2])[:4]]
+    sim.set_profiling(True)
+    sim.step(min(steps, 20))
+    sim.sync()
     nx, ny, nz = sim.shape
     cells = nx * ny * nz
     kern = {}
@@ -69,7 +74,7 @@ def run_gpu(spec, precision, steps, warmup):
         "setup_s": setup_s,
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": ach / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "k_march_plain" if onepass else "k_fused_e",
+                     "kernel": "k_march" if onepass else "k_step_e",
                      "bytes_per_launch": e["bytes_per_launch"], "mean_launch_ms": e["mean_ms"]},
         "h_update": h_upd,
         "kernels": kern,
@@ -78,7 +83,6 @@ def run_gpu(spec, precision, steps, warmup):
         "device_bytes": sim.memory_bytes(),
         "cell_counts": dict(zip(("pml", "ade"), sim.cell_counts())),
     }
-    flux = [float(v) for v in sim.flux(ids[2])[:4]]
     out["flux_sample"] = flux
     sim.close()
     return out
@@ -418,22 +422,22 @@ def main():
         c3 = c3_mixed_precision(args)
         print(f"[bench] c3 fp32 {c3['fp32_mcells_per_s']:.0f} fp64 {c3['fp64_mcells_per_s']:.0f} Mcell/s, "
               f"spectra err {max(c3['fp32_spectra_max_rel_err_vs_gpu_fp64']):.2e}", file=sys.stderr, flush=True)
-    # the FP32 x-face tiles (plain tiles reaching into an x PML slab, a
-    # launch of their own beside the dominant kernel): the same figures
+    # the FP32 x-face tiles (plain tiles reaching into an x PML slab, beside
+    # the plain ones in the dominant kernel): the same figures
     xf = r32["kernels"].get("x_face")
     xface = None
     if xf:
         ach = xf["bytes_per_launch"] / (xf["mean_ms"] * 1e-3) / 1e9
         xface = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
-                 "traffic": None, "kernel": "k_march_plain_xf", "bytes_per_launch": xf["bytes_per_launch"],
+                 "traffic": None, "kernel": "k_march_xf", "bytes_per_launch": xf["bytes_per_launch"],
                  "mean_launch_ms": xf["mean_ms"]}
     if args.n == 512 and args.seed == 0:  # the workload the summary profiles
-        tb, src = profiled_traffic(r32["roofline"]["kernel"], "fp32", "k_march_plain_gold_dimer_512.md")
+        tb, src = profiled_traffic(r32["roofline"]["kernel"], "fp32", "k_march_gold_dimer_512.md")
         r32["roofline"]["traffic"] = tb
         if tb is not None:
             r32["roofline"]["traffic_source"] = src
         if xface:
-            xface["traffic"], _ = profiled_traffic("k_march_plain_xf", "fp32", "k_march_plain_gold_dimer_512.md")
+            xface["traffic"], _ = profiled_traffic("k_march_xf", "fp32", "k_march_gold_dimer_512.md")
     line = {
         "metric": METRIC,
         "value": r32["value"],
