@@ -10,7 +10,6 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 #include "fdtd_internal.h"
@@ -1022,16 +1021,17 @@ int read_back(Sim* s, std::vector<ReadPart> parts) {
     }
     if (e != hipSuccess) err.store((int)e);
   };
-  std::vector<std::thread> th;
+  std::thread th[kReadThreads - 1];
   for (int w = 1; w < kReadThreads; ++w) {
     try {
-      th.emplace_back(work, w);
-    } catch (const std::system_error&) {
+      th[w - 1] = std::thread(work, w);
+    } catch (...) {
       break;  // no more threads: those there are (the caller's at least) read it all
     }
   }
   work(0);
-  for (auto& t : th) t.join();
+  for (auto& t : th)
+    if (t.joinable()) t.join();
   const hipError_t es = hipStreamSynchronize(s->stream);
   const hipError_t e = err.load() != hipSuccess ? (hipError_t)err.load() : es;
   return done(e == hipSuccess ? 0 : hip_check(e, "result read"));
