@@ -1834,6 +1834,7 @@ __global__ __launch_bounds__(256) void k_monitors(FieldArgs<real> a, MonList<rea
 // TFSF wave 103 / 84, 160^3 FP32 91 / 80.
 struct Parts {
   int32_t mon, ade, mix, xf, plain, gen;  // blocks of each part (0: not in this launch)
+  int32_t line;                           // 8: the incident line's block (before mon), 0: none
 };
 
 // The kernel arguments a cell update needs, loaded in one batch: left to the
@@ -1883,11 +1884,54 @@ __global__ __launch_bounds__(256) void k_step_e(FieldArgs<real> a, PmlArgs<real>
   e_column<real, KZ>(a, p, src, nsrc, i, j, tz, a.h[0], a.h[1], a.h[2], a.e[0], a.e[1], a.e[2]);
 }
 
-// Two-kernel step, H half: monitors of this step (E), every cell.
+// point probes, sim3/program.f90:445-451
+// ---------------------------------------------------------------------------
+// TFSF incident line (sim1/program.f90:217-262, mod1/BERpmly_ExHz_mod.f90).
+// One workgroup walks the line; the PML object's own fields pe, ph live on
+// cells 1..npml and n-npml+1..n and hand over at the slab edges.
+struct TfsfLine {
+  double *e, *h, *pe, *ph;
+  const double *f1, *f2, *g1, *g2;
+  int32_t n, npml, src, lo, hi, comp, hc, axis, sg;
+  double ck, ku;
+};
+
+// one workgroup: the line's E half step and its PML
+__device__ __forceinline__ void tfsf_line_e(const TfsfLine& L, double g) {
+  const int N = L.n, P = L.npml, hi = N - P + 1;
+  for (int j = P + 1 + (int)threadIdx.x; j <= hi - 1; j += blockDim.x) {
+    double v = L.e[j] + L.ck * (L.h[j] - L.h[j - 1]);
+    if (j == L.src) v = v + g;
+    L.e[j] = v;
+  }
+  if (P > 0) {
+    for (int j = 1 + (int)threadIdx.x; j <= P; j += blockDim.x)
+      L.pe[j] = L.f1[j] * L.pe[j] + L.f2[j] * (L.ph[j] - L.ph[j - 1]);
+    for (int j = hi + (int)threadIdx.x; j <= N; j += blockDim.x)
+      L.pe[j] = L.f1[j] * L.pe[j] + L.f2[j] * (L.ph[j] - L.ph[j - 1]);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      L.pe[P + 1] = L.e[P + 1];
+      L.e[P] = L.pe[P];
+      L.pe[hi - 1] = L.e[hi - 1];
+      L.e[hi] = L.pe[hi];
+    }
+  }
+}
+
+// Two-kernel step, H half: monitors of this step (E), every cell; with one
+// TFSF the E half step of its incident line too (pt.line, the first block: the
+// E launch read the line's H, k_tfsf_h reads its E): as a launch of its own it
+// cost 4.8 us of the 85 us a step of 150 x 137 x 211 cells takes.
 template <typename real, int KZ>
 __global__ __launch_bounds__(256) void k_step_h(FieldArgs<real> a, PmlArgs<real> p, Parts pt, MonList<real> mon,
-                                                SegGrid gt) {
+                                                SegGrid gt, TfsfLine line, double line_g) {
   int b = (int)blockIdx.x;
+  if (b < pt.line) {
+    if (b == 0) tfsf_line_e(line, line_g);
+    return;
+  }
+  b -= pt.line;
   if (b < pt.mon) {
     mon_block(mon, a.px, a.pxy, b, [&](int c) -> const real* { return c < 3 ? a.e[c] : a.h[c - 3]; });
     return;
@@ -2155,18 +2199,6 @@ __global__ __launch_bounds__(256, 2) void k_dft_accum(const real* __restrict__ s
   }
 }
 
-// point probes, sim3/program.f90:445-451
-// ---------------------------------------------------------------------------
-// TFSF incident line (sim1/program.f90:217-262, mod1/BERpmly_ExHz_mod.f90).
-// One workgroup walks the line; the PML object's own fields pe, ph live on
-// cells 1..npml and n-npml+1..n and hand over at the slab edges.
-struct TfsfLine {
-  double *e, *h, *pe, *ph;
-  const double *f1, *f2, *g1, *g2;
-  int32_t n, npml, src, lo, hi, comp, hc, axis, sg;
-  double ck, ku;
-};
-
 inline TfsfLine tfsf_line(const Sim* s, const Tfsf& t) {
   TfsfLine L;
   const int64_t m = t.n + 2;
@@ -2194,27 +2226,7 @@ inline TfsfLine tfsf_line(const Sim* s, const Tfsf& t) {
 
 // E half step of the line: ex_inc update (:222-224), the pulse (:228-229),
 // mypmly_inc%updateE (:231; updateE_pmy_low/high + setboundaryEa/Eb)
-__global__ __launch_bounds__(256) void k_tfsf_line_e(TfsfLine L, double g) {
-  const int N = L.n, P = L.npml, hi = N - P + 1;
-  for (int j = P + 1 + (int)threadIdx.x; j <= hi - 1; j += blockDim.x) {
-    double v = L.e[j] + L.ck * (L.h[j] - L.h[j - 1]);
-    if (j == L.src) v = v + g;
-    L.e[j] = v;
-  }
-  if (P > 0) {
-    for (int j = 1 + (int)threadIdx.x; j <= P; j += blockDim.x)
-      L.pe[j] = L.f1[j] * L.pe[j] + L.f2[j] * (L.ph[j] - L.ph[j - 1]);
-    for (int j = hi + (int)threadIdx.x; j <= N; j += blockDim.x)
-      L.pe[j] = L.f1[j] * L.pe[j] + L.f2[j] * (L.ph[j] - L.ph[j - 1]);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      L.pe[P + 1] = L.e[P + 1];
-      L.e[P] = L.pe[P];
-      L.pe[hi - 1] = L.e[hi - 1];
-      L.e[hi] = L.pe[hi];
-    }
-  }
-}
+__global__ __launch_bounds__(256) void k_tfsf_line_e(TfsfLine L, double g) { tfsf_line_e(L, g); }
 
 // H half step of the TFSF: block 0 advances the line (hz_inc update :252-254,
 // mypmly_inc%updateH :255) and records its probes; the other blocks apply
@@ -2669,15 +2681,15 @@ int step_impl(Sim* s) {
   // TFSF lines: E half step after the main E stage (the D terms above read
   // h(lo-1) before this step's line H update); H half step, consistency
   // terms on H and the line probes after the main H stage
+  auto line_pulse = [&](const fdtd_pulse& pu) {
+    const double tt = (double)(n - 1) * s->dt;
+    return pu.amplitude * (std::exp(-0.5 * ((tt - pu.t0) / pu.st) * ((tt - pu.t0) / pu.st)) * std::sin(pu.w0 * tt));
+  };
   auto tfsf_e = [&](hipStream_t sq) {
     if (s->dry) return;
     for (const auto& t : s->tfsfs) {
-      const fdtd_pulse& pu = t.p.pulse;
-      const double tt = (double)(n - 1) * s->dt;
-      const double g = pu.amplitude * (std::exp(-0.5 * ((tt - pu.t0) / pu.st) * ((tt - pu.t0) / pu.st)) *
-                                       std::sin(pu.w0 * tt));
       Timer tm(s, FDTD_K_MAT);
-      hipLaunchKernelGGL(k_tfsf_line_e, dim3(1), dim3(256), 0, sq, tfsf_line(s, t), g);
+      hipLaunchKernelGGL(k_tfsf_line_e, dim3(1), dim3(256), 0, sq, tfsf_line(s, t), line_pulse(t.p.pulse));
     }
   };
   auto tfsf_h = [&](hipStream_t sq, PmlArgs<real> pa, int all_faces) {
@@ -2949,15 +2961,19 @@ int step_impl(Sim* s) {
         hipLaunchKernelGGL((k_lord<real, true>), dim3((unsigned)((g.ncells + 255) / 256)), dim3(256), 0, st, a,
                            lord_coef(g), g.d_cells, g.d_mask, (double*)g.d_state, g.ncells, src, nsrc);
     }
-    tfsf_e(st);
+    const bool with_line = !apart && !s->dry && s->tfsfs.size() == 1;
+    if (!with_line) tfsf_e(st);
     {
       const MonList<real> mon = e_samples();
       Parts pt{};
       pt.mon = round8(mon.nblk);
+      pt.line = with_line ? 8 : 0;  // a whole round of blocks over the XCDs
+      const TfsfLine line = with_line ? tfsf_line(s, s->tfsfs[0]) : TfsfLine{};
+      const double line_g = with_line ? line_pulse(s->tfsfs[0].p.pulse) : 0.0;
       Timer tm(s, FDTD_K_H);
       by_zm([&](auto kz) {
-        hipLaunchKernelGGL((k_step_h<real, decltype(kz)::value>), dim3((unsigned)(pt.mon + tiles)), dim3(256), 0, st,
-                           a, p, pt, mon, gt);
+        hipLaunchKernelGGL((k_step_h<real, decltype(kz)::value>), dim3((unsigned)(pt.line + pt.mon + tiles)), dim3(256),
+                           0, st, a, p, pt, mon, gt, line, line_g);
       });
     }
     tfsf_h(st, p, 1);

@@ -229,3 +229,19 @@ def test_packed_field_reads(n, precision):
         sim.set_field(c, f)
         assert np.array_equal(sim.field(c), f), c
     sim.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("zm", ["1", "4"])
+def test_incident_line_beside_the_h_half(zm, precision, monkeypatch):
+    """The incident line's E half step as a block of the H launch (one TFSF)
+    and as a launch of its own (profiling): the same bits, line included."""
+    from test_gpu_tfsf import _tfsf_through_pml
+
+    monkeypatch.setenv("FDTD_ONEPASS", "0")
+    monkeypatch.setenv("FDTD_ZMARCH", zm)
+    spec = dict(_tfsf_through_pml(nsteps=150), dft=[])
+    a, ia, pa = _run(spec, precision, (1, 85, 64))
+    b, ib, pb = _run(spec, precision, (1, 85, 64), profiling=True)
+    assert np.abs(a.field(0)).max() > 0 or np.abs(a.field(2)).max() > 0
+    _same(a, ia, pa, b, ib, pb, spec)
