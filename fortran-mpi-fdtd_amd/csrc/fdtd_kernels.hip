@@ -1638,9 +1638,11 @@ __device__ __forceinline__ void staged_e_cell(const FieldArgs<real>& a, const Sr
   }
 }
 
-// updateH, sim3/include/myfdtd_func.f90:45-64, of one main-row cell
+// updateH, sim3/include/myfdtd_func.f90:45-64, of one main-row cell; the row
+// below the upper slab is copied into the slab's ghost row (ref_pml_e_cell).
 template <typename real>
-__device__ __forceinline__ void staged_h_cell(const FieldArgs<real>& a, int i, int j, int k) {
+__device__ __forceinline__ void staged_h_cell(const FieldArgs<real>& a, const RefPmlArgs<real>& p,
+                                              const StagedRows& rows, int i, int j, int k) {
   const int c = i + a.px * j + a.pxy * k;
   const real ex = a.e[0][c], ey = a.e[1][c], ez = a.e[2][c];
   const real curleyz = a.e[1][c + a.pxy] - ey;
@@ -1658,16 +1660,24 @@ __device__ __forceinline__ void staged_h_cell(const FieldArgs<real>& a, int i, i
   put_h_ghost(a.h[0], hx, i, j, k, c, a);
   put_h_ghost(a.h[1], hy, i, j, k, c, a);
   put_h_ghost(a.h[2], hz, i, j, k, c, a);
+  if (j + 1 == rows.jb) {
+    const int64_t o = i + p.sxy * k;  // slab row 0
+    p.s[1][S_HXY][o] = hx;
+    p.s[1][S_HZY][o] = hz;
+  }
 }
 
 // Reference y-slab PML, E: updateEs (mod3/BERpmly_mod.f90:117-159) driven by
 // split H only, then setboundayEya/Eyb (:200-225,255-278).  Slab 0 holds
 // rows 0..P+1, slab 1 rows jb-1..ny+1; split ghosts stay zero.  The module
 // copies the main fields of the row beyond a slab's inner one into the
-// slab's ghost row (E and H of rows P+1 and jb-1); the only reads of those
-// copies are E of row P+1 in the H update of row P and H of row jb-1 in the E
-// update of row jb, which take the main fields here, so that the slab's
-// cells need nothing another workgroup of the launch writes.
+// slab's ghost row (E and H of rows P+1 and jb-1).  Two of the copies are
+// read.  H of row jb-1, in the next step's E update of row jb: it is the row
+// as updateH left it, whatever the TFSF terms or the caller add to H after
+// that, so the thread that updates the row keeps the copy (staged_h_cell;
+// the slab's H cells, beside it in the launch, do not read it).  E of row
+// P+1, in the H update of row P of the same step: nothing writes it in
+// between, and the H update takes the main field.
 template <typename real>
 __device__ __forceinline__ void ref_pml_e_cell(const FieldArgs<real>& a, const RefPmlArgs<real>& p, int i, int jr,
                                                int k) {
@@ -1680,9 +1690,8 @@ __device__ __forceinline__ void ref_pml_e_cell(const FieldArgs<real>& a, const R
   const int64_t o = i + p.sx * jl + p.sxy * k;
   const int64_t ojm = o - p.sx, okm = o - p.sxy, oim = o - 1;
   const int c = i + a.px * j + a.pxy * k;
-  const bool edge = sl == 1 && j == p.jb;  // the row below is the main one jb-1
   const real curlHzy_p = S[S_HZX][o] + S[S_HZY][o];
-  const real curlHzy_m = edge ? -a.h[2][c - a.px] : -S[S_HZX][ojm] - S[S_HZY][ojm];
+  const real curlHzy_m = -S[S_HZX][ojm] - S[S_HZY][ojm];
   const real curlHyz_p = -S[S_HYZ][o] - S[S_HYX][o];
   const real curlHyz_m = S[S_HYZ][okm] + S[S_HYX][okm];
   const real curlHxz_p = S[S_HXY][o] + S[S_HXZ][o];
@@ -1692,7 +1701,7 @@ __device__ __forceinline__ void ref_pml_e_cell(const FieldArgs<real>& a, const R
   const real curlHyx_p = S[S_HYZ][o] + S[S_HYX][o];
   const real curlHyx_m = -S[S_HYZ][oim] - S[S_HYX][oim];
   const real curlHxy_p = -S[S_HXY][o] - S[S_HXZ][o];
-  const real curlHxy_m = edge ? a.h[0][c - a.px] : S[S_HXY][ojm] + S[S_HXZ][ojm];
+  const real curlHxy_m = S[S_HXY][ojm] + S[S_HXZ][ojm];
   const real f1x = pr[0 * ps + i], f2x = pr[1 * ps + i];
   const real f1y = pr[2 * ps + j], f2y = pr[3 * ps + j];
   const real f1z = pr[4 * ps + k], f2z = pr[5 * ps + k];
@@ -2051,7 +2060,7 @@ __global__ __launch_bounds__(256) void k_staged_h(FieldArgs<real> a, RefPmlArgs<
   }
   if (!seg_of(gt, b - pt.mix, a.xcdmap, tx, r)) return;
   const int i = tx * 64 + ((int)threadIdx.x & 63) + 1, kz = fast_quot(gt.ny, r);
-  if (i <= a.nx) staged_h_cell(a, i, r - kz * gt.ny.d + rows.j0, kz + 1);
+  if (i <= a.nx) staged_h_cell(a, rp, rows, i, r - kz * gt.ny.d + rows.j0, kz + 1);
 }
 
 // x-face tiles of 4 rows (FDTD_XFACE_BY=4)
