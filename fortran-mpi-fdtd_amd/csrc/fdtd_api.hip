@@ -73,8 +73,11 @@ void dev_free(Sim* s, void* p) {
 
 double* reduction_buffer(Sim* s, size_t bytes) {
   if (s->red_cap < bytes) {
-    s->d_red = (double*)dev_alloc(s, bytes);
-    s->red_cap = s->d_red ? bytes : 0;
+    double* p = (double*)dev_alloc(s, bytes);
+    if (!p) return nullptr;  // the smaller buffer stays
+    if (s->d_red) dev_free(s, s->d_red);
+    s->d_red = p;
+    s->red_cap = bytes;
   }
   return s->d_red;
 }
@@ -1039,15 +1042,26 @@ int read_back(Sim* s, std::vector<ReadPart> parts) {
 
 // The interior of a field as FP64 without ghosts, x fastest: packed on the
 // device (launch_pack) into planes of a buffer of at most kPackBytes, which
-// go to the caller as they are.  Without that buffer (no memory) the ghosted
-// array is copied and converted here, one thread and three passes over new
-// pages: 48^3 FP64 0.60 ms a read so, 0.40 packed; 96^3 FP64 0.88 and 0.42;
-// 256^3 FP32 27 and 4.7.
+// go to the caller as they are.  The buffer is there for the read alone:
+// kept by the handle it would be memory that its admission to a pool did not
+// count (keeping it saves 0.01-0.04 ms a read, 0.3 at 256^3).  Without it (no
+// memory) the ghosted array is copied and converted here, one thread and
+// three passes over new pages: 48^3 FP64 0.53-0.60 ms a read so, 0.41 packed;
+// 96^3 FP64 0.87 and 0.44; 256^3 FP32 27 and 5.0.
 template <typename real>
 int read_field(Sim* s, void* src, double* dst) {
   const size_t plane = (size_t)s->nx * s->ny;
   const int per = (int)std::min<size_t>((size_t)s->nz, std::max<size_t>(1, kPackBytes / (plane * sizeof(double))));
-  if (double* pk = reduction_buffer(s, plane * sizeof(double) * (size_t)per)) {
+  struct Buffer {
+    hipStream_t stream;
+    void* p = nullptr;
+    ~Buffer() {
+      if (p) (void)hipFreeAsync(p, stream);
+    }
+  } buf{s->stream};
+  FDTD_HIP(hipSetDevice(s->device));
+  if (hipMallocAsync(&buf.p, plane * sizeof(double) * (size_t)per, s->stream) == hipSuccess) {
+    double* pk = (double*)buf.p;
     for (int k = 1; k <= s->nz; k += per) {
       const int n = std::min(per, s->nz - k + 1);
       int rc = launch_pack(s, src, k, n, pk);
@@ -1056,6 +1070,7 @@ int read_field(Sim* s, void* src, double* dst) {
     }
     return 0;
   }
+  buf.p = nullptr;
   (void)hipGetLastError();
   std::vector<real> h((size_t)s->ncell_alloc);
   int rc = read_back(s, {{h.data(), src, h.size() * sizeof(real)}});

@@ -245,3 +245,29 @@ def test_incident_line_beside_the_h_half(zm, precision, monkeypatch):
     b, ib, pb = _run(spec, precision, (1, 85, 64), profiling=True)
     assert np.abs(a.field(0)).max() > 0 or np.abs(a.field(2)).max() > 0
     _same(a, ia, pa, b, ib, pb, spec)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_reads_leave_the_device_memory_as_it_was(precision):
+    """A field read takes no device memory beyond its own time; the buffer of
+    the energy and flux sums is replaced where a larger one is needed, so the
+    handle holds the larger one alone."""
+    import fdtd_amd
+    from fdtd_amd import workloads
+
+    spec = workloads.c1_gold_sphere(nsteps=8, n=32)
+    om = list(workloads.wavelength_frequencies(400e-9, 900e-9, 4096))
+    spec["dft"] = [dict(spec["dft"][0], omega=om)]
+    sim, ids, _ = fdtd_amd.make_simulation(spec, precision=precision, engine="fused")
+    sim.step(4)
+    m0 = sim.memory_bytes()
+    f = [sim.field(c) for c in range(6)]
+    assert sim.memory_bytes() == m0
+    we = sim.energy()
+    m1 = sim.memory_bytes()
+    flux = sim.flux(ids[0])
+    assert sim.memory_bytes() - m0 == 8 * 4096 and m1 - m0 <= 8 * 4096
+    assert sim.energy() == we and np.array_equal(sim.flux(ids[0]), flux)
+    assert all(np.array_equal(sim.field(c), f[c]) for c in range(6))
+    assert sim.memory_bytes() - m0 == 8 * 4096
+    sim.close()
