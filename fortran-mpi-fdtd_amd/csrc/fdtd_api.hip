@@ -538,6 +538,8 @@ int commit_impl(Sim* s) {
 
   // FDTD_XCD_MAP=0: blocks in launch order, not dealt to the XCDs
   if (const char* e = std::getenv("FDTD_XCD_MAP")) s->xcdmap = std::atoi(e) != 0;
+  // FDTD_DFT_FUSE=0: monitors in launches of their own
+  if (const char* e = std::getenv("FDTD_DFT_FUSE")) s->dft_fuse = std::atoi(e) != 0;
   // layout: rows are whole 128-byte lines and the first interior cell of
   // every row starts a line (the field pointer is offset by line-1 cells
   // inside its allocation), so each wavefront's 64 cells span the fewest lines

@@ -267,6 +267,9 @@ struct Sim {
   // two-kernel step: E and H tiles span zm planes (1, 2, 4 or 8), each
   // thread marching its column and carrying the neighbour plane in registers
   int zm = 1;
+  // FDTD_DFT_FUSE=0: each step's monitors are sampled by a launch at its end
+  // instead of beside the launches that follow the fields (the same bits)
+  bool dft_fuse = true;
   // monitors of the last step made that are still to be sampled (at the
   // latest at the end of the fdtd_step call), and its probes: 1 the time and
   // E, 2 H, 3 all of a record at probe_out

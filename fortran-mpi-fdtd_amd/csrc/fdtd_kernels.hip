@@ -2749,13 +2749,14 @@ int step_impl(Sim* s) {
       s->probe_tn = (double)n * s->dt;
     }
   };
-  // profiling: every part a launch of its own, timed
-  const bool apart = s->profiling;
+  // profiling: every part a launch of its own, timed; FDTD_DFT_FUSE=0: the
+  // monitors alone
+  const bool apart = s->profiling, mon_apart = apart || !s->dft_fuse;
   // in the H launch E is final and H is not: it samples E, the next step's
   // first launch H
   auto e_samples = [&]() {
     MonList<real> mon{};
-    if (apart) return mon;
+    if (mon_apart) return mon;
     sample(7, [&](const MonPend& q) {
       if (mon.nplanes == kMonPlanes) {
         launch_monitors(s, mon);
@@ -2986,7 +2987,7 @@ int step_impl(Sim* s) {
       });
     }
     tfsf_h(st, p, 1);
-    apart ? pend(63, 3) : pend(56, 2);
+    mon_apart ? pend(63, 3) : pend(56, 2);
   } else {
     RefPmlArgs<real> rp{};
     if (refy) rp = ref_pml_args<real>(s);
@@ -3063,9 +3064,9 @@ int step_impl(Sim* s) {
       }
     }
     tfsf_h(st, PmlArgs<real>{}, 0);
-    apart ? pend(63, 3) : pend(56, 2);
+    mon_apart ? pend(63, 3) : pend(56, 2);
   }
-  if (apart) flush_pending<real>(s);
+  if (mon_apart) flush_pending<real>(s);
   // dry steps (the autotuner's) sample into the ring slot the next real step
   // overwrites, so each step form is timed with its sampling cost, and
   // neither advance the ring, fold nor record probes

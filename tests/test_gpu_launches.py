@@ -271,3 +271,33 @@ def test_reads_leave_the_device_memory_as_it_was(precision):
     assert all(np.array_equal(sim.field(c), f[c]) for c in range(6))
     assert sim.memory_bytes() - m0 == 8 * 4096
     sim.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("form", [{"FDTD_ONEPASS": "0"}, {"FDTD_ONEPASS": "1", "FDTD_ONEPASS_BY": "2"}, "staged"])
+def test_samples_beside_the_launches_and_alone(form, precision, monkeypatch):
+    """Eleven planes and four probes sampled beside the step's launches, in
+    calls that end before, at and behind a DFT block: the same bits as
+    sampled by a launch at each step's end (FDTD_DFT_FUSE=0), and as with
+    every part in a launch of its own (profiling)."""
+    import fdtd_amd
+
+    spec = _spec(groups=2)
+    if form == "staged":
+        spec["pml"].update(mode="ref_y", npml=[0, 5, 0])
+    else:
+        for k, v in form.items():
+            monkeypatch.setenv(k, v)
+    runs = []
+    for fuse, prof in (("1", False), ("0", False), ("1", True)):
+        monkeypatch.setenv("FDTD_DFT_FUSE", fuse)
+        sim, ids, pids = fdtd_amd.make_simulation(spec, precision=precision)
+        sim.set_profiling(prof)
+        for n in (1, 62, 1, 1, 64, 2):
+            sim.step(n)
+        runs.append((sim, ids, pids))
+    for r in runs[1:]:
+        _same(*runs[0], *r, spec)
+    assert all(np.abs(runs[0][0].dft(i, d["comps"][-1])[0]).max() > 0 for i, d in zip(runs[0][1], spec["dft"]))
+    for r in runs:
+        r[0].close()
