@@ -138,8 +138,9 @@ struct Inst {
   int32_t probe_c[kMaxProbe];  // ghosted cell offsets
   double* probe_rec;           // [n-1][probe][3]
   int32_t probe_cap;           // steps the buffer holds
-  // rows with a DFT line or a probe
-  int32_t nmon, mon_row[kMaxDft + kMaxProbe];
+  // rows with a DFT line or a probe, and which (bits: the lines, then the
+  // probes)
+  int32_t nmon, mon_row[kMaxDft + kMaxProbe], mon_sel[kMaxDft + kMaxProbe];
   // TMz: fields, Ez splits (PML cells only), profiles f1 f2 g1 g2 [nx+2]
   // along x then [ny+2] along y, PML depths Px (x) and P (y, above)
   int32_t tmz, Px;
@@ -550,7 +551,7 @@ __device__ __forceinline__ int xcd_block(int b) {
 
 // ---- plain row strips ------------------------------------------------------------
 // A wavefront's kRowsPerWave rows are "plain" when none is a PML, source
-// (E), monitor (H) or TFSF row and (TMz) none of its lanes lies in an x slab: the cell update is
+// (E) or TFSF row and (TMz) none of its lanes lies in an x slab: the cell update is
 // then the interior one of e_tez / h_tez / e_tmz / h_tmz, and the loads of
 // all rows are issued before the first row's stores (one memory round trip
 // for the strip instead of one per row).  The arithmetic is the same,
@@ -578,29 +579,28 @@ __device__ __forceinline__ bool strip_plain(const Inst<real>& S, int i0, int j0,
     if (a >= j0 && a <= j1) return false;
     if (S.tf_hi > 0 && b >= j0 && b <= j1) return false;
   }
-  if (e_half) {
+  if (e_half)
     for (int j = j0; j <= j1; ++j)
       if (src_row(S, j)) return false;
-  } else {
-    for (int m = 0; m < S.nmon; ++m)
-      if (S.mon_row[m] >= j0 && S.mon_row[m] <= j1) return false;
-  }
   return true;
 }
 
-// Monitors of cell (i, j) after step n, block slot b: the DFT lines' samples
-// of the row (sample step recorded by the row's first cell, 0 when the
-// line's gate is closed) and the probes at the cell.  Called by the thread
-// that has just written the cell's H, so it reads E and H as the step left
-// them.
+// Monitors `sel` of cell (i, j) after step n, block slot b: the DFT lines'
+// samples of the row (sample step recorded by the row's first cell, 0 when
+// the line's gate is closed) and the probes at the cell.  Called by the
+// thread that has just written the cell's H, so it reads E and H as the step
+// left them.  `sel` names the row's own: every line and probe asked in turn
+// is a chain of scalar loads each, on rows that were left out of the strips
+// besides: a batch of 8 x 1024^2 FP32 with four lines and eight probes each
+// took 73.1 us a step so, 71.7 with the monitors in a launch of their own, 65.5
+// now (61.0 without monitors).
 template <typename real>
-__device__ __forceinline__ void mon_cell(const Inst<real>& S, int i, int j, int n, int b) {
+__device__ __forceinline__ void mon_cell(const Inst<real>& S, int i, int j, uint32_t sel, int n, int b) {
   const int c = i + S.px * j;
   const real e = (S.tmz ? S.ez : S.ex)[c], h = (S.tmz ? S.hx : S.hz)[c];
   const int e_bit = S.tmz ? FDTD2D_DFT_EZ : FDTD2D_DFT_EX, h_bit = S.tmz ? FDTD2D_DFT_HX : FDTD2D_DFT_HZ;
-  for (int l = 0; l < S.ndft; ++l) {
-    const DftDev& D = S.dft[l];
-    if (D.j != j) continue;
+  for (uint32_t q = sel & ((1u << kMaxDft) - 1); q; q &= q - 1) {
+    const DftDev& D = S.dft[__builtin_ctz(q)];
     const bool open = n >= D.n_begin && (D.n_end <= 0 || n <= D.n_end);
     if (i == 1) D.sstep[b] = open ? n : 0;
     if (!open) continue;
@@ -612,13 +612,15 @@ __device__ __forceinline__ void mon_cell(const Inst<real>& S, int i, int j, int 
     if (D.mask & h_bit) *samp = h;
   }
   // probes: (n*dt, Ex, Hz), sim2/program.f90:376,397,417; TMz (n*dt, Ez, Hx)
-  for (int p = 0; p < S.nprobe; ++p)
+  for (uint32_t q = sel >> kMaxDft; q; q &= q - 1) {
+    const int p = __builtin_ctz(q);
     if (S.probe_c[p] == c && n - 1 < S.probe_cap) {
       double* r = S.probe_rec + ((int64_t)(n - 1) * S.nprobe + p) * 3;
       r[0] = (double)n * S.dt;
       r[1] = (double)e;
       r[2] = (double)h;
     }
+  }
 }
 
 // D of a strip, which nothing else of the step reads; NT: nontemporal (k2_e)
@@ -922,19 +924,20 @@ __global__ __launch_bounds__(kTX * kWaves) void k2_h(const Inst<real>* __restric
         h_tmz_strip(S, i, j0);
       else
         h_tez_strip(S, i, j0);
-      continue;
+    } else {
+      real carry = 0;
+      for (int r = 0; r < kRowsPerWave; ++r) {
+        const int j = j0 + r;
+        if (j > S.ny) break;
+        if (S.tmz)
+          h_tmz(S, i, j, carry, r > 0);
+        else
+          h_tez(S, i, j, carry, r > 0);
+      }
     }
-    real carry = 0;
-    for (int r = 0; r < kRowsPerWave; ++r) {
-      const int j = j0 + r;
-      if (j > S.ny) break;
-      if (S.tmz)
-        h_tmz(S, i, j, carry, r > 0);
-      else
-        h_tez(S, i, j, carry, r > 0);
-      bool mon = false;
-      for (int m = 0; m < S.nmon; ++m) mon |= S.mon_row[m] == j;
-      if (mon) mon_cell(S, i, j, n, st);
+    for (int m = 0; m < S.nmon; ++m) {
+      const int j = S.mon_row[m];
+      if (j >= j0 && j < j0 + kRowsPerWave) mon_cell(S, i, j, (uint32_t)S.mon_sel[m], n, st);
     }
   }
 }
@@ -1772,7 +1775,12 @@ Inst<real> make_inst(Sim* s, int tile0) {
     std::sort(rows.begin(), rows.end());
     rows.erase(std::unique(rows.begin(), rows.end()), rows.end());
     d.nmon = (int32_t)rows.size();
-    std::copy(rows.begin(), rows.end(), d.mon_row);
+    for (int m = 0; m < d.nmon; ++m) {
+      d.mon_row[m] = rows[(size_t)m];
+      for (size_t l = 0; l < s->dfts.size(); ++l) d.mon_sel[m] |= (s->dfts[l].j == d.mon_row[m]) << l;
+      for (size_t q = 0; q < s->probes.size(); ++q)
+        d.mon_sel[m] |= (s->probes[q].second == d.mon_row[m]) << (kMaxDft + q);
+    }
   }
   if (s->has_tf) {
     d.tf_on = 1;

@@ -115,3 +115,49 @@ def test_marked_d(polarization, precision, monkeypatch):
     assert np.any(got[0][0] != 0)
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("polarization", ["tez", "tmz"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_monitors_of_one_strip(polarization, precision):
+    """Four lines and eight probes on the rows of one wavefront strip (21-24
+    of interior cells), the rows beside it and a row alone, lines of both
+    components, of E and of H alone, with a gate: simulations in a batch and
+    alone give the same bits, and hold the oracle's samples."""
+    import oracle
+    from fdtd_amd import sim2d
+
+    tm = polarization == "tmz"
+    spec = sim2d.sweep_instance(np.random.default_rng(3), side=96, nsteps=80, npml=8, polarization=polarization)
+    spec["grid"]["nx"] = 150
+    spec["materials"] = spec["materials"][:1]
+    spec["sources"][0]["j"] = 18
+    om = spec["dft"][0]["omega"][:9]
+    e, h = (sim2d.DFT_EZ, sim2d.DFT_HX) if tm else (sim2d.DFT_EX, sim2d.DFT_HZ)
+    spec["dft"] = [{"j": 21, "omega": om}, {"j": 22, "omega": om, "mask": e, "n_begin": 20, "n_end": 70},
+                   {"j": 24, "omega": om, "mask": h}, {"j": 21, "omega": om, "mask": e | h, "n_begin": 33}]
+    spec["probes"] = [[1, 21], [64, 22], [65, 23], [150, 24], [128, 24], [129, 20], [5, 25], [70, 60]]
+    other = dict(spec, dft=spec["dft"][:1], probes=[])
+    sims = [sim2d.make_simulation2d(s, precision=precision) for s in (spec, other, spec)]
+    alone = sim2d.make_simulation2d(spec, precision=precision)
+    batch = sim2d.Batch2D([s[0] for s in sims])
+    ref = oracle.make_simulation2d(spec)
+    for n in (1, 32, 47):
+        batch.run([n, n // 2, n])
+        alone[0].step(n)
+        ref[0].step(n)
+    batch.sync()
+    tol = 1e-12 if precision == "fp64" else 1e-4
+    for x, y, z, d in zip(sims[0][1], alone[1], ref[1], spec["dft"]):
+        for c in [(sim2d.EZ2 if tm else sim2d.EX2)] * bool(d.get("mask", e) & e) + \
+                 [(sim2d.HX2 if tm else sim2d.HZ2)] * bool(d.get("mask", h) & h):
+            for u, v, w, o in zip(sims[0][0].dft(x, c), sims[2][0].dft(x, c), alone[0].dft(y, c), ref[0].dft(z, c)):
+                assert np.array_equal(u, v) and np.array_equal(u, w)
+                check(f"strip dft {polarization} {precision} {c}", relerr(u, o), tol)
+    for x, y, z in zip(sims[0][2], alone[2], ref[2]):
+        u = sims[0][0].probe(x)
+        assert np.array_equal(u, sims[2][0].probe(x)) and np.array_equal(u, alone[0].probe(y))
+        check(f"strip probe {polarization} {precision}", relerr(u, ref[0].probe(z)), tol)
+    batch.close()
+    for s in (*sims, alone, ref):
+        s[0].close()
