@@ -1046,10 +1046,12 @@ int read_back(Sim* s, std::vector<ReadPart> parts) {
 // device (launch_pack) into planes of a buffer of at most kPackBytes, which
 // go to the caller as they are.  The buffer is there for the read alone:
 // kept by the handle it would be memory that its admission to a pool did not
-// count (keeping it saves 0.01-0.04 ms a read, 0.3 at 256^3).  Without it (no
-// memory) the ghosted array is copied and converted here, one thread and
-// three passes over new pages: 48^3 FP64 0.53-0.60 ms a read so, 0.41 packed;
-// 96^3 FP64 0.87 and 0.44; 256^3 FP32 27 and 5.0.
+// count.  Small fields (kPackFrom), and any without that memory, are copied
+// as they lie and converted here.  us a read into touched pages, converted
+// here against packed: FP64 40^3 51 : 60, 48^3 137 : 77, 64^3 245 : 160, 96^3
+// 790 : 435; FP32, of which the link then carries half the bytes, 48^3 52 : 75,
+// 64^3 160 : 165, 256 x 256 x 8 250 : 280, 80^3 248 : 265, 96^3 455 : 435; new
+// pages, 96^3 FP64 2050 : 810, FP32 600 : 450; 256^3 FP32 27,000 : 5,000.
 template <typename real>
 int read_field(Sim* s, void* src, double* dst) {
   const size_t plane = (size_t)s->nx * s->ny;
@@ -1062,7 +1064,8 @@ int read_field(Sim* s, void* src, double* dst) {
     }
   } buf{s->stream};
   FDTD_HIP(hipSetDevice(s->device));
-  if (hipMallocAsync(&buf.p, plane * sizeof(double) * (size_t)per, s->stream) == hipSuccess) {
+  if (plane * s->nz * sizeof(double) >= kPackFrom[sizeof(real) == 4] &&
+      hipMallocAsync(&buf.p, plane * sizeof(double) * (size_t)per, s->stream) == hipSuccess) {
     double* pk = (double*)buf.p;
     for (int k = 1; k <= s->nz; k += per) {
       const int n = std::min(per, s->nz - k + 1);

@@ -126,7 +126,9 @@ constexpr size_t kReadRingFrom = (size_t)16 << 20;
 constexpr int kReadThreads = 4;
 constexpr size_t kReadSlot = (size_t)2 << 20;
 constexpr int kReadRings = 4;
-// Device buffer of a packed field read (at least one plane; read_field).
+// Packed field reads: from how many result bytes (FP64, FP32 fields) and
+// the device buffer (at least one plane; read_field).
+constexpr size_t kPackFrom[2] = {(size_t)768 << 10, (size_t)6 << 20};
 constexpr size_t kPackBytes = (size_t)32 << 20;
 
 // Planes a general workgroup of the one-pass step marches through (at most).

@@ -301,3 +301,19 @@ def test_samples_beside_the_launches_and_alone(form, precision, monkeypatch):
     assert all(np.abs(runs[0][0].dft(i, d["comps"][-1])[0]).max() > 0 for i, d in zip(runs[0][1], spec["dft"]))
     for r in runs:
         r[0].close()
+
+
+@pytest.mark.parametrize("precision,n", [("fp64", (256, 128, 3)), ("fp64", (255, 128, 3)), ("fp32", (256, 512, 6)),
+                                         ("fp32", (257, 511, 6))])
+def test_field_reads_at_the_packing_line(precision, n):
+    """Fields of 768 KiB (FP64) and 6 MiB (FP32) of results, from which on
+    they are packed on the device, and just below: the field set, and the
+    device memory as it was."""
+    import fdtd_amd
+
+    sim = fdtd_amd.Simulation(*n, 1e-9, 0.5, precision=precision, engine="fused")
+    f = np.random.default_rng(n[0]).standard_normal(n).astype(np.float32).astype(np.float64)
+    sim.set_field(2, f)
+    m = sim.memory_bytes()
+    assert np.array_equal(sim.field(2), f) and sim.memory_bytes() == m
+    sim.close()
