@@ -71,10 +71,6 @@ template <typename real>
 __device__ __forceinline__ real ld_at(const real* p, uint32_t off) {
   return *(const real*)((const char*)p + off);
 }
-template <typename real>
-__device__ __forceinline__ void st_at(real* p, uint32_t off, real v) {
-  *(real*)((char*)p + off) = v;
-}
 // NT: a nontemporal store (streams_past_llc)
 template <bool NT, typename real>
 __device__ __forceinline__ void put(real* p, real v) {
@@ -476,14 +472,16 @@ __device__ __forceinline__ void e_mixed_block(const FieldArgs<real>& a, const Pm
 // ---------------------------------------------------------------------------
 // FUSED engine: H half step (myfdtd_func.f90:45-64 + split-field H) of one
 // cell, as the E step in a load phase (h_cell_load) and an arithmetic and
-// store phase (h_cell_store).  z march: with use_carry, Ex and Ey of plane
+// store phase (h_cell_store), with 64-bit lane addresses: from row addresses
+// and 32-bit offsets, as the march does, two-kernel H takes 175 against 165 us
+// at 203^3 FP64, 79.9 against 79.2 in FP32, and k_gen_h 251 against 246 us at
+// 320^3 FP64, 82.8 against 77.9 in FP32.  z march: with use_carry, Ex and Ey of plane
 // k come from cex, cey (loaded as plane k+1 by the previous plane of the
 // same thread).  In place HO* are H* and pw is p; over two copies the old
 // H and splits come from HO* and p, the new ones go to H* and pw.
 template <typename real>
 struct HCellIn {
-  int c, rb, s;
-  uint32_t ib;
+  int c, s;
   bool pml, sx, sy, sz;
   real ex, ey, ez, ey_kp, ex_kp, ez_jp, ex_jp, ez_ip, ey_ip;
   real h0[3], sp[6], gx1, gx2, gy1, gy2, gz1, gz2;
@@ -491,22 +489,17 @@ struct HCellIn {
 
 template <typename real, int FACE = 0>
 __device__ __forceinline__ void h_cell_load(const FieldArgs<real>& a, const PmlArgs<real>& p, int i, int j, int k,
-                                            int jb, bool use_carry, real cex, real cey, const real* E0, const real* E1,
+                                            bool use_carry, real cex, real cey, const real* E0, const real* E1,
                                             const real* E2, const real* HO0, const real* HO1, const real* HO2,
                                             HCellIn<real>& in) {
-  const int rb = a.px * jb + a.pxy * k, co = i + a.px * (j - jb), c = rb + co;
-  const uint32_t ib = (uint32_t)co * (uint32_t)sizeof(real), ip = ib + (uint32_t)sizeof(real);
-  // wave-uniform row addresses and the cell's 32-bit byte offset from them
-  // (the E update holds too many of them: 64-bit offsets are faster there)
+  const int c = i + a.px * j + a.pxy * k;
   in.c = c;
-  in.rb = rb;
-  in.ib = ib;
-  in.ex = use_carry ? cex : ld_at(E0 + rb, ib);
-  in.ey = use_carry ? cey : ld_at(E1 + rb, ib);
-  in.ez = ld_at(E2 + rb, ib);
-  in.ey_kp = ld_at(E1 + (rb + a.pxy), ib); in.ex_kp = ld_at(E0 + (rb + a.pxy), ib);
-  in.ez_jp = ld_at(E2 + (rb + a.px), ib); in.ex_jp = ld_at(E0 + (rb + a.px), ib);
-  in.ez_ip = ld_at(E2 + rb, ip); in.ey_ip = ld_at(E1 + rb, ip);
+  in.ex = use_carry ? cex : E0[c];
+  in.ey = use_carry ? cey : E1[c];
+  in.ez = E2[c];
+  in.ey_kp = E1[c + a.pxy]; in.ex_kp = E0[c + a.pxy];
+  in.ez_jp = E2[c + a.px]; in.ex_jp = E0[c + a.px];
+  in.ez_ip = E2[c + 1]; in.ey_ip = E1[c + 1];
   in.pml = FACE ? true : in_pml(p.P, i, j, k, a.nx, a.ny, a.nz);
   in.s = 0;
   in.sx = in.sy = in.sz = false;
@@ -538,11 +531,11 @@ __device__ __forceinline__ void h_cell_load(const FieldArgs<real>& a, const PmlA
     if (sx) { in.sp[0] = p.s[S_HYX][s]; in.sp[1] = p.s[S_HZX][s]; }
     if (sy) { in.sp[2] = p.s[S_HXY][s]; in.sp[3] = p.s[S_HZY][s]; }
     if (sz) { in.sp[4] = p.s[S_HXZ][s]; in.sp[5] = p.s[S_HYZ][s]; }
-    if (!(sy && sz)) in.h0[0] = ld_at(HO0 + rb, ib);
-    if (!(sz && sx)) in.h0[1] = ld_at(HO1 + rb, ib);
-    if (!(sx && sy)) in.h0[2] = ld_at(HO2 + rb, ib);
+    if (!(sy && sz)) in.h0[0] = HO0[c];
+    if (!(sz && sx)) in.h0[1] = HO1[c];
+    if (!(sx && sy)) in.h0[2] = HO2[c];
   } else {
-    in.h0[0] = ld_at(HO0 + rb, ib); in.h0[1] = ld_at(HO1 + rb, ib); in.h0[2] = ld_at(HO2 + rb, ib);
+    in.h0[0] = HO0[c]; in.h0[1] = HO1[c]; in.h0[2] = HO2[c];
   }
 }
 
@@ -565,9 +558,9 @@ __device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const Pml
     if (in.sy) { pw.s[S_HXY][s] = hxy; pw.s[S_HZY][s] = hzy; }
     if (in.sz) { pw.s[S_HXZ][s] = hxz; pw.s[S_HYZ][s] = hyz; }
     const real hx = hxy + hxz, hy = hyz + hyx, hz = hzx + hzy;
-    st_at(H0 + in.rb, in.ib, hx);
-    st_at(H1 + in.rb, in.ib, hy);
-    st_at(H2 + in.rb, in.ib, hz);
+    H0[c] = hx;
+    H1[c] = hy;
+    H2[c] = hz;
     put_h_ghost(H0, hx, i, j, k, c, a);
     put_h_ghost(H1, hy, i, j, k, c, a);
     put_h_ghost(H2, hz, i, j, k, c, a);
@@ -579,9 +572,9 @@ __device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const Pml
   const real hx = in.h0[0] + a.ku * (curleyz + curlezy);
   const real hy = in.h0[1] + a.ku * (curlezx + curlexz);
   const real hz = in.h0[2] + a.ku * (curlexy + curleyx);
-  st_at(H0 + in.rb, in.ib, hx);
-  st_at(H1 + in.rb, in.ib, hy);
-  st_at(H2 + in.rb, in.ib, hz);
+  H0[c] = hx;
+  H1[c] = hy;
+  H2[c] = hz;
   put_h_ghost(H0, hx, i, j, k, c, a);
   put_h_ghost(H1, hy, i, j, k, c, a);
   put_h_ghost(H2, hz, i, j, k, c, a);
@@ -589,11 +582,11 @@ __device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const Pml
 
 template <typename real>
 __device__ __forceinline__ void fused_h_cell(const FieldArgs<real>& a, const PmlArgs<real>& p,
-                                             const PmlArgs<real>& pw, int i, int j, int k, real& cex, real& cey, bool use_carry, const real* E0, const real* E1,
-                                             const real* E2, const real* HO0, const real* HO1, const real* HO2,
+                                             const PmlArgs<real>& pw, int i, int j, int k, real& cex, real& cey,
+                                             bool use_carry, const real* E0, const real* E1, const real* E2, const real* HO0, const real* HO1, const real* HO2,
                                              real* H0, real* H1, real* H2) {
   HCellIn<real> in;
-  h_cell_load(a, p, i, j, k, j, use_carry, cex, cey, E0, E1, E2, HO0, HO1, HO2, in);
+  h_cell_load(a, p, i, j, k, use_carry, cex, cey, E0, E1, E2, HO0, HO1, HO2, in);
   cex = in.ex_kp;
   cey = in.ey_kp;
   h_cell_store(a, pw, i, j, k, in, H0, H1, H2);
@@ -1210,7 +1203,7 @@ __device__ __forceinline__ void march_block(const FieldArgs<real>& a, const Marc
 // cell per thread; the E update marched so holds too many registers and
 // runs slower).
 template <typename real>
-__device__ __forceinline__ bool gen_cell(const FieldArgs<real>& a, const TileList& tl, int b, int& i, int& j, int& jb, int& k0,
+__device__ __forceinline__ bool gen_cell(const FieldArgs<real>& a, const TileList& tl, int b, int& i, int& j, int& k0,
                                          int& k1, bool& wide, int& pl, int& face) {
   int lb = deal(b, tl.tper, a.xcdmap);
   if (lb >= tl.n * tl.nsplit) return false;
@@ -1221,8 +1214,7 @@ __device__ __forceinline__ bool gen_cell(const FieldArgs<real>& a, const TileLis
   wide = bw == 64;
   const int t = (int)threadIdx.x;
   i = T[0] + (t & (bw - 1));
-  jb = T[2];
-  j = jb + (wide ? __builtin_amdgcn_readfirstlane(t >> 6) : t / bw);
+  j = T[2] + (wide ? __builtin_amdgcn_readfirstlane(t >> 6) : t / bw);
   k0 = T[4];
   k1 = T[6];
   face = T[7];
@@ -1234,9 +1226,9 @@ template <typename real>
 __device__ __forceinline__ void gen_e_block(const FieldArgs<real>& a, const PmlArgs<real>& p, const PmlArgs<real>& pw,
                                             const MarchArgs<real>& m, const TileList& tl, const SrcArgs<real>& src,
                                             int nsrc, int b) {
-  int i, j, jb, k0, k1, pl, face;
+  int i, j, k0, k1, pl, face;
   bool wide;
-  if (!gen_cell(a, tl, b, i, j, jb, k0, k1, wide, pl, face)) return;
+  if (!gen_cell(a, tl, b, i, j, k0, k1, wide, pl, face)) return;
   const int k = k0 + pl;
   if (k > k1) return;
   real sv[3] = {0, 0, 0};
@@ -1269,13 +1261,13 @@ __device__ __forceinline__ void gen_e_block(const FieldArgs<real>& a, const PmlA
 // one (i, j) column of planes k0..k1, pipelined by hand (see above)
 template <typename real, int FACE>
 __device__ __forceinline__ void gen_h_column(const FieldArgs<real>& a, const PmlArgs<real>& p, const PmlArgs<real>& pw,
-                                             const MarchArgs<real>& m, int i, int j, int jb, int k0, int k1) {
+                                             const MarchArgs<real>& m, int i, int j, int k0, int k1) {
   HCellIn<real> cur, nxt;
-  h_cell_load<real, FACE>(a, p, i, j, k0, jb, false, (real)0, (real)0, a.e[0], a.e[1], a.e[2], m.ho[0], m.ho[1],
+  h_cell_load<real, FACE>(a, p, i, j, k0, false, (real)0, (real)0, a.e[0], a.e[1], a.e[2], m.ho[0], m.ho[1],
                           m.ho[2], cur);
   for (int k = k0; k <= k1; ++k) {
     const int kn = min(k + 1, k1);
-    h_cell_load<real, FACE>(a, p, i, j, kn, jb, kn > k, cur.ex_kp, cur.ey_kp, a.e[0], a.e[1], a.e[2], m.ho[0],
+    h_cell_load<real, FACE>(a, p, i, j, kn, kn > k, cur.ex_kp, cur.ey_kp, a.e[0], a.e[1], a.e[2], m.ho[0],
                             m.ho[1], m.ho[2], nxt);
     h_cell_store(a, pw, i, j, k, cur, a.h[0], a.h[1], a.h[2]);
     cur = nxt;
@@ -1285,15 +1277,15 @@ __device__ __forceinline__ void gen_h_column(const FieldArgs<real>& a, const Pml
 template <typename real>
 __global__ __launch_bounds__(256) void k_gen_h(FieldArgs<real> a, PmlArgs<real> p, PmlArgs<real> pw,
                                                MarchArgs<real> m, TileList tl) {
-  int i, j, jb, k0, k1, pl, face;
+  int i, j, k0, k1, pl, face;
   bool wide;
-  if (!gen_cell(a, tl, (int)blockIdx.x, i, j, jb, k0, k1, wide, pl, face)) return;
+  if (!gen_cell(a, tl, (int)blockIdx.x, i, j, k0, k1, wide, pl, face)) return;
   if (face == 2)
-    gen_h_column<real, 2>(a, p, pw, m, i, j, jb, k0, k1);
+    gen_h_column<real, 2>(a, p, pw, m, i, j, k0, k1);
   else if (face == 1)
-    gen_h_column<real, 1>(a, p, pw, m, i, j, jb, k0, k1);
+    gen_h_column<real, 1>(a, p, pw, m, i, j, k0, k1);
   else
-    gen_h_column<real, 0>(a, p, pw, m, i, j, jb, k0, k1);
+    gen_h_column<real, 0>(a, p, pw, m, i, j, k0, k1);
 }
 
 // ---------------------------------------------------------------------------
