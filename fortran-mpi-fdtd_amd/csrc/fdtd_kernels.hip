@@ -2056,10 +2056,10 @@ __global__ __launch_bounds__(256) void k_staged_h(FieldArgs<real> a, RefPmlArgs<
 }
 
 // x-face tiles of 4 rows (FDTD_XFACE_BY=4)
-template <typename real, bool PER>
+template <typename real, bool PER, bool NT>
 __global__ __launch_bounds__(256) void k_xface4(FieldArgs<real> a, MarchArgs<real> m, SrcArgs<real> src, int nsrc,
                                                 TileList xf, XfArgs<real> x) {
-  march_block<real, 4, true, PER, false>(a, m, xf, src, nsrc, x, (int)blockIdx.x);
+  march_block<real, 4, true, PER, NT>(a, m, xf, src, nsrc, x, (int)blockIdx.x);
 }
 
 // cos/sin table of one block of samples: tab[(b*nfreq + m)*2 + {0,1}]
@@ -2863,7 +2863,10 @@ int step_impl(Sim* s) {
         auto go = [&](auto kern) {
           hipLaunchKernelGGL(kern, dim3((unsigned)all.xf), dim3(256), 0, st, an, m, src, nsrc, tx, xa);
         };
-        per ? go(k_xface4<real, true>) : go(k_xface4<real, false>);
+        if (s->nt_march)
+          per ? go(k_xface4<real, true, true>) : go(k_xface4<real, false, true>);
+        else
+          per ? go(k_xface4<real, true, false>) : go(k_xface4<real, false, false>);
       }
     };
     const bool xf4 = s->n_tl_xf && s->tl_bx == 4;

@@ -317,3 +317,15 @@ def test_field_reads_at_the_packing_line(precision, n):
     m = sim.memory_bytes()
     assert np.array_equal(sim.field(2), f) and sim.memory_bytes() == m
     sim.close()
+
+
+@pytest.mark.parametrize("bx", ["2", "4"])
+def test_marked_stores_of_the_x_face_tiles(bx, monkeypatch):
+    """The x-face tiles of 2 rows (in the march's launch) and of 4 (their
+    own), stores marked and not: the same bits."""
+    from test_gpu_onepass import _cases, _run as run, _same as same
+
+    spec = _cases()["x_edges"]
+    env = {"FDTD_ONEPASS": "1", "FDTD_ONEPASS_BY": "4", "FDTD_ONEPASS_KC": "16", "FDTD_XFACE_BY": bx}
+    got = [run(spec, "fp32", dict(env, FDTD_NT=nt), monkeypatch) for nt in "01"]
+    same(*got[0], *got[1])
