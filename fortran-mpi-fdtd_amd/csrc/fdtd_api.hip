@@ -483,7 +483,10 @@ bool onepass_fits(const Sim* s) { return (uint64_t)s->pxy * s->wsize < ((uint64_
 // FP64 320^3 1003 : 1031; STAGED FP64, 9 arrays (D, read and written): 100 x
 // 800 x 25 74 : 67, 110 x 1000 x 25 (208 MiB) 94 : 84, 125 x 1100 x 25 (261
 // MiB) 113 : 126, 125 x 1266 x 25 125 : 143.  Marked loads of the fields that
-// neighbouring tiles share lose everywhere.
+// neighbouring tiles share lose everywhere.  The rule sees one handle: jobs of
+// a pool beside each other have less of the cache each, but four of 67-203
+// cells a side take 71.7 ms a pass by the rule, 74.3 all unmarked and 69-72
+// all marked.
 bool streams_past_llc(const Sim* s, int arrays) {
   if (const char* e = std::getenv("FDTD_NT")) return std::atoi(e) != 0;
   return (uint64_t)s->ncell_alloc * s->wsize * arrays > ((uint64_t)256 << 20) / 8 * 7;

@@ -2481,12 +2481,16 @@ struct Timer {
   }
 };
 
-// From this many workgroups of plain rows on, the lists of a two-kernel E
-// launch have a launch of their own: beside them the rows' kernel holds the
-// registers of the dispersive update (FP32: seven wavefronts a SIMD instead of
+// FP32: from this many workgroups of plain rows on, the lists of a two-kernel
+// E launch have a launch of their own.  Beside them the rows' kernel holds the
+// registers of the dispersive update (seven wavefronts a SIMD instead of
 // eight), which costs more than a launch once the rows fill the GPU many
-// times over.  FP32 cubes with a gold sphere, one launch against two, us a
-// step: 128 cells a side 46 / 52, 160: 89 / 92, 203: 195 / 192, 256: 361 / 356.
+// times over.  In FP64 the rows alone hold as many (four wavefronts either
+// way), and one launch is the better at every size.  Cubes with a gold sphere,
+// one launch against two, us a step: FP32 96 cells a side 27.2 / 33.1, 128: 46.2
+// / 50.2, 160: 87.0 / 88.3, 203: 229 / 224, 256: 401 / 389, 320: 747 / 725; FP64
+// 96: 43.0 / 48.7, 160: 193 / 197, 203: 403 / 410, 256: 693 / 701, 320: 1320 /
+// 1327.
 constexpr int kListsApart = 32768;
 
 // the segment grid of `rows` rows of nx cells (SegGrid) and its blocks
@@ -2949,7 +2953,7 @@ int step_impl(Sim* s) {
           Timer tm(s, FDTD_K_ADE);
           launch(Parts{0, all.ade, 0, 0, 0, 0}, 0);
         }
-      } else if (tiles < kListsApart) {
+      } else if (sizeof(real) == 8 || tiles < kListsApart) {
         launch(all, tiles);
       } else {
         launch(Parts{}, tiles);
