@@ -32,7 +32,7 @@
 // no z variation (sim3/include/myfdtd_func.f90:19-64 with the z differences
 // zero; mod3/BERpmly_mod.f90:117-195 on the x and y faces):
 //   E: non-PML cells Dz += Ku ((Hy(i)-Hy(i-1)) + (Hx(j-1)-Hx(j))), line
-//      sources on Dz, Ez = Dz*gax (dispersive cells: their own launch);
+//      sources on Dz, Ez = Dz*gax (dispersive cells: beside the tiles);
 //      PML cells Ezx, Ezy split updates scaled by the cell's PML medium, the
 //      source on Ezy, Ez = Ezx + Ezy; periodic x: ghost columns of Ez.
 //   H: non-PML cells Hx -= Ku (Ez(j+1)-Ez(j)), Hy += Ku (Ez(i+1)-Ez(i));
@@ -298,8 +298,6 @@ void* upload(std::vector<DevBuf>& list, size_t* total, const void* data, size_t 
 }
 
 // ---- kernels -------------------------------------------------------------------------
-__device__ __forceinline__ int tile_inst_of(const int32_t* tile_inst, int t) { return tile_inst[t]; }
-
 template <typename real>
 __device__ __forceinline__ bool in_pml_tmz(const Inst<real>& S, int i, int j) {
   return (S.Px > 0 && (i <= S.Px || i > S.nx - S.Px)) || (S.P > 0 && (j <= S.P || j > S.ny - S.P));

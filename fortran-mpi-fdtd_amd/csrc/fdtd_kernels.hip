@@ -11,11 +11,14 @@
 // Two engines:
 //  FUSED  (production): E = E + Ku*gax*curl H per cell (D is kept only in
 //         dispersive cells), split-field PML cells in the same kernel,
-//         source folded in; one H kernel; one kernel per group of
-//         dispersive cells.
+//         source folded in.  A step is an E and an H launch, the
+//         dispersive cells and the monitors beside the cells (k_step_e,
+//         k_step_h), or one pass over two copies of the fields (k_march,
+//         k_gen_e, k_gen_h); Lorentz groups have launches of their own.
 //  STAGED (reference order): updateD, source, material E = D*gax,
 //         dispersive ADE, y-slab PML with interface copies, updateH,
-//         y-slab PML H -- one kernel per stage, D kept everywhere.
+//         y-slab PML H -- the reference's stages in two launches
+//         (k_staged_e, k_staged_h), D kept everywhere.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -583,8 +586,9 @@ __device__ __forceinline__ void h_cell_store(const FieldArgs<real>& a, const Pml
 template <typename real>
 __device__ __forceinline__ void fused_h_cell(const FieldArgs<real>& a, const PmlArgs<real>& p,
                                              const PmlArgs<real>& pw, int i, int j, int k, real& cex, real& cey,
-                                             bool use_carry, const real* E0, const real* E1, const real* E2, const real* HO0, const real* HO1, const real* HO2,
-                                             real* H0, real* H1, real* H2) {
+                                             bool use_carry, const real* E0, const real* E1, const real* E2,
+                                             const real* HO0, const real* HO1, const real* HO2, real* H0, real* H1,
+                                             real* H2) {
   HCellIn<real> in;
   h_cell_load(a, p, i, j, k, use_carry, cex, cey, E0, E1, E2, HO0, HO1, HO2, in);
   cex = in.ex_kp;
@@ -1469,7 +1473,7 @@ __global__ __launch_bounds__(256) void k_ade_multi(FieldArgs<real> a, AdeMulti g
 // with the S of the previous step, then per pole S_l <- ga_l*S_l +
 // gb_l*S_l(older) + gc_l*E, in the module's operation order.  FUSED: D is
 // kept in state word 0 and advanced here from curl H (E-form engine), as
-// k_ade does.  State SoA, word w of component q for cell e at
+// ade_cell does.  State SoA, word w of component q for cell e at
 // state[(w*3+q)*n + e]; words: [D], S_l (l < np), S_l one step older.  FP64
 // in both precisions; E is stored in field precision.
 template <typename real, bool FUSED>
@@ -1785,7 +1789,7 @@ struct MonList {
 template <typename real, typename Fields>
 __device__ __forceinline__ void mon_block(const MonList<real>& m, int px, int pxy, int b, const Fields& F) {
   if (b >= m.nblk) return;
-  if (b >= m.blk[m.nplanes]) {  // probes (incident-line probes are written by k_tfsf_h)
+  if (b >= m.blk[m.nplanes]) {  // point probes, sim3/program.f90:445-451 (incident-line probes are written by k_tfsf_h)
     const int p = (b - m.blk[m.nplanes]) * 256 + (int)threadIdx.x;
     if (p >= m.nprobe || m.ppos[3 * p] < 0) return;
     const int64_t c = m.ppos[3 * p] + px * m.ppos[3 * p + 1] + pxy * m.ppos[3 * p + 2];
@@ -1885,7 +1889,6 @@ __global__ __launch_bounds__(256) void k_step_e(FieldArgs<real> a, PmlArgs<real>
   e_column<real, KZ>(a, p, src, nsrc, i, j, tz, a.h[0], a.h[1], a.h[2], a.e[0], a.e[1], a.e[2]);
 }
 
-// point probes, sim3/program.f90:445-451
 // ---------------------------------------------------------------------------
 // TFSF incident line (sim1/program.f90:217-262, mod1/BERpmly_ExHz_mod.f90).
 // One workgroup walks the line; the PML object's own fields pe, ph live on
