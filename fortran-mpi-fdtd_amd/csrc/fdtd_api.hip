@@ -924,7 +924,9 @@ int flush_profile(Sim* s) {
 // most kReadRings, each held by one read at a time, freed with the last
 // handle.  Not a handle's own: freeing pinned memory waits for every stream
 // of the device, so a handle destroyed after a read would stall behind the
-// other jobs of a pool.
+// other jobs of a pool.  Beside them as many device buffers of kPackKeep
+// bytes for packed field reads (read_field), likewise: a read ends with its
+// stream waited for, so the next one may run on any stream of the device.
 struct ReadRings {
   std::mutex mu;
   char* idle[kReadRings] = {};
@@ -945,13 +947,55 @@ struct ReadRings {
     std::lock_guard<std::mutex> lk(mu);
     idle[nidle++] = p;
   }
-  void handle(int d) {
+  struct Pack {
+    void* p;
+    int device;
+  };
+  Pack packs[kReadRings] = {};
+  int npidle = 0, npall = 0;
+  void* take_pack(const Sim* s) {
     std::lock_guard<std::mutex> lk(mu);
-    handles += d;
-    if (handles) return;
+    for (int q = 0; q < npidle; ++q)
+      if (packs[q].device == s->device) {
+        void* p = packs[q].p;
+        packs[q] = packs[--npidle];
+        return p;
+      }
+    void* p = nullptr;
+    if (npall == kReadRings) return nullptr;
+    if (hipMallocAsync(&p, kPackKeep, s->stream) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    ++npall;
+    return p;
+  }
+  void give_pack(const Sim* s, void* p) {
+    std::lock_guard<std::mutex> lk(mu);
+    packs[npidle++] = {p, s->device};
+  }
+  void opened() {
+    std::lock_guard<std::mutex> lk(mu);
+    ++handles;
+  }
+  // s is being destroyed, its stream still there
+  void closed(const Sim* s) {
+    std::lock_guard<std::mutex> lk(mu);
+    if (--handles) return;
     while (nidle) {
       (void)hipHostFree(idle[--nidle]);
       --nall;
+    }
+    while (npidle) {
+      const Pack& k = packs[--npidle];
+      if (k.device == s->device) {
+        (void)hipFreeAsync(k.p, s->stream);
+      } else {
+        (void)hipSetDevice(k.device);
+        (void)hipFree(k.p);
+        (void)hipSetDevice(s->device);
+      }
+      --npall;
     }
   }
 };
@@ -1047,38 +1091,48 @@ int read_back(Sim* s, std::vector<ReadPart> parts) {
 
 // The interior of a field as FP64 without ghosts, x fastest: packed on the
 // device (launch_pack) into planes of a buffer of at most kPackBytes, which
-// go to the caller as they are.  The buffer is there for the read alone:
-// kept by the handle it would be memory that its admission to a pool did not
-// count.  Small fields (kPackFrom), and any without that memory, are copied
-// as they lie and converted here.  us a read into touched pages, converted
-// here against packed: FP64 40^3 51 : 60, 48^3 137 : 77, 64^3 245 : 160, 96^3
-// 790 : 435; FP32, of which the link then carries half the bytes, 48^3 52 : 75,
-// 64^3 160 : 165, 256 x 256 x 8 250 : 280, 80^3 248 : 265, 96^3 455 : 435; new
-// pages, 96^3 FP64 2050 : 810, FP32 600 : 450; 256^3 FP32 27,000 : 5,000.
+// go to the caller as they are.  The buffer is there for the read alone, up
+// to kPackKeep one that the process's reads share: kept by the handle it would
+// be memory that its admission to a pool did not count (taking and giving
+// back one each time costs 14 us of 77, 48^3 FP64).  Small fields (kPackFrom),
+// and any without that memory, are copied as they lie and converted here.  us
+// a read into touched pages, converted here against packed: FP64 40^3 51 : 60,
+// 48^3 137 : 63, 64^3 245 : 147, 96^3 790 : 425; FP32, of which the link then
+// carries half the bytes, 48^3 52 : 75, 64^3 160 : 165, 256 x 256 x 8 250 : 280,
+// 80^3 248 : 265, 96^3 455 : 435; new pages, 96^3 FP64 2050 : 810, FP32 600 :
+// 450; 256^3 FP32 27,000 : 5,000.
 template <typename real>
 int read_field(Sim* s, void* src, double* dst) {
   const size_t plane = (size_t)s->nx * s->ny;
   const int per = (int)std::min<size_t>((size_t)s->nz, std::max<size_t>(1, kPackBytes / (plane * sizeof(double))));
   struct Buffer {
-    hipStream_t stream;
-    void* p = nullptr;
+    const Sim* s;
+    void *own = nullptr, *shared = nullptr;
     ~Buffer() {
-      if (p) (void)hipFreeAsync(p, stream);
+      if (own) (void)hipFreeAsync(own, s->stream);
+      if (shared) read_rings().give_pack(s, shared);
     }
-  } buf{s->stream};
+  } buf{s};
   FDTD_HIP(hipSetDevice(s->device));
-  if (plane * s->nz * sizeof(double) >= kPackFrom[sizeof(real) == 4] &&
-      hipMallocAsync(&buf.p, plane * sizeof(double) * (size_t)per, s->stream) == hipSuccess) {
-    double* pk = (double*)buf.p;
+  double* pk = nullptr;
+  if (plane * s->nz * sizeof(double) >= kPackFrom[sizeof(real) == 4]) {
+    const size_t need = plane * sizeof(double) * (size_t)per;
+    if (need <= kPackKeep) pk = (double*)(buf.shared = read_rings().take_pack(s));
+    if (!pk && hipMallocAsync(&buf.own, need, s->stream) == hipSuccess) pk = (double*)buf.own;
+  }
+  if (pk) {
     for (int k = 1; k <= s->nz; k += per) {
       const int n = std::min(per, s->nz - k + 1);
       int rc = launch_pack(s, src, k, n, pk);
       if (!rc) rc = read_back(s, {{dst + plane * (size_t)(k - 1), pk, plane * sizeof(double) * (size_t)n}});
-      if (rc) return rc;
+      if (rc) {
+        (void)hipStreamSynchronize(s->stream);  // before another read may take the buffer
+        return rc;
+      }
     }
     return 0;
   }
-  buf.p = nullptr;
+  buf.own = nullptr;
   (void)hipGetLastError();
   std::vector<real> h((size_t)s->ncell_alloc);
   int rc = read_back(s, {{h.data(), src, h.size() * sizeof(real)}});
@@ -1545,7 +1599,7 @@ int fdtd_create(fdtd_sim** out, const fdtd_grid* g) {
     delete s;
     return hip_check(e, "hipStreamCreate");
   }
-  read_rings().handle(1);
+  read_rings().opened();
   *out = s;
   return 0;
 }
@@ -1560,12 +1614,12 @@ int fdtd_destroy(fdtd_sim* s) {
   }
   for (auto ev : s->event_pool) (void)hipEventDestroy(ev);
   for (auto& b : s->allocs) (void)hipFreeAsync(b.p, s->stream);
+  read_rings().closed(s);
   if (s->stream) {
     (void)hipStreamSynchronize(s->stream);
     (void)hipStreamDestroy(s->stream);
   }
   delete s;
-  read_rings().handle(-1);
   return 0;
 }
 

@@ -130,6 +130,7 @@ constexpr int kReadRings = 4;
 // the device buffer (at least one plane; read_field).
 constexpr size_t kPackFrom[2] = {(size_t)768 << 10, (size_t)6 << 20};
 constexpr size_t kPackBytes = (size_t)32 << 20;
+constexpr size_t kPackKeep = (size_t)2 << 20;  // a shared buffer (ReadRings), at most kReadRings of them
 
 // Planes a general workgroup of the one-pass step marches through (at most).
 constexpr int kGenKc = 4;

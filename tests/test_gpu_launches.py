@@ -329,3 +329,39 @@ def test_marked_stores_of_the_x_face_tiles(bx, monkeypatch):
     env = {"FDTD_ONEPASS": "1", "FDTD_ONEPASS_BY": "4", "FDTD_ONEPASS_KC": "16", "FDTD_XFACE_BY": bx}
     got = [run(spec, "fp32", dict(env, FDTD_NT=nt), monkeypatch) for nt in "01"]
     same(*got[0], *got[1])
+
+
+def test_packed_reads_from_more_threads_than_buffers():
+    """Six threads, a handle each, reading fields of 0.8-2 MiB (the four
+    shared buffers) and of 2.7 MiB (buffers of their own) while handles come
+    and go: the fields set, every time, and no device memory of the handles."""
+    import threading
+
+    import fdtd_amd
+
+    bad = []
+
+    def work(q):
+        try:
+            rng = np.random.default_rng(q)
+            for r in range(6):
+                n = [(48, 48, 48), (61, 64, 64), (40, 90, 60), (70, 70, 72)][(q + r) % 4]
+                sim = fdtd_amd.Simulation(*n, 1e-9, 0.5, precision="fp64", engine="fused")
+                f = rng.standard_normal(n)
+                sim.set_field(r % 6, f)
+                m = sim.memory_bytes()
+                for _ in range(8):
+                    if not np.array_equal(sim.field(r % 6), f):
+                        bad.append((q, r))
+                if sim.memory_bytes() != m:
+                    bad.append((q, r, "memory"))
+                sim.close()
+        except Exception as e:  # noqa: BLE001 - reported below
+            bad.append((q, repr(e)))
+
+    th = [threading.Thread(target=work, args=(q,)) for q in range(6)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad, bad
