@@ -7,7 +7,7 @@
 // the H half step, whose threads also write the monitors' samples (each
 // launch costs a small simulation 2-4 us however little it does: the
 // shipped 2D case takes 22.3 us a step with the dispersive cells, the
-// monitors and the step advance in launches of their own, 15.2 us without).
+// monitors and the step advance in launches of their own, 14.3 us without).
 // Thirty-two steps, the DFT fold and the advance of the step counters are
 // captured once in a HIP graph and replayed; the step number of each
 // simulation lives on the device, so simulations with different step counts
